@@ -49,10 +49,21 @@ __device__ __forceinline__ uint64_t wave_sum(uint64_t v) {
     return v;
 }
 
-// Adds a per-thread count to a device counter with one atomic per wave.
+// Adds a per-thread count to a device counter with one atomic per workgroup:
+// every thread of a workgroup of at most 512 threads calls it.  Atomics on one
+// address complete one after another, about 12 ns each: with one per wave the
+// 65536 waves of bin_iq_combine_kernel spent 803 us on 60M windows.
 __device__ __forceinline__ void add_counter(uint64_t* ctr, uint64_t v) {
+    __shared__ uint64_t part[8];
     v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0 && v) atomicAdd((unsigned long long*)ctr, (unsigned long long)v);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t sum = 0;
+        for (unsigned w = 0; w < (blockDim.x + 63) / 64; ++w) sum += part[w];
+        if (sum) atomicAdd((unsigned long long*)ctr, (unsigned long long)sum);
+    }
+    __syncthreads();                                      // part may be used again
 }
 
 __device__ __forceinline__ uint64_t wave_max(uint64_t v) {
@@ -63,10 +74,19 @@ __device__ __forceinline__ uint64_t wave_max(uint64_t v) {
     return v;
 }
 
-// Raises a device counter to the wave's largest value, one atomic per wave.
+// Raises a device counter to the workgroup's largest value, one atomic per
+// workgroup (every thread calls it, as add_counter).
 __device__ __forceinline__ void max_counter(uint64_t* ctr, uint64_t v) {
+    __shared__ uint64_t part[8];
     v = wave_max(v);
-    if ((threadIdx.x & 63) == 0 && v) atomicMax((unsigned long long*)ctr, (unsigned long long)v);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t most = 0;
+        for (unsigned w = 0; w < (blockDim.x + 63) / 64; ++w) most = part[w] > most ? part[w] : most;
+        if (most) atomicMax((unsigned long long*)ctr, (unsigned long long)most);
+    }
+    __syncthreads();
 }
 
 // ------------------------------------------------------------ claim map
@@ -2151,33 +2171,44 @@ __global__ __launch_bounds__(kBlock) void dn_apply_kernel(BinPlan P, Tables T, u
     bin_apply_body<true>(P, T, counters, slice, slots);
 }
 
-// Per-read new k-mers from the window flags; adds the total to n_unique.  A
-// workgroup takes kBlock consecutive reads; their flags are one contiguous
-// range, staged in LDS with coalesced loads when it fits.
+// Per-read new k-mers from the window flags (0 or 1 each); adds the total to
+// n_unique.  kReadLanes lanes share a read and take its flags four at a time,
+// so a wave's loads are contiguous runs of four reads: bound by the flags'
+// bytes.  (A thread per read over flags staged in LDS spent 225 us on 1M
+// reads of 120 windows, most of it on one counter atomic per wave.)
+constexpr int kReadLanes = 16;
 constexpr int kReadNewStage = 32768;
+
+// Sum of v over the kReadLanes lanes of a read.
+__device__ __forceinline__ uint32_t read_lanes_sum(uint32_t v) {
+#pragma unroll
+    for (int o = kReadLanes / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
 
 __global__ __launch_bounds__(kBlock) void bin_read_new_kernel(const int64_t* kmer_off, uint64_t n_reads,
                                                             const uint8_t* flags, uint64_t* n_new,
                                                             uint64_t* counters) {
-    __shared__ uint8_t fl[kReadNewStage];
+    constexpr uint64_t kReads = kBlock / kReadLanes;      // reads of a workgroup at a time
+    const int sub = threadIdx.x % kReadLanes;
     uint64_t tot = 0;
-    for (uint64_t r0 = (uint64_t)blockIdx.x * kBlock; r0 < n_reads; r0 += (uint64_t)gridDim.x * kBlock) {
-        const uint64_t r1 = r0 + kBlock < n_reads ? r0 + kBlock : n_reads;
-        const int64_t k0 = kmer_off[r0], k1 = kmer_off[r1];
-        const bool staged = k1 - k0 <= kReadNewStage;
-        __syncthreads();
-        if (staged)
-            for (int64_t i = threadIdx.x; i < k1 - k0; i += kBlock) fl[i] = flags[k0 + i];
-        __syncthreads();
-        const uint64_t r = r0 + threadIdx.x;
-        if (r < r1) {
-            uint64_t c = 0;
+    for (uint64_t r0 = (uint64_t)blockIdx.x * kReads; r0 < n_reads; r0 += (uint64_t)gridDim.x * kReads) {
+        const uint64_t r = r0 + threadIdx.x / kReadLanes;
+        uint32_t c = 0;
+        if (r < n_reads) {
             const int64_t a = kmer_off[r], b = kmer_off[r + 1];
-            if (staged) {
-                for (int64_t k = a; k < b; ++k) c += fl[k - k0];
-            } else {
-                for (int64_t k = a; k < b; ++k) c += flags[k];
+            for (int64_t k = a + 4 * sub; k < b; k += 4 * kReadLanes) {
+                if (k + 4 <= b) {
+                    uint32_t w;
+                    __builtin_memcpy(&w, flags + k, 4);
+                    c += (uint32_t)__popc(w);
+                } else {
+                    for (int64_t i = k; i < b; ++i) c += flags[i];
+                }
             }
+        }
+        c = read_lanes_sum(c);
+        if (sub == 0 && r < n_reads) {
             if (n_new) n_new[r] += c;
             tot += c;
         }
@@ -2226,23 +2257,40 @@ __global__ void bin_iq_combine_kernel(const uint32_t* vq, const int64_t* nk, uin
 // StreamingSolidFilter::Filter::filter_sequence (solidifier.hh:58-73) per read
 // from its insert_and_query counts, with the reference's types: count_t
 // against a uint32_t threshold, a float ratio compared in double with
-// 1.0 - min_prop_solid.  Reads shorter than K do not pass.
-__global__ void solid_reads_kernel(const int64_t* off, const int64_t* kmer_off, uint64_t n_reads, int K,
-                                   const int16_t* counts, uint32_t threshold, float min_prop_solid,
-                                   uint8_t* passed) {
-    for (uint64_t r = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; r < n_reads;
-         r += (uint64_t)gridDim.x * blockDim.x) {
-        const int64_t len = off[r + 1] - off[r];
-        if (len < K) {
-            passed[r] = 0;
-            continue;
-        }
+// 1.0 - min_prop_solid.  Reads shorter than K do not pass.  kReadLanes lanes
+// share a read and take its counts four at a time: bound by the counts' bytes
+// (a thread per read, each on its own line, took 862 us for 500k reads).
+__global__ __launch_bounds__(kBlock) void solid_reads_kernel(const int64_t* off, const int64_t* kmer_off,
+                                                           uint64_t n_reads, int K, const int16_t* counts,
+                                                           uint32_t threshold, float min_prop_solid,
+                                                           uint8_t* passed) {
+    constexpr uint64_t kReads = kBlock / kReadLanes;
+    const int sub = threadIdx.x % kReadLanes;
+    for (uint64_t r0 = (uint64_t)blockIdx.x * kReads; r0 < n_reads; r0 += (uint64_t)gridDim.x * kReads) {
+        const uint64_t r = r0 + threadIdx.x / kReadLanes;
+        const bool live = r < n_reads;
+        const int64_t len = live ? off[r + 1] - off[r] : 0;
         uint32_t n_not_solid = 0;
-        for (int64_t k = kmer_off[r]; k < kmer_off[r + 1]; ++k)
-            n_not_solid += (uint32_t)(int)counts[k] < threshold ? 1u : 0u;
-        const uint32_t n_kmers = (uint32_t)(len - K + 1);
-        const bool fails = (double)((float)n_not_solid / (float)n_kmers) >= (1.0 - (double)min_prop_solid);
-        passed[r] = fails ? 0 : 1;
+        if (live && len >= K) {
+            const int64_t a = kmer_off[r], b = kmer_off[r + 1];
+            for (int64_t k = a + 4 * sub; k < b; k += 4 * kReadLanes) {
+                int16_t c[4];
+                if (k + 4 <= b) {
+                    __builtin_memcpy(c, counts + k, 8);
+                } else {
+                    for (int i = 0; i < 4; ++i) c[i] = k + i < b ? counts[k + i] : (int16_t)0;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) n_not_solid += k + i < b && (uint32_t)(int)c[i] < threshold ? 1u : 0u;
+            }
+        }
+        n_not_solid = read_lanes_sum(n_not_solid);
+        if (sub == 0 && live) {
+            const uint32_t n_kmers = (uint32_t)(len - K + 1);
+            const bool fails =
+                len < K || (double)((float)n_not_solid / (float)n_kmers) >= (1.0 - (double)min_prop_solid);
+            passed[r] = fails ? 0 : 1;
+        }
     }
 }
 
@@ -2681,7 +2729,7 @@ void launch_hash_query(const Launch& L, const uint64_t* h, uint64_t n, const Tab
 void launch_bit_union(uint32_t* me, const uint32_t* other, uint64_t n_words, int count_bits, uint64_t* counters,
                       hipStream_t s) {
     const uint64_t g = (n_words + 255) / 256;
-    bit_union_kernel<<<(unsigned)(g < 16384 ? (g ? g : 1) : 16384), 256, 0, s>>>(me, other, n_words, count_bits,
+    bit_union_kernel<<<(unsigned)(g < 2048 ? (g ? g : 1) : 2048), 256, 0, s>>>(me, other, n_words, count_bits,
                                                                               counters);
 }
 
@@ -2742,8 +2790,8 @@ void launch_bin_apply(const BinPlan& P, const Tables& T, uint64_t* counters, int
 
 void launch_bin_read_new(const int64_t* kmer_off, uint64_t n_reads, const uint8_t* flags, uint64_t* n_new,
                          uint64_t* counters, hipStream_t s) {
-    const uint64_t g = (n_reads + kBlock - 1) / kBlock;
-    bin_read_new_kernel<<<(unsigned)(g < 4096 ? (g ? g : 1) : 4096), kBlock, 0, s>>>(kmer_off, n_reads, flags, n_new,
+    const uint64_t g = (n_reads + kBlock / kReadLanes - 1) / (kBlock / kReadLanes);
+    bin_read_new_kernel<<<(unsigned)(g < 2048 ? (g ? g : 1) : 2048), kBlock, 0, s>>>(kmer_off, n_reads, flags, n_new,
                                                                                   counters);
 }
 
@@ -2816,8 +2864,8 @@ void launch_zero_words(uint32_t* p, const int64_t* n, uint64_t max_n, hipStream_
 
 void launch_solid_reads(const int64_t* off, const int64_t* kmer_off, uint64_t n_reads, int K, const int16_t* counts,
                         uint32_t threshold, float min_prop_solid, uint8_t* passed, hipStream_t s) {
-    const uint64_t g = (n_reads + 255) / 256;
-    solid_reads_kernel<<<(unsigned)(g < 16384 ? (g ? g : 1) : 16384), 256, 0, s>>>(off, kmer_off, n_reads, K, counts,
+    const uint64_t g = (n_reads + kBlock / kReadLanes - 1) / (kBlock / kReadLanes);
+    solid_reads_kernel<<<(unsigned)(g < 2048 ? (g ? g : 1) : 2048), kBlock, 0, s>>>(off, kmer_off, n_reads, K, counts,
                                                                                 threshold, min_prop_solid, passed);
 }
 
