@@ -403,23 +403,43 @@ int check_kernel_errors(gt_storage* st, hipStream_t s) {
     return GT_OK;
 }
 
-// Prepares tile_read (and kmer_off when wanted) for one call.
-int prepare_reads(Scratch& sc, Reads& R, bool want_kmer_off, hipStream_t s) {
+// Prepares tile_read (and kmer_off when wanted) for one call, and clears
+// n_new (n_reads entries) when given.  A small batch takes one launch for all
+// of it, which then also starts the call's first generations (bump; see
+// next_gen); *bumped says whether it did.
+struct GenBump {
+    uint64_t* storage_gen = nullptr;
+    uint64_t* claim_gen = nullptr;
+    bool bumped = false;
+};
+
+int prepare_reads(Scratch& sc, Reads& R, bool want_kmer_off, hipStream_t s, uint64_t* n_new = nullptr,
+                  GenBump* bump = nullptr) {
     const int64_t n_tiles = (R.n_bases + kTileGrain - 1) / kTileGrain;
     GT_TRY(sc.tile_read.ensure((size_t)(n_tiles + 1) * sizeof(uint32_t)));
-    // tile_read entries are all written for well-formed offsets; zero first so
-    // malformed offsets stay in bounds.
-    launch_fill_u64(sc.tile_read.as<uint64_t>(), (sc.tile_read.bytes) / 8, 0, s);
-    launch_tile_read(R.off, R.n_reads, R.n_bases, sc.tile_read.as<uint32_t>(), n_tiles, R.dyn, s);
     R.tile_read = sc.tile_read.as<uint32_t>();
     R.kmer_off = nullptr;
     if (want_kmer_off) {
         GT_TRY(sc.kmer_off.ensure((R.n_reads + 1) * sizeof(int64_t)));
         GT_TRY(sc.scan_blocks.ensure((scan_block_count(R.n_reads) + 1) * sizeof(int64_t)));
-        launch_kmer_offsets(R.off, R.n_reads, R.K, sc.kmer_off.as<int64_t>(), sc.scan_blocks.as<int64_t>(), R.dyn,
-                            s);
         R.kmer_off = sc.kmer_off.as<int64_t>();
     }
+    if (!R.dyn && layout_is_small(R.n_reads, R.n_bases)) {
+        launch_layout_small(R.off, R.n_reads, R.n_bases, R.K, sc.tile_read.as<uint32_t>(),
+                            want_kmer_off ? sc.kmer_off.as<int64_t>() : nullptr, n_new,
+                            bump ? bump->storage_gen : nullptr, bump ? bump->claim_gen : nullptr, s);
+        if (bump) bump->bumped = true;
+        GT_HIP(hipGetLastError());
+        return GT_OK;
+    }
+    // tile_read entries are all written for well-formed offsets; zero first so
+    // malformed offsets stay in bounds.
+    launch_fill_u64(sc.tile_read.as<uint64_t>(), (sc.tile_read.bytes) / 8, 0, s);
+    launch_tile_read(R.off, R.n_reads, R.n_bases, sc.tile_read.as<uint32_t>(), n_tiles, R.dyn, s);
+    if (want_kmer_off)
+        launch_kmer_offsets(R.off, R.n_reads, R.K, sc.kmer_off.as<int64_t>(), sc.scan_blocks.as<int64_t>(), R.dyn,
+                            s);
+    if (n_new) launch_fill_u64(n_new, R.n_reads, 0, s);
     GT_HIP(hipGetLastError());
     return GT_OK;
 }
@@ -490,11 +510,6 @@ int prepare_claims(Scratch& sc, int kind, uint32_t n_tables, uint64_t n_starts, 
     if (kind == kExact) {
         uint64_t sb = std::min<uint64_t>(starts, 1ULL << 31);
         if (cap) sb = std::min(sb, cap);
-        if (sc.fixed) {
-            if (sc.fresh.bytes < sb) sb = sc.fresh.bytes / kTileMax * kTileMax;
-        } else {
-            GT_TRY(sc.fresh.ensure(sb));
-        }
         if (sb == 0) return fail(GT_ERR_INTERNAL, "scratch too small");
         if (!sc.claim_cap) GT_TRY(alloc_claims(sc, 2, s));   // unused by the exact set; a valid view
         *sub = sb;
@@ -523,12 +538,13 @@ int prepare_claims(gt_storage* st, uint64_t n_starts, uint64_t* sub, hipStream_t
 // 32 bits) and of the claim map.  Claim-map keys keep 28 bits of the map's
 // generation, so the map is cleared whenever that field would wrap, and
 // values that are 0 in those bits are skipped (cleared keys read as gen 0).
-int next_gen(gt_storage* st, Scratch& sc, hipStream_t s) {
+// `bumped`: a layout launch of this call already raised both counters once.
+int next_gen(gt_storage* st, Scratch& sc, hipStream_t s, bool bumped = false) {
     if (st->gen_issued + 2 >= 0xFFFFFFFFULL || sc.claim_gen_issued + 2 >= 0xFFFFFFFFULL)
         return fail(GT_ERR_INTERNAL, "batch generation counter exhausted");
     st->gen_issued++;
     sc.claim_gen_issued++;
-    launch_bump_gen(st->counters.as<uint64_t>() + kGen, sc.claim_gen.as<uint64_t>(), s);
+    if (!bumped) launch_bump_gen(st->counters.as<uint64_t>() + kGen, sc.claim_gen.as<uint64_t>(), s);
     if ((sc.claim_gen_issued & kGenKeyMask) == 0) {
         launch_fill_u64(sc.claim_keys.as<uint64_t>(), sc.claim_cap, 0, s);
         launch_fill_u64(sc.claim_vals.as<uint64_t>(), sc.claim_cap, 0, s);
@@ -581,23 +597,40 @@ Launch make_launch(int kind, hipStream_t s) {
 Launch make_launch(hipStream_t s) { return make_launch(0, s); }
 Launch make_launch(const gt_storage* st, hipStream_t s) { return make_launch(st->kind, s); }
 
+// Launch of a walk over n_starts start positions.  Below kSmallStarts the
+// tuned tile shape leaves CUs without waves to hide a window's chain of table
+// accesses behind, so a thread takes four windows together instead (the
+// kernels' kPerSmall form): 500 reads into a 4 x 1e6 Bloom filter went from
+// 365 to 191 us, 4167 reads against 4 x 2^28 counts from 86 to 58 us.
+constexpr uint64_t kSmallStarts = 1ULL << 22;
+Launch make_launch(const gt_storage* st, uint64_t n_starts, hipStream_t s) {
+    Launch L = make_launch(st->kind, s);
+    if (n_starts < kSmallStarts) {
+        L.per = 4;
+        L.grid = std::max(1, g_dev.cus * 8);
+    }
+    return L;
+}
+
 // Device work of one first-touch sub-batch [Rs.b0, Rs.b1) with the given
 // claim map and fresh buffer.  For the exact set, `growth` allows a
 // synchronising capacity check (never while a graph is being captured).
 int enqueue_subbatch(gt_storage* st, Scratch& sc, const Launch& L, const Reads& Rs, uint64_t* n_new,
-                     uint8_t* new_flags, hipStream_t s, bool growth) {
+                     uint8_t* new_flags, hipStream_t s, bool growth, bool bumped = false) {
     uint64_t* ctr = st->counters.as<uint64_t>();
     uint8_t* fresh = sc.fresh.as<uint8_t>();
-    GT_TRY(next_gen(st, sc, s));
+    GT_TRY(next_gen(st, sc, s, bumped));
     const ClaimMap cm = claim_view(sc);
     if (st->kind == kExact) {
         const uint64_t nstarts = (uint64_t)(Rs.b1 - Rs.b0);
         if (growth && 2 * (st->ecount_ub + nstarts) > st->ecap) {
-            // Bound the growth by this sub-batch's fresh windows.
+            // Bound the growth by this sub-batch's absent windows.
             launch_fill_u64(ctr + kFresh, 1, 0, s);
             {
                 ProfScope ps("exact_lookup", s);
-                launch_exact_lookup(L, Rs, st->exact_view(), fresh, ctr);
+                Launch LL = L;
+                if (LL.per < kPerMin) LL.per = kPerMin;
+                launch_exact_lookup(LL, Rs, st->exact_view(), nullptr, ctr);
             }
             GT_HIP(hipGetLastError());
             uint64_t c[kNCounters];
@@ -606,20 +639,20 @@ int enqueue_subbatch(gt_storage* st, Scratch& sc, const Launch& L, const Reads& 
             GT_TRY(exact_reserve(st, c[kFresh], s));
             st->ecount_ub += c[kFresh];
         } else {
-            ProfScope ps("exact_lookup", s);
-            launch_exact_lookup(L, Rs, st->exact_view(), fresh, ctr);
             st->ecount_ub += nstarts;
         }
         const ExactSet E = st->exact_view();
         {
             ProfScope ps("exact_insert", s);
-            launch_exact_insert(L, Rs, E, fresh, ctr);
+            launch_exact_add(L, Rs, E, n_new, ctr);
         }
-        {
+        if (new_flags) {
             ProfScope ps("exact_resolve", s);
-            launch_exact_resolve(L, Rs, E, fresh, n_new, new_flags, ctr);
+            Launch LL = L;
+            if (LL.per < kPerMin) LL.per = kPerMin;
+            launch_exact_flags(LL, Rs, E, new_flags, ctr);
         }
-        launch_exact_tail(ctr, s);
+        launch_exact_reads_tail(Rs, E, ctr, s);
     } else {
         const Tables T = st->tables_view();
         {
@@ -879,8 +912,14 @@ int dbg_insert_impl(gt_storage* st, Scratch& sc, Reads R, uint64_t* n_new, uint8
         return GT_OK;
     }
     const bool binned = use_binned(st, sc, R);
-    GT_TRY(prepare_reads(sc, R, new_flags != nullptr || binned, s));
-    if (n_new) launch_fill_u64(n_new, R.n_reads, 0, s);
+    uint64_t sub = 0;
+    GenBump bump;
+    if (!binned) {
+        GT_TRY(prepare_claims(sc, st->kind, st->n_tables, (uint64_t)R.n_bases, &sub, s));
+        bump.storage_gen = st->counters.as<uint64_t>() + kGen;
+        bump.claim_gen = sc.claim_gen.as<uint64_t>();
+    }
+    GT_TRY(prepare_reads(sc, R, new_flags != nullptr || binned, s, n_new, binned ? nullptr : &bump));
     if (binned) {
         const int rc = binned_insert_impl(st, sc, R, n_new, new_flags, nullptr, s);
         if (rc != GT_ERR_OUT_OF_MEMORY) return rc;
@@ -891,15 +930,14 @@ int dbg_insert_impl(gt_storage* st, Scratch& sc, Reads R, uint64_t* n_new, uint8
         sc.bin_dig2.release();
         sc.bin_flags.release();
         sc.bin_vq.release();
+        GT_TRY(prepare_claims(sc, st->kind, st->n_tables, (uint64_t)R.n_bases, &sub, s));
     }
-    uint64_t sub = 0;
-    GT_TRY(prepare_claims(sc, st->kind, st->n_tables, (uint64_t)R.n_bases, &sub, s));
-    const Launch L = make_launch(st, s);
+    const Launch L = make_launch(st, std::min<uint64_t>(sub, (uint64_t)R.n_bases), s);
     for (int64_t b0 = 0; b0 < R.n_bases; b0 += (int64_t)sub) {
         Reads Rs = R;
         Rs.b0 = b0;
         Rs.b1 = std::min<int64_t>(R.n_bases, b0 + (int64_t)sub);
-        GT_TRY(enqueue_subbatch(st, sc, L, Rs, n_new, new_flags, s, true));
+        GT_TRY(enqueue_subbatch(st, sc, L, Rs, n_new, new_flags, s, true, b0 == 0 && bump.bumped));
     }
     return GT_OK;
 }
@@ -921,6 +959,7 @@ int hashes_insert_impl(gt_storage* st, const uint64_t* h, uint64_t n, uint8_t* i
     uint64_t* ctr = st->counters.as<uint64_t>();
     uint64_t sub = 0;
     GT_TRY(prepare_claims(st, n, &sub, s));
+    if (st->kind == kExact) GT_TRY(st->own.fresh.ensure(std::min(sub, n)));
     for (uint64_t i0 = 0; i0 < n; i0 += sub) {
         const uint64_t m = std::min<uint64_t>(sub, n - i0);
         GT_TRY(next_gen(st, st->own, s));
@@ -1571,7 +1610,7 @@ int gt_dbg_query_dev(gt_storage* st, uint16_t K, int canonical, int mode, const 
     GT_TRY(prepare_reads(st, R, true, s));
     {
         ProfScope ps("query", s);
-        launch_query(make_launch(st, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
+        launch_query(make_launch(st, n_bases, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
     }
     GT_HIP(hipGetLastError());
     if (st->use_bigcount && st->big.aux) {
@@ -1668,7 +1707,7 @@ int gt_dbg_insert_and_query_dev(gt_storage* st, uint16_t K, int canonical, int m
     // sparseppstorage.cc:21-25); a query after the batch gives exactly that
     // (and -1 for skipped windows).
     GT_TRY(prepare_reads(st, R, true, s));
-    launch_query(make_launch(st, s), R, st->tables_view(), st->exact_or_empty(), counts, nullptr);
+    launch_query(make_launch(st, n_bases, s), R, st->tables_view(), st->exact_or_empty(), counts, nullptr);
     GT_HIP(hipGetLastError());
     return GT_OK;
 }
@@ -2204,7 +2243,7 @@ int gt_autotune(gt_storage* st, uint16_t K, int canonical, int mode, const uint8
                 // read-only passes: the claim (or lookup) pass writes only
                 // scratch; a later insert starts a new generation first.
                 if (st->kind == kExact) {
-                    launch_exact_lookup(L, R, st->exact_view(), st->own.fresh.as<uint8_t>(), ctr);
+                    launch_exact_lookup(L, R, st->exact_view(), nullptr, ctr);
                 } else {
                     launch_claim(L, R, st->tables_view(), claim_view(st->own), st->own.fresh.as<uint8_t>(), ctr);
                 }
@@ -2595,7 +2634,7 @@ int gt_dbg_query_ws_dev(gt_storage* st, gt_workspace* ws, uint16_t K, int canoni
     GT_TRY(prepare_reads(ws->sc, R, true, s));
     {
         ProfScope ps("query", s);
-        launch_query(make_launch(st, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
+        launch_query(make_launch(st, n_bases, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
     }
     GT_HIP(hipGetLastError());
     return GT_OK;

@@ -193,6 +193,51 @@ __device__ uint64_t exact_insert(const ExactSet& es, uint64_t key, uint64_t* err
     return kEmpty;
 }
 
+// The stamp of keys that a rehash moved: generation 0, older than every batch's.
+constexpr uint64_t kOldStamp = ~0ULL << 32;
+
+// Whether a key with this (inverted) stamp came with the running batch: not
+// stamped yet, or stamped with its generation.  Keys of earlier batches carry
+// their own batch's stamp, or kOldStamp after a rehash.
+__device__ __forceinline__ bool stamp_is_fresh(uint64_t inv, uint32_t gen) {
+    return inv == ~0ULL || (uint32_t)(inv >> 32) == ~gen;
+}
+
+// Finds or inserts key, probing from slot: its slot (kEmpty when the probe
+// limit is reached) and whether it came with the running batch.  A plain load
+// may show a slot as it was when the kernel began: then it shows it free, and
+// the compare-and-swap gives the key that took it meanwhile, which is of this
+// batch; a key of an earlier batch is always shown, with its own stamp.
+struct ExactHit {
+    uint64_t slot;
+    bool fresh;
+};
+
+__device__ __forceinline__ ulonglong2 exact_pair(const ExactSet& es, uint64_t slot) {
+    return *reinterpret_cast<const ulonglong2*>(exact_key(es, slot));
+}
+
+__device__ __forceinline__ ExactHit exact_add(const ExactSet& es, uint64_t key, uint64_t slot, uint32_t gen,
+                                              uint64_t* errors) {
+    if (key == kEmpty) {
+        atomicOr(es.ones, 1u);
+        return {es.cap, stamp_is_fresh(load_relaxed(exact_stamp(es, es.cap)), gen)};
+    }
+    const uint64_t mask = es.cap - 1;
+    for (uint64_t probes = 0; probes < es.cap; ++probes) {
+        const ulonglong2 kv = exact_pair(es, slot);
+        if (kv.x == key) return {slot, stamp_is_fresh(kv.y, gen)};
+        if (kv.x == kEmpty) {
+            const uint64_t prev = atomicCAS((unsigned long long*)exact_key(es, slot), (unsigned long long)kEmpty,
+                                            (unsigned long long)key);
+            if (prev == kEmpty || prev == key) return {slot, true};
+        }
+        slot = (slot + 1) & mask;
+    }
+    atomicOr((unsigned long long*)errors, (unsigned long long)kErrProbe);
+    return {kEmpty, false};
+}
+
 // ------------------------------------------------------------ storage reads
 
 // Bloom: presence of bin b of table i (bit b%8 of byte b/8, which is bit b%32
@@ -277,6 +322,10 @@ __device__ __forceinline__ uint32_t neighbors_present(const Tables& T, const Exa
 }
 
 // ------------------------------------------------------------ tile walker
+
+__device__ __forceinline__ uint64_t kmer_value(uint64_t fw, uint64_t rc, int canonical) {
+    return canonical ? (fw < rc ? fw : rc) : fw;
+}
 
 // LDS of the tile walker for tiles of up to TILE starts.
 template <int TILE>
@@ -387,6 +436,26 @@ __device__ __forceinline__ void seg_values(const Sh& sh, Sg* sg, int u, int L) {
     sg->bq[u] = (uint8_t)bq;
 }
 
+// A thread's PER windows taken together (batches too small to hide the latency
+// of one window's table accesses behind other waves): values, reads and read
+// starts; bit j of `in`: window j lies in a read; bit j of `valid`: it also
+// holds no non-ACGT byte that the mode skips.
+template <int PER>
+struct Windows {
+    int64_t s0;
+    uint64_t h[PER];
+    uint32_t r[PER];
+    int64_t rstart[PER];
+    uint32_t in, valid;
+};
+
+// Ops that take a thread's windows together define kTogether and
+// together(const Windows<PER>&); their seg_scratch() gives stitched starts.
+template <class Op, class = void>
+struct TakesTogether : std::false_type {};
+template <class Op>
+struct TakesTogether<Op, std::void_t<decltype(Op::kTogether)>> : std::true_type {};
+
 template <int PER, int BLK = kBlock, class Op, class Sh>
 __device__ void walk_tiles(const Reads& R, Sh& sh, Op& op) {
     constexpr int kTile = BLK * PER;
@@ -420,7 +489,7 @@ __device__ void walk_tiles(const Reads& R, Sh& sh, Op& op) {
             for (int i = tid; i < span; i += BLK) sh.bytes[i] = i < nload ? R.seq[t0 + i] : 0;
         }
         if (tid == 0) {
-            const int64_t g_end = (t0 + kTile) / kTileGrain;
+            const int64_t g_end = (t0 + kTile + kTileGrain - 1) / kTileGrain;
             uint32_t rl = R.tile_read[t0 / kTileGrain];
             uint32_t rh = g_end < n_grains ? R.tile_read[g_end] : (uint32_t)(n_reads - 1);
             if (rl >= n_reads) rl = (uint32_t)(n_reads - 1);
@@ -501,6 +570,33 @@ __device__ void walk_tiles(const Reads& R, Sh& sh, Op& op) {
                 for (int k = K - 1; k >= 0; --k) rc = gt_rotl(rc, 1) ^ sh.tr[B[li + k]];
             }
 
+            if constexpr (TakesTogether<Op>::value) {
+                Windows<PER> w;
+                w.s0 = s0;
+                w.in = w.valid = 0;
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    const int64_t s = s0 + j;
+                    if (j > 0) {
+                        const uint8_t out = B[li + j - 1], in = B[li + j + K - 1];
+                        fw = gt_rotl(fw, 1) ^ gt_rotl(sh.tf[out], Kr) ^ sh.tf[in];
+                        rc = gt_rotr(rc ^ gt_rotl(sh.tr[in], Kr) ^ sh.tr[out], 1);
+                        bad += (int)!gt_is_acgt(in) - (int)!gt_is_acgt(out);
+                    }
+                    while (s >= rend && r < rh) {
+                        ++r;
+                        rstart = rend;
+                        rend = cached ? sh.roff[r + 1 - rl] : R.off[r + 1];
+                    }
+                    const uint32_t in_read = s < s_end && s >= rstart && s + K <= rend ? 1u : 0u;
+                    w.h[j] = kmer_value(fw, rc, R.canonical);
+                    w.r[j] = r;
+                    w.rstart[j] = rstart;
+                    w.in |= in_read << j;
+                    w.valid |= (R.mode == kRaw || bad == 0 ? in_read : 0u) << j;
+                }
+                op.together(w);
+            } else
             for (int j = 0; j < PER; ++j) {
                 const int64_t s = s0 + j;
                 if (s >= s_end) break;
@@ -531,10 +627,6 @@ __device__ void walk_tiles(const Reads& R, Sh& sh, Op& op) {
         }
         call_end_tile(op, tile, 0);
     }
-}
-
-__device__ __forceinline__ uint64_t kmer_value(uint64_t fw, uint64_t rc, int canonical) {
-    return canonical ? (fw < rc ? fw : rc) : fw;
 }
 
 // Packed index of the first window starting at or after base x (x a multiple
@@ -572,6 +664,34 @@ struct ReadAcc {
     }
 };
 
+// The same for windows taken together: bit j of is_new adds one to read
+// w.r[j].  Lanes whose new windows are all of one read are summed over the
+// wave's lanes of that read (a wave's 64 x PER starts lie in a few reads), so
+// a read gets one atomic per wave and not one per lane.
+template <int PER>
+__device__ __forceinline__ void add_to_reads(uint64_t* out, const Windows<PER>& w, uint32_t is_new) {
+    if (!out) return;
+    if (w.r[0] != w.r[PER - 1]) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            if (is_new >> j & 1u) atomicAdd((unsigned long long*)&out[w.r[j]], 1ULL);
+        is_new = 0;
+    }
+    static_assert(PER <= 7, "three bits of a lane's count are summed");
+    const uint32_t n = (uint32_t)__popc(is_new);
+    uint64_t left = __ballot(n != 0);
+    while (left) {
+        const int lead = __builtin_ctzll(left);
+        const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)w.r[0], lead);
+        const bool mine = n != 0 && w.r[0] == r;
+        const uint32_t sum = (uint32_t)__popcll(__ballot(mine && (n & 1u))) +
+                             2u * (uint32_t)__popcll(__ballot(mine && (n & 2u))) +
+                             4u * (uint32_t)__popcll(__ballot(mine && (n & 4u)));
+        if ((int)(threadIdx.x & 63) == lead) atomicAdd((unsigned long long*)&out[r], (unsigned long long)sum);
+        left &= ~__ballot(mine);
+    }
+}
+
 // ------------------------------------------------------------ Bloom / CMS ops
 
 // Claim pass: reads the tables only.  For each table whose bin is empty at
@@ -605,6 +725,85 @@ struct ClaimOp {
     }
     __device__ void begin_tile(int64_t) {}
     __device__ void flush() {}
+};
+
+// The claim pass over a thread's windows together: the bins of four tables of
+// every window are read together, then the claim slots of the empty ones, then
+// the slots are taken, then stamped.  A lookup that meets another key is
+// finished by claim_insert.
+struct ClaimTogetherOp : ClaimOp {
+    static constexpr bool kTogether = true;
+    template <int PER>
+    __device__ void together(const Windows<PER>& w) {
+        uint8_t mask[PER] = {};
+#pragma unroll
+        for (uint32_t g = 0; g < (uint32_t)kMaxTables; g += 4) {
+            if (g >= T.n) break;
+            uint32_t bin[4][PER];                          // table sizes are below 2^32
+            uint32_t word[4][PER];
+#pragma unroll
+            for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    word[t][j] = 1;
+                    if (g + t < T.n && (w.valid >> j & 1u)) {
+                        const uint64_t b = gt_fastmod(w.h[j], T.p[g + t], T.m[g + t]);
+                        bin[t][j] = (uint32_t)b;
+                        word[t][j] = T.kind == kBit
+                                         ? reinterpret_cast<const uint32_t*>(T.base[g + t])[b >> 5] >> (b & 31)
+                                         : (uint32_t)T.base[g + t][b];
+                    }
+                }
+            }
+            uint64_t slot[4][PER], cur[4][PER];
+            uint32_t empty = 0;                            // bit t * PER + j
+#pragma unroll
+            for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    if (T.kind == kBit ? word[t][j] & 1u : word[t][j]) continue;
+                    empty |= 1u << (t * PER + j);
+                    mask[j] |= (uint8_t)(1u << (g + t < 7 ? g + t : 7));
+                    slot[t][j] = claim_slot(cm, claim_key(gen, g + t, bin[t][j]));
+                    cur[t][j] = load_relaxed(&cm.keys[slot[t][j]]);
+                }
+            }
+            // as the first steps of claim_insert: a slot of an earlier
+            // generation is free; cur = the key found in it
+#pragma unroll
+            for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    if (!(empty >> (t * PER + j) & 1u)) continue;
+                    const uint64_t key = claim_key(gen, g + t, bin[t][j]);
+                    if ((cur[t][j] >> 36) != (key >> 36)) {
+                        const uint64_t prev = atomicCAS((unsigned long long*)&cm.keys[slot[t][j]],
+                                                        (unsigned long long)cur[t][j], (unsigned long long)key);
+                        cur[t][j] = prev == cur[t][j] ? key : prev;
+                    }
+                }
+            }
+#pragma unroll
+            for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    if (!(empty >> (t * PER + j) & 1u)) continue;
+                    const uint64_t key = claim_key(gen, g + t, bin[t][j]);
+                    const uint64_t stamp = claim_stamp(gen, (uint32_t)(w.s0 + j - b0));
+                    if (cur[t][j] == key)
+                        atomicMax((unsigned long long*)&cm.vals[slot[t][j]], (unsigned long long)stamp);
+                    else
+                        claim_insert(cm, key, stamp, errors);
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (!(w.valid >> j & 1u)) continue;
+            fresh[w.s0 + j - b0] = mask[j];
+            n_fresh += mask[j] != 0;
+        }
+    }
 };
 
 // Saturating byte increment (bytestorage.cc:88-93: +1 while below 255) with
@@ -668,9 +867,113 @@ struct ApplyOp {
     __device__ void flush() { acc.flush(); }
 };
 
+// The apply pass over a thread's windows together, four tables at a time: the
+// updates of every window are in flight together, then the claim slots of the
+// bins that were empty.
+struct ApplyTogetherOp : ApplyOp {
+    static constexpr bool kTogether = true;
+    template <int PER>
+    __device__ void together(const Windows<PER>& w) {
+        uint8_t mask[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) mask[j] = w.valid >> j & 1u ? fresh[w.s0 + j - b0] : (uint8_t)0;
+        uint32_t is_new = 0;
+#pragma unroll
+        for (uint32_t g = 0; g < (uint32_t)kMaxTables; g += 4) {
+            if (g >= T.n) break;
+            uint32_t bin[4][PER];                          // table sizes are below 2^32
+            uint32_t old[4][PER];
+#pragma unroll
+            for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    if (g + t >= T.n || !(w.valid >> j & 1u)) continue;
+                    const uint64_t b = gt_fastmod(w.h[j], T.p[g + t], T.m[g + t]);
+                    bin[t][j] = (uint32_t)b;
+                    if (T.kind == kBit)
+                        old[t][j] = atomicOr(reinterpret_cast<uint32_t*>(T.base[g + t]) + (b >> 5), 1u << (b & 31));
+                    else
+                        old[t][j] = __hip_atomic_load(reinterpret_cast<uint32_t*>(T.base[g + t] + (b & ~3ULL)),
+                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+            if (T.kind == kByte) {
+                // one saturating increment of the word read; a word that changed
+                // meanwhile goes to byte_sat_inc
+                uint32_t seen[4][PER];
+#pragma unroll
+                for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                    for (int j = 0; j < PER; ++j) {
+                        seen[t][j] = old[t][j];
+                        if (g + t >= T.n || !(w.valid >> j & 1u)) continue;
+                        const uint32_t sh = (uint32_t)(bin[t][j] & 3) * 8u;
+                        if ((old[t][j] >> sh & 0xFFu) != 255u)
+                            seen[t][j] = atomicCAS(reinterpret_cast<uint32_t*>(T.base[g + t] + (bin[t][j] & ~3u)),
+                                                   old[t][j], old[t][j] + (1u << sh));
+                    }
+                }
+#pragma unroll
+                for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                    for (int j = 0; j < PER; ++j) {
+                        if (g + t >= T.n || !(w.valid >> j & 1u)) continue;
+                        old[t][j] = seen[t][j] == old[t][j]
+                                        ? old[t][j] >> ((uint32_t)(bin[t][j] & 3) * 8u) & 0xFFu
+                                        : byte_sat_inc(T.base[g + t], bin[t][j]);
+                    }
+                }
+            }
+            if (g == 0) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j)
+                    if (w.valid >> j & 1u)
+                        n_occ += T.kind == kBit ? !(old[0][j] >> (bin[0][j] & 31) & 1u) : old[0][j] == 0;
+            }
+            // claimed bins: the home slots together, the rest by claim_find
+            uint64_t slot[4][PER], key[4][PER];
+#pragma unroll
+            for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    if (g + t >= T.n || !(mask[j] >> (g + t < 7 ? g + t : 7) & 1u)) continue;
+                    slot[t][j] = claim_slot(cm, claim_key(gen, g + t, bin[t][j]));
+                    key[t][j] = cm.keys[slot[t][j]];
+                }
+            }
+            uint64_t val[4][PER];
+#pragma unroll
+            for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    if (g + t >= T.n || !(mask[j] >> (g + t < 7 ? g + t : 7) & 1u)) continue;
+                    const uint64_t k = claim_key(gen, g + t, bin[t][j]);
+                    val[t][j] = key[t][j] == k ? cm.vals[slot[t][j]] : claim_find(cm, k);
+                }
+            }
+#pragma unroll
+            for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    if (g + t >= T.n || !(mask[j] >> (g + t < 7 ? g + t : 7) & 1u)) continue;
+                    if (val[t][j] == claim_stamp(gen, (uint32_t)(w.s0 + j - b0))) is_new |= 1u << j;
+                }
+            }
+        }
+        n_new += (uint64_t)__popc(is_new);
+        add_to_reads(acc.out, w, is_new);
+        if (new_flags) {
+#pragma unroll
+            for (int j = 0; j < PER; ++j)
+                if (w.in >> j & 1u) new_flags[kmer_off[w.r[j]] + (w.s0 + j - w.rstart[j])] = is_new >> j & 1u;
+        }
+    }
+};
+
 // ------------------------------------------------------------ exact-set ops
 
-// Lookup pass: a window is fresh iff its value is absent at batch start.
+// Counts the windows whose value is absent (an upper bound of the keys that a
+// batch adds; fresh, when given, gets a byte per start).
 struct ExactLookupOp {
     ExactSet E;
     uint8_t* fresh;
@@ -680,63 +983,130 @@ struct ExactLookupOp {
     __device__ void operator()(int64_t s, uint32_t, int64_t, uint64_t fw, uint64_t rc, bool valid) {
         if (!valid) return;
         const uint8_t f = exact_find(E, kmer_value(fw, rc, canonical)) == kEmpty;
-        fresh[s - b0] = f;
+        if (fresh) fresh[s - b0] = f;
         n_fresh += f;
     }
     __device__ void begin_tile(int64_t) {}
     __device__ void flush() {}
 };
 
-// Insert pass: fresh windows insert their value and stamp its slot.  The
-// slot's stamp word is kept inverted (a new table is all ~0): an atomicMin of
-// ~(gen:32 | ~ordinal:32) keeps the largest stamp, which is the current
-// batch's smallest ordinal.
-struct ExactInsertOp {
+// Insert pass: finds or inserts every window's value and, when the value came
+// with this batch, lowers its slot's stamp to the window's.  The stamp word
+// is kept inverted (a new table is all ~0): ~(gen:32 | ~ordinal:32), so the
+// smallest stamp is the batch's smallest ordinal on that key, the window that
+// goetia's sequential insert reports as new (sparseppstorage.hh:92-97).  The
+// value the stamp had says what changed hands: none (~0), and the window is
+// its key's first so far; a larger ordinal, and newness moves here from the
+// read that holds that window.  Both are sums, so their order does not matter
+// and no second pass has to look every key up again (one random line access
+// per window less than claiming and then resolving).
+struct ExactAddOp {
     ExactSet E;
-    const uint8_t* fresh;
     int64_t b0;
-    int canonical;
     uint32_t gen;
+    const int64_t* off;
+    uint64_t n_reads;
     uint64_t* errors;
-    __device__ void operator()(int64_t s, uint32_t, int64_t, uint64_t fw, uint64_t rc, bool valid) {
-        if (!valid || !fresh[s - b0]) return;
-        const uint64_t slot = exact_insert(E, kmer_value(fw, rc, canonical), errors);
-        if (slot != kEmpty)
-            atomicMin((unsigned long long*)exact_stamp(E, slot),
-                      (unsigned long long)~claim_stamp(gen, (uint32_t)(s - b0)));
+    uint64_t* per_read;                    // new k-mers per read, or null
+    uint64_t n_new = 0;
+    uint64_t last_ins = 0;                 // position + 1 of the last inserted window
+
+    // The read holding start s (the last with off[r] <= s) loses a new window.
+    __device__ void take_back(int64_t s) {
+        if (!per_read) return;
+        uint64_t lo = 0, hi = n_reads - 1;
+        while (lo < hi) {
+            const uint64_t mid = (lo + hi + 1) >> 1;
+            if (off[mid] <= s) lo = mid; else hi = mid - 1;
+        }
+        atomicAdd((unsigned long long*)&per_read[lo], ~0ULL);
+    }
+    __device__ __forceinline__ uint64_t stamp(uint64_t slot, int64_t s) {
+        return atomicMin((unsigned long long*)exact_stamp(E, slot),
+                         (unsigned long long)~claim_stamp(gen, (uint32_t)(s - b0)));
+    }
+    // Whether the window at s became its key's first, from the stamp before it.
+    __device__ __forceinline__ bool won(uint64_t before, int64_t s) {
+        if (before == ~0ULL) {
+            n_new++;
+            return true;
+        }
+        if (before <= ~claim_stamp(gen, (uint32_t)(s - b0))) return false;
+        take_back(b0 + (int64_t)(uint32_t)before);
+        return true;
+    }
+    // The home slots of all windows are read together, then the free ones are
+    // claimed together, then the stamps: four windows of a thread take the
+    // latency of one.
+    static constexpr bool kTogether = true;
+    template <int PER>
+    __device__ void together(const Windows<PER>& w) {
+        uint64_t slot[PER];
+        ulonglong2 kv[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            slot[j] = w.h[j] == kEmpty ? 0 : exact_home(E, w.h[j]);
+            if (w.valid >> j & 1u) kv[j] = exact_pair(E, slot[j]);
+        }
+        uint64_t got[PER];
+        uint32_t todo = 0, fresh = 0;      // windows to probe on, windows of new keys
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            got[j] = kEmpty;
+            if (!(w.valid >> j & 1u)) continue;
+            last_ins = (uint64_t)(w.s0 + j - b0) + 1;
+            if (w.h[j] != kEmpty && kv[j].x == w.h[j])
+                fresh |= (stamp_is_fresh(kv[j].y, gen) ? 1u : 0u) << j;
+            else if (w.h[j] != kEmpty && kv[j].x == kEmpty)
+                got[j] = atomicCAS((unsigned long long*)exact_key(E, slot[j]), (unsigned long long)kEmpty,
+                                   (unsigned long long)w.h[j]);
+            else
+                todo |= 1u << j;
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (!(w.valid >> j & 1u)) continue;
+            if (!(todo >> j & 1u) && kv[j].x == kEmpty) {
+                if (got[j] == kEmpty || got[j] == w.h[j]) fresh |= 1u << j; else todo |= 1u << j;
+            }
+            if (todo >> j & 1u) {
+                const ExactHit x = exact_add(E, w.h[j], slot[j], gen, errors);
+                slot[j] = x.slot;
+                fresh |= (x.fresh ? 1u : 0u) << j;
+            }
+        }
+        uint64_t before[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) before[j] = fresh >> j & 1u ? stamp(slot[j], w.s0 + j) : 0;
+        uint32_t is_new = 0;
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            if (fresh >> j & 1u) is_new |= (won(before[j], w.s0 + j) ? 1u : 0u) << j;
+        add_to_reads(per_read, w, is_new);
     }
     __device__ void begin_tile(int64_t) {}
     __device__ void flush() {}
 };
 
-// Resolve pass: the fresh window whose stamp its slot kept (the batch's
-// smallest ordinal on that key) is the one goetia's sequential insert reports
-// as new (sparseppstorage.hh:92-97).
-struct ExactResolveOp {
+// New flags of an exact-set batch whose stamps are final: a window is new iff
+// its key's slot kept its stamp.
+struct ExactFlagOp {
     ExactSet E;
-    const uint8_t* fresh;
     int64_t b0;
     int canonical;
     uint32_t gen;
     const int64_t* kmer_off;
     uint8_t* new_flags;
-    ReadAcc acc;
-    uint64_t n_new = 0;
-    uint64_t last_ins = 0, last_new = 0;   // position + 1 of the last inserted / new window
     __device__ void operator()(int64_t s, uint32_t r, int64_t rstart, uint64_t fw, uint64_t rc, bool valid) {
         bool is_new = false;
-        if (valid && fresh[s - b0]) {
+        if (valid) {
             const uint64_t slot = exact_find(E, kmer_value(fw, rc, canonical));
             is_new = slot != kEmpty && *exact_stamp(E, slot) == ~claim_stamp(gen, (uint32_t)(s - b0));
         }
-        if (valid) last_ins = (uint64_t)(s - b0) + 1;
-        if (is_new) last_new = (uint64_t)(s - b0) + 1;
-        n_new += is_new;
-        acc.add(r, is_new);
-        if (new_flags) new_flags[kmer_off[r] + (s - rstart)] = is_new;
+        new_flags[kmer_off[r] + (s - rstart)] = is_new;
     }
     __device__ void begin_tile(int64_t) {}
-    __device__ void flush() { acc.flush(); }
+    __device__ void flush() {}
 };
 
 // ------------------------------------------------------------ query / degrees
@@ -793,6 +1163,56 @@ struct QueryOp {
             for (int i = threadIdx.x; i < n; i += kBlock) counts[k0 + i] = st->out[i];
         }
     }
+};
+
+// The query of a thread's windows together: every table read of all of them
+// is in flight at once, and counts are written straight out.
+struct QueryTogetherOp {
+    Tables T;
+    ExactSet E;
+    const int64_t* kmer_off;
+    int16_t* counts;
+    uint64_t* hashes;
+    static constexpr bool kTogether = true;
+    template <int PER>
+    __device__ void together(const Windows<PER>& w) {
+        int16_t c[PER];
+        if (T.kind == kExact) {
+            uint64_t key[PER];
+#pragma unroll
+            for (int j = 0; j < PER; ++j)
+                if (w.valid >> j & 1u) key[j] = *exact_key(E, w.h[j] == kEmpty ? 0 : exact_home(E, w.h[j]));
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                c[j] = 0;
+                if (!(w.valid >> j & 1u)) continue;
+                const bool settled = w.h[j] != kEmpty && (key[j] == w.h[j] || key[j] == kEmpty);
+                c[j] = (settled ? key[j] == w.h[j] : exact_find(E, w.h[j]) != kEmpty) ? 1 : 0;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < PER; ++j) c[j] = T.kind == kBit ? 1 : 255;
+            GT_FOR_TABLES(i, T) {
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    if (!(w.valid >> j & 1u)) continue;
+                    const uint64_t b = gt_fastmod(w.h[j], T.p[i], T.m[i]);
+                    const int16_t x = T.kind == kBit ? (int16_t)bit_get(T.base[i], b) : (int16_t)T.base[i][b];
+                    c[j] = x < c[j] ? x : c[j];
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (!(w.in >> j & 1u)) continue;
+            const int64_t k = kmer_off[w.r[j]] + (w.s0 + j - w.rstart[j]);
+            const bool valid = w.valid >> j & 1u;
+            if (counts) counts[k] = valid ? c[j] : (int16_t)-1;
+            if (hashes) hashes[k] = valid ? w.h[j] : 0;
+        }
+    }
+    __device__ void begin_tile(int64_t) {}
+    __device__ void flush() {}
 };
 
 // Hashing only: fw / rc / validity per window.
@@ -916,61 +1336,101 @@ struct DegreeOp {
 
 // ------------------------------------------------------------ kernels
 
+// An op whose windows start from stitched segments (see SegScratchT).
+template <class Op>
+struct Stitched : Op {
+    SegScratch* seg;
+    __device__ SegScratch* seg_scratch() { return seg; }
+};
+
+// Windows per thread of the kernels that take them together.
+constexpr int kPerSmall = 4;
+
 template <int PER>
 __global__ __launch_bounds__(kBlock) void claim_kernel(Reads R, Tables T, ClaimMap cm, uint8_t* fresh,
                                                      uint64_t* counters) {
-    __shared__ TileShared sh;
-    ClaimOp op{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, counters + kErrors};
-    walk_tiles<PER>(R, sh, op);
-    add_counter(counters + kFresh, op.n_fresh);
+    __shared__ TileSharedT<kBlock * PER> sh;
+    if constexpr (PER == kPerSmall) {
+        __shared__ SegScratch seg;
+        Stitched<ClaimTogetherOp> op{{{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, counters + kErrors}}, &seg};
+        walk_tiles<PER>(R, sh, op);
+        add_counter(counters + kFresh, op.n_fresh);
+    } else {
+        ClaimOp op{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, counters + kErrors};
+        walk_tiles<PER>(R, sh, op);
+        add_counter(counters + kFresh, op.n_fresh);
+    }
 }
 
 template <int PER>
 __global__ __launch_bounds__(kBlock) void apply_kernel(Reads R, Tables T, ClaimMap cm, const uint8_t* fresh,
                                                      uint64_t* n_new, uint8_t* new_flags, uint64_t* counters) {
-    __shared__ TileShared sh;
-    ApplyOp op{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, R.kmer_off, new_flags, ReadAcc{n_new}};
-    walk_tiles<PER>(R, sh, op);
-    add_counter(counters + kNUnique, op.n_new);
-    add_counter(counters + kNOccupied, op.n_occ);
+    __shared__ TileSharedT<kBlock * PER> sh;
+    uint64_t nn, occ;
+    if constexpr (PER == kPerSmall) {
+        __shared__ SegScratch seg;
+        Stitched<ApplyTogetherOp> op{
+            {{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, R.kmer_off, new_flags, ReadAcc{n_new}}}, &seg};
+        walk_tiles<PER>(R, sh, op);
+        nn = op.n_new;
+        occ = op.n_occ;
+    } else {
+        ApplyOp op{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, R.kmer_off, new_flags, ReadAcc{n_new}};
+        walk_tiles<PER>(R, sh, op);
+        nn = op.n_new;
+        occ = op.n_occ;
+    }
+    add_counter(counters + kNUnique, nn);
+    add_counter(counters + kNOccupied, occ);
 }
 
 template <int PER>
 __global__ __launch_bounds__(kBlock) void exact_lookup_kernel(Reads R, ExactSet E, uint8_t* fresh,
                                                             uint64_t* counters) {
-    __shared__ TileShared sh;
+    __shared__ TileSharedT<kBlock * PER> sh;
     ExactLookupOp op{E, fresh, R.b0, R.canonical};
     walk_tiles<PER>(R, sh, op);
     add_counter(counters + kFresh, op.n_fresh);
 }
 
-template <int PER>
-__global__ __launch_bounds__(kBlock) void exact_insert_kernel(Reads R, ExactSet E, const uint8_t* fresh,
-                                                            uint64_t* counters) {
-    __shared__ TileShared sh;
-    ExactInsertOp op{E, fresh, R.b0, R.canonical, current_gen(counters), counters + kErrors};
-    walk_tiles<PER>(R, sh, op);
+// One pass per batch, always four windows of a thread together (bound by the
+// random line accesses: a load, a compare-and-swap and an atomicMin of a
+// window's slot).  Looking every window up, then inserting and stamping the
+// absent ones, then looking them up again took 40.2 ms for the 264M bases of
+// 220k uneven reads at 5% substitutions; this takes 20 ms.
+__global__ __launch_bounds__(kBlock) void exact_add_kernel(Reads R, ExactSet E, uint64_t* n_new, uint64_t* counters) {
+    __shared__ TileSharedT<kBlock * kPerSmall> sh;
+    __shared__ SegScratch seg;
+    uint64_t n_reads;
+    int64_t n_bases;
+    batch_sizes(R, n_reads, n_bases);      // the reads that are there, not a captured batch's bound
+    Stitched<ExactAddOp> op{{E, R.b0, current_gen(counters), R.off, n_reads, counters + kErrors, n_new}, &seg};
+    walk_tiles<kPerSmall>(R, sh, op);
+    add_counter(counters + kNUnique, op.n_new);
+    max_counter(counters + kLastIns, op.last_ins);
 }
 
 template <int PER>
-__global__ __launch_bounds__(kBlock) void exact_resolve_kernel(Reads R, ExactSet E, const uint8_t* fresh,
-                                                             uint64_t* n_new, uint8_t* new_flags,
-                                                             uint64_t* counters) {
-    __shared__ TileShared sh;
-    ExactResolveOp op{E, fresh, R.b0, R.canonical, current_gen(counters), R.kmer_off, new_flags, ReadAcc{n_new}};
+__global__ __launch_bounds__(kBlock) void exact_flag_kernel(Reads R, ExactSet E, uint8_t* new_flags,
+                                                          const uint64_t* counters) {
+    __shared__ TileSharedT<kBlock * PER> sh;
+    ExactFlagOp op{E, R.b0, R.canonical, current_gen(counters), R.kmer_off, new_flags};
     walk_tiles<PER>(R, sh, op);
-    add_counter(counters + kNUnique, op.n_new);
-    max_counter(counters + kLastIns, op.last_ins);
-    max_counter(counters + kLastNew, op.last_new);
 }
 
 template <int PER>
 __global__ __launch_bounds__(kBlock) void query_kernel(Reads R, Tables T, ExactSet E, int16_t* counts,
                                                      uint64_t* hashes) {
     __shared__ TileSharedT<kBlock * PER> sh;
-    __shared__ QueryStage<kBlock * PER> st;
-    QueryOp<kBlock * PER> op{T, E, R, kBlock * PER, counts, hashes, &st};
-    walk_tiles<PER>(R, sh, op);
+    if constexpr (PER == kPerSmall) {
+        __shared__ SegScratch seg;
+        Stitched<QueryTogetherOp> op{{T, E, R.kmer_off, counts, hashes}, &seg};
+        walk_tiles<PER>(R, sh, op);
+    } else {
+        __shared__ QueryStage<kBlock * PER> st;
+        QueryOp<kBlock * PER> op{T, E, R, kBlock * PER, counts, hashes, &st};
+        walk_tiles<PER>(R, sh, op);
+    }
 }
 
 template <int PER>
@@ -1188,6 +1648,69 @@ __global__ __launch_bounds__(kScanBlock) void scan_add_kernel(int64_t* kmer_off,
     }
 }
 
+// Layout of a small batch by one workgroup: what tile_read_kernel and the
+// three steps above do, and optionally clears the per-read outputs and starts
+// the batch's first-touch generations.  A batch of a few thousand reads is
+// bound by its launches (about 5 us each, seven of them before the first
+// k-mer was hashed), not by this kernel's one CU.
+constexpr int kLayoutBlock = 1024;
+constexpr uint64_t kLayoutReads = 16 * kLayoutBlock;      // at most 16 reads per thread
+constexpr int64_t kLayoutTiles = 32 * kLayoutBlock;
+
+__global__ __launch_bounds__(kLayoutBlock) void layout_small_kernel(const int64_t* off, uint32_t n_reads,
+                                                                  int64_t n_bases, int K, uint32_t* tile_read,
+                                                                  uint32_t n_tiles, int64_t* kmer_off,
+                                                                  uint64_t* n_new, uint64_t* storage_gen,
+                                                                  uint64_t* claim_gen) {
+    __shared__ int64_t part[kLayoutBlock / 64];
+    const uint32_t tid = threadIdx.x;
+    // tile_read entries are all written for well-formed offsets; zero first so
+    // malformed offsets stay in bounds
+    for (uint32_t t = tid; t <= n_tiles; t += kLayoutBlock) tile_read[t] = 0;
+    if (n_new)
+        for (uint32_t r = tid; r < n_reads; r += kLayoutBlock) n_new[r] = 0;
+    if (tid == 0) {
+        if (storage_gen) *storage_gen += 1;
+        if (claim_gen) *claim_gen += 1;
+    }
+    __syncthreads();
+    const uint32_t per = (n_reads + kLayoutBlock - 1) / kLayoutBlock;
+    const uint32_t r0 = tid * per < n_reads ? tid * per : n_reads;
+    const uint32_t r1 = r0 + per < n_reads ? r0 + per : n_reads;
+    int64_t sum = 0;
+    int64_t at = r0 < r1 ? off[r0] : 0;
+    for (uint32_t r = r0; r < r1; ++r) {
+        const int64_t end = off[r + 1];
+        int64_t a = at < 0 ? 0 : (at > n_bases ? n_bases : at);
+        int64_t b = end < a ? a : (end > n_bases ? n_bases : end);
+        for (int64_t t = (a + kTileGrain - 1) / kTileGrain; t * kTileGrain < b && t < (int64_t)n_tiles; ++t)
+            tile_read[t] = r;
+        sum += end - at >= K ? end - at - K + 1 : 0;
+        at = end;
+    }
+    if (!kmer_off) return;
+    const int lane = tid & 63, wave = tid >> 6;
+    int64_t x = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int64_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) part[wave] = x;
+    __syncthreads();
+    int64_t run = x - sum, total = 0;
+    for (int v = 0; v < kLayoutBlock / 64; ++v) {
+        run += v < wave ? part[v] : 0;
+        total += part[v];
+    }
+    for (uint32_t r = r0; r < r1; ++r) {
+        const int64_t len = off[r + 1] - off[r];
+        kmer_off[r] = run;
+        run += len >= K ? len - K + 1 : 0;
+    }
+    if (tid == 0) kmer_off[n_reads] = total;
+}
+
 // Starts a new first-touch generation of a storage and of a claim map (one
 // lane; stream-ordered before the sub-batch that uses them).
 __global__ void bump_gen_kernel(uint64_t* storage_gen, uint64_t* claim_gen) {
@@ -1197,15 +1720,38 @@ __global__ void bump_gen_kernel(uint64_t* storage_gen, uint64_t* claim_gen) {
     }
 }
 
-// After an exact-set sub-batch: if it inserted anything, record whether its
-// last inserted value was already present (kNOccupied), and clear the
-// positions for the next sub-batch.
+// After an exact-set sub-batch of values: if it inserted anything, record
+// whether its last inserted value was already present (kNOccupied), and clear
+// the positions for the next sub-batch.
 __global__ void exact_tail_kernel(uint64_t* counters) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         const uint64_t li = counters[kLastIns], ln = counters[kLastNew];
         if (li) counters[kNOccupied] = li != ln;
         counters[kLastIns] = 0;
         counters[kLastNew] = 0;
+    }
+}
+
+// The same after a sub-batch of reads (one wave): its last inserted window was
+// new exactly when its key's slot kept that window's stamp.
+__global__ void exact_reads_tail_kernel(Reads R, ExactSet E, uint64_t* counters) {
+    const uint64_t li = counters[kLastIns];
+    if (li == 0 || blockIdx.x || threadIdx.x >= 64) return;
+    const uint8_t* w = R.seq + R.b0 + (int64_t)(li - 1);
+    uint64_t fw = 0, rc = 0;
+    for (int k = (int)threadIdx.x; k < R.K; k += 64) {
+        fw ^= gt_rotl(c_char_hash[w[k]], (unsigned)(R.K - 1 - k));
+        rc ^= gt_rotl(c_char_hash[gt_complement(w[k])], (unsigned)k);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        fw ^= __shfl_xor(fw, o, 64);
+        rc ^= __shfl_xor(rc, o, 64);
+    }
+    if (threadIdx.x == 0) {
+        const uint64_t slot = exact_find(E, kmer_value(fw, rc, R.canonical));
+        const uint64_t mine = ~claim_stamp(current_gen(counters), (uint32_t)(li - 1));
+        counters[kNOccupied] = slot == kEmpty || *exact_stamp(E, slot) != mine;
+        counters[kLastIns] = 0;
     }
 }
 
@@ -1229,13 +1775,18 @@ __global__ void bit_union_kernel(uint32_t* me, const uint32_t* other, uint64_t n
     add_counter(counters + kNOccupied, added);
 }
 
-// Rehash of an exact set into a larger one (stamps are per batch and not kept).
+// Rehash of an exact set into a larger one; every key it moves is an earlier
+// batch's (kOldStamp).
 __global__ void exact_rehash_kernel(ExactSet from, ExactSet to, uint64_t* counters) {
     for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < from.cap;
          i += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t k = *exact_key(from, i);
-        if (k != kEmpty) exact_insert(to, k, counters + kErrors);
+        if (k != kEmpty) {
+            const uint64_t slot = exact_insert(to, k, counters + kErrors);
+            if (slot != kEmpty) *exact_stamp(to, slot) = kOldStamp;
+        }
     }
+    if (blockIdx.x == 0 && threadIdx.x == 0 && *from.ones) *exact_stamp(to, to.cap) = kOldStamp;
 }
 
 // Compacts the keys of an exact set into out (count in *n).
@@ -2702,28 +3253,55 @@ void launch_fill_u64(uint64_t* p, uint64_t n, uint64_t v, hipStream_t s) {
     fill_u64_kernel<<<(unsigned)(g < 16384 ? g : 16384), 256, 0, s>>>(p, n, v);
 }
 
+// The same with four windows of a thread taken together for launches that ask
+// for it (make_launch).
+#define GT_TILE_LAUNCH_SMALL(L, kernel, ...)                                                  \
+    do {                                                                                      \
+        if ((L).per == kPerSmall)                                                             \
+            kernel<kPerSmall><<<tile_grid(L, R), kBlock, 0, (L).stream>>>(__VA_ARGS__);       \
+        else                                                                                  \
+            GT_TILE_LAUNCH(L, kernel, __VA_ARGS__);                                           \
+    } while (0)
+
+bool layout_is_small(uint64_t n_reads, int64_t n_bases) {
+    return n_reads <= kLayoutReads && (n_bases + kTileGrain - 1) / kTileGrain <= kLayoutTiles;
+}
+
+void launch_layout_small(const int64_t* off, uint64_t n_reads, int64_t n_bases, int K, uint32_t* tile_read,
+                         int64_t* kmer_off, uint64_t* n_new, uint64_t* storage_gen, uint64_t* claim_gen,
+                         hipStream_t s) {
+    const int64_t n_tiles = (n_bases + kTileGrain - 1) / kTileGrain;
+    layout_small_kernel<<<1, kLayoutBlock, 0, s>>>(off, (uint32_t)n_reads, n_bases, K, tile_read, (uint32_t)n_tiles,
+                                                  kmer_off, n_new, storage_gen, claim_gen);
+}
+
 void launch_claim(const Launch& L, const Reads& R, const Tables& T, const ClaimMap& cm, uint8_t* fresh,
                   uint64_t* counters) {
-    GT_TILE_LAUNCH(L, claim_kernel, R, T, cm, fresh, counters);
+    GT_TILE_LAUNCH_SMALL(L, claim_kernel, R, T, cm, fresh, counters);
 }
 
 void launch_apply(const Launch& L, const Reads& R, const Tables& T, const ClaimMap& cm, const uint8_t* fresh,
                   uint64_t* n_new, uint8_t* new_flags, uint64_t* counters) {
-    GT_TILE_LAUNCH(L, apply_kernel, R, T, cm, fresh, n_new, new_flags, counters);
+    GT_TILE_LAUNCH_SMALL(L, apply_kernel, R, T, cm, fresh, n_new, new_flags, counters);
 }
 
 void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* fresh, uint64_t* counters) {
     GT_TILE_LAUNCH(L, exact_lookup_kernel, R, E, fresh, counters);
 }
 
-void launch_exact_insert(const Launch& L, const Reads& R, const ExactSet& E, const uint8_t* fresh,
-                         uint64_t* counters) {
-    GT_TILE_LAUNCH(L, exact_insert_kernel, R, E, fresh, counters);
+void launch_exact_add(const Launch& L, const Reads& R, const ExactSet& E, uint64_t* n_new, uint64_t* counters) {
+    Launch small = L;
+    small.per = kPerSmall;
+    exact_add_kernel<<<tile_grid(small, R), kBlock, 0, L.stream>>>(R, E, n_new, counters);
 }
 
-void launch_exact_resolve(const Launch& L, const Reads& R, const ExactSet& E, const uint8_t* fresh,
-                          uint64_t* n_new, uint8_t* new_flags, uint64_t* counters) {
-    GT_TILE_LAUNCH(L, exact_resolve_kernel, R, E, fresh, n_new, new_flags, counters);
+void launch_exact_flags(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* new_flags,
+                        const uint64_t* counters) {
+    GT_TILE_LAUNCH(L, exact_flag_kernel, R, E, new_flags, counters);
+}
+
+void launch_exact_reads_tail(const Reads& R, const ExactSet& E, uint64_t* counters, hipStream_t s) {
+    exact_reads_tail_kernel<<<1, 64, 0, s>>>(R, E, counters);
 }
 
 void launch_bump_gen(uint64_t* storage_gen, uint64_t* claim_gen, hipStream_t s) {
@@ -2736,7 +3314,7 @@ void launch_exact_tail(uint64_t* counters, hipStream_t s) {
 
 void launch_query(const Launch& L, const Reads& R, const Tables& T, const ExactSet& E, int16_t* counts,
                   uint64_t* hashes) {
-    GT_TILE_LAUNCH(L, query_kernel, R, T, E, counts, hashes);
+    GT_TILE_LAUNCH_SMALL(L, query_kernel, R, T, E, counts, hashes);
 }
 
 void launch_hash(const Launch& L, const Reads& R, uint64_t* fw, uint64_t* rc, uint8_t* valid) {

@@ -10,13 +10,19 @@ namespace gt {
 struct Launch {
     int grid;              // workgroups for tile walkers (persistent grid)
     hipStream_t stream;
-    int per;               // windows per thread: 8, 16 or 32
+    int per;               // windows per thread: 8, 16 or 32; 4 = taken together (small batches)
 };
 
 void launch_tile_read(const int64_t* off, uint64_t n_reads, int64_t n_bases, uint32_t* tile_read,
                       int64_t n_tiles, const int64_t* dyn, hipStream_t s);
 void launch_kmer_offsets(const int64_t* off, uint64_t n_reads, int K, int64_t* kmer_off,
                          int64_t* block_sums, const int64_t* dyn, hipStream_t s);
+// One-launch layout of small batches (layout_is_small): tile_read, kmer_off
+// and, where given, cleared n_new and the two generation bumps.
+bool layout_is_small(uint64_t n_reads, int64_t n_bases);
+void launch_layout_small(const int64_t* off, uint64_t n_reads, int64_t n_bases, int K, uint32_t* tile_read,
+                         int64_t* kmer_off, uint64_t* n_new, uint64_t* storage_gen, uint64_t* claim_gen,
+                         hipStream_t s);
 void launch_bump_gen(uint64_t* storage_gen, uint64_t* claim_gen, hipStream_t s);
 uint64_t scan_block_count(uint64_t n_reads);
 void launch_fill_u64(uint64_t* p, uint64_t n, uint64_t v, hipStream_t s);
@@ -26,11 +32,11 @@ void launch_claim(const Launch& L, const Reads& R, const Tables& T, const ClaimM
 void launch_apply(const Launch& L, const Reads& R, const Tables& T, const ClaimMap& cm, const uint8_t* fresh,
                   uint64_t* n_new, uint8_t* new_flags, uint64_t* counters);
 void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* fresh, uint64_t* counters);
-void launch_exact_insert(const Launch& L, const Reads& R, const ExactSet& E, const uint8_t* fresh,
-                         uint64_t* counters);
+void launch_exact_add(const Launch& L, const Reads& R, const ExactSet& E, uint64_t* n_new, uint64_t* counters);
+void launch_exact_flags(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* new_flags,
+                        const uint64_t* counters);
 void launch_exact_tail(uint64_t* counters, hipStream_t s);
-void launch_exact_resolve(const Launch& L, const Reads& R, const ExactSet& E, const uint8_t* fresh,
-                          uint64_t* n_new, uint8_t* new_flags, uint64_t* counters);
+void launch_exact_reads_tail(const Reads& R, const ExactSet& E, uint64_t* counters, hipStream_t s);
 void launch_query(const Launch& L, const Reads& R, const Tables& T, const ExactSet& E, int16_t* counts,
                   uint64_t* hashes);
 void launch_hash(const Launch& L, const Reads& R, uint64_t* fw, uint64_t* rc, uint8_t* valid);

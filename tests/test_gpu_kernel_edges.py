@@ -93,3 +93,65 @@ def test_per_read_sums_and_solid_reads_at_every_length(oracle, monkeypatch, spre
             c = np.asarray(o2.insert_and_query_sequence(s, K))
             share = float(np.float32(int((c < thr).sum())) / np.float32(len(c)))
             assert passed[r] == (not share >= 1.0 - float(np.float32(prop)))
+
+
+@pytest.mark.parametrize('kind,n_tables', [(1, 1), (1, 4), (1, 6), (2, 2), (2, 4), (2, 9), (3, 0)])
+@pytest.mark.parametrize('K,mode', [(21, N.MODE_RAW), (31, N.MODE_SKIP_N), (255, N.MODE_RAW)])
+def test_small_batches_take_windows_together(oracle, kind, n_tables, K, mode):
+    """Batches around one tile of 1024 starts, hot k-mers (several windows of a
+    thread on one bin or slot), reads below K, N bases, and a second batch over
+    the first one's keys: n_new, flags, counts, counters, tables."""
+    sizes = [4001, 4003, 4007, 4013, 4019, 4021, 4027, 4049, 4051][:n_tables]
+    for lengths in ([K], [K - 1, K + 3], [300, 0, 421, 300, 3], [1024], [1025], [257] * 40, [150] * 300):
+        g, o = _pair(oracle, kind, sizes, K, mode=mode)
+        for seed in (1, 2):
+            b = _reads(seed, lengths, genome=max(500, max(lengths)), n_rate=0.003)
+            hot = np.frombuffer(b'A' * (K + 40) + b'ACAC' * 100, np.uint8)
+            b = ReadBatch(np.concatenate([b.seq, hot]), np.append(b.offsets, b.n_bases + len(hot)))
+            _, e_new, e_flags = o.insert_reads_flags(b.seq, b.offsets, K, True, mode)
+            n_new, flags = g.insert_sequences(b, new_flags=True)
+            np.testing.assert_array_equal(n_new, e_new)
+            np.testing.assert_array_equal(flags, np.asarray(e_flags, bool))
+            np.testing.assert_array_equal(g.query_sequences(b), o.query_reads(b.seq, b.offsets, K, True, mode))
+            assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+        if kind == 3:
+            np.testing.assert_array_equal(g.S.keys(), np.sort(o.exact_keys()))
+        else:
+            for x, y in zip(g.get_raw(), o.tables()):
+                np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize('n_reads', [1, 1023, 1025, 16384, 16385])
+def test_layout_of_small_batches(oracle, n_reads):
+    """Either side of the one-launch layout's limit: packed results of reads of
+    0 to 60 bases, and one long read over many tiles."""
+    K = 21
+    rng = np.random.default_rng(n_reads)
+    lengths = rng.integers(0, 60, n_reads)
+    lengths[n_reads // 2] = 9000
+    b = _reads(n_reads, list(lengths), genome=9500)
+    g, o = _pair(oracle, 2, [50021, 50023], K)
+    _, e_new = o.insert_reads(b.seq, b.offsets, K)
+    np.testing.assert_array_equal(g.insert_sequences(b), e_new)
+    np.testing.assert_array_equal(g.query_sequences(b), o.query_reads(b.seq, b.offsets, K))
+
+
+def test_exact_set_moves_newness_and_grows(oracle):
+    """Keys of earlier batches stay old through a rehash (n_new 0 when they
+    come again), the all-ones key's stand-in included, and newness ends at the
+    smallest window when many reads hold the same keys."""
+    K = 25
+    g, o = _pair(oracle, 3, (), K)
+    for step, n in enumerate((40, 400, 4000, 40, 4000)):
+        b = _reads(100 + (step % 3), [80] * n, genome=300 * (1 + n // 10), sub=0.0)
+        for _ in range(2):
+            _, e_new = o.insert_reads(b.seq, b.offsets, K)
+            np.testing.assert_array_equal(g.insert_sequences(b), e_new)
+            assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+    for v in (0, 2 ** 64 - 1, 2 ** 64 - 1, 5):
+        assert g.S.insert(v) == o.insert(v)
+    b = _reads(7, [120] * 30000, genome=2_000_000)
+    _, e_new = o.insert_reads(b.seq, b.offsets, K)
+    np.testing.assert_array_equal(g.insert_sequences(b), e_new)
+    assert not g.S.insert(2 ** 64 - 1) and not o.insert(2 ** 64 - 1)
+    assert g.n_unique() == o.n_unique
