@@ -213,6 +213,8 @@ uint32_t log2u(uint64_t p) {
 struct Scratch {
     DevBuf claim_keys, claim_vals, claim_gen;
     uint64_t claim_cap = 0;
+    DevBuf claim_direct;               // direct claim map: a stamp per bin (generations from claim_gen)
+    bool direct = false;               // the running call claims directly (prepare_claims)
     uint64_t claim_gen_issued = 0;     // bumps enqueued so far (the device counter follows it)
     DevBuf fresh, tile_read, kmer_off, scan_blocks;
     // binned insert: events of the two partition passes, first-pass digit
@@ -492,26 +494,52 @@ int alloc_claims(Scratch& sc, uint64_t want, hipStream_t s) {
     launch_fill_u64(sc.claim_keys.as<uint64_t>(), want, 0, s);
     launch_fill_u64(sc.claim_vals.as<uint64_t>(), want, 0, s);
     launch_fill_u64(sc.claim_gen.as<uint64_t>(), 1, 0, s);
+    // stamps of the direct map carry the generations that start over here
+    if (sc.claim_direct.p) launch_fill_u64(sc.claim_direct.as<uint64_t>(), sc.claim_direct.bytes / 8, 0, s);
     GT_HIP(hipGetLastError());
     sc.claim_cap = want;
     sc.claim_gen_issued = 0;
     return GT_OK;
 }
 
+// Bins of a storage whose batches of n_starts starts claim them directly (a
+// stamp word per bin), or 0: when that takes no more memory than the hashed
+// map's slots for the batch, or no more than 2^22 words (goetia's default
+// tables, 4 x 1e6 bins).
+uint64_t direct_claim_bins(const gt_storage* st, const Scratch& sc, uint64_t n_starts) {
+    if (sc.fixed || st->kind == kExact) return 0;
+    uint64_t bins = 0;
+    for (uint64_t p : st->sizes) bins += p;
+    return bins <= std::max<uint64_t>(1ULL << 22, 2 * (uint64_t)st->n_tables * n_starts) && bins < (1ULL << 32) ? bins
+                                                                                                              : 0;
+}
+
 // Largest sub-batch (in start positions, a multiple of kTileMax) whose claims fit
 // the claim map at load factor <= 1/2; grows the claim map and fresh buffer
-// as needed for this call (fixed scratch only checks).
-int prepare_claims(Scratch& sc, int kind, uint32_t n_tables, uint64_t n_starts, uint64_t* sub, hipStream_t s) {
+// as needed for this call (fixed scratch only checks).  sc.direct says which
+// map the call's claims go to; a direct map's older stamps, of this or other
+// storages' batches on the scratch, are earlier generations.
+int prepare_claims(gt_storage* st, Scratch& sc, uint64_t n_starts, uint64_t* sub, hipStream_t s) {
     const uint64_t kMaxClaimCap = 1ULL << 29;      // 8 GiB of claim slots
     const uint64_t kMinClaimCap = 1ULL << 16;
-    const uint64_t per = std::max<uint32_t>(n_tables, 1);
+    const uint64_t per = std::max<uint32_t>(st->n_tables, 1);
     const uint64_t cap = sub_batch_cap();
     const uint64_t starts = (n_starts + kTileMax - 1) / kTileMax * kTileMax;
-    if (kind == kExact) {
+    const uint64_t direct = direct_claim_bins(st, sc, n_starts);
+    sc.direct = direct != 0;
+    if (st->kind == kExact || direct) {
         uint64_t sb = std::min<uint64_t>(starts, 1ULL << 31);
         if (cap) sb = std::min(sb, cap);
         if (sb == 0) return fail(GT_ERR_INTERNAL, "scratch too small");
-        if (!sc.claim_cap) GT_TRY(alloc_claims(sc, 2, s));   // unused by the exact set; a valid view
+        if (!sc.claim_cap) GT_TRY(alloc_claims(sc, 2, s));   // the generation counter, and a valid view
+        if (direct) {
+            GT_TRY(sc.fresh.ensure(sb));
+            if (sc.claim_direct.bytes < direct * sizeof(uint64_t)) {
+                GT_TRY(sc.claim_direct.ensure(direct * sizeof(uint64_t)));
+                launch_fill_u64(sc.claim_direct.as<uint64_t>(), sc.claim_direct.bytes / 8, 0, s);
+                GT_HIP(hipGetLastError());
+            }
+        }
         *sub = sb;
         return GT_OK;
     }
@@ -528,10 +556,6 @@ int prepare_claims(Scratch& sc, int kind, uint32_t n_tables, uint64_t n_starts, 
     if (sb == 0) return fail(GT_ERR_INTERNAL, "claim map too small");
     *sub = sb;
     return GT_OK;
-}
-
-int prepare_claims(gt_storage* st, uint64_t n_starts, uint64_t* sub, hipStream_t s) {
-    return prepare_claims(st->own, st->kind, st->n_tables, n_starts, sub, s);
 }
 
 // Enqueues the next first-touch generation of the storage (exact-set stamps,
@@ -555,11 +579,22 @@ int next_gen(gt_storage* st, Scratch& sc, hipStream_t s, bool bumped = false) {
     return GT_OK;
 }
 
-ClaimMap claim_view(const Scratch& sc) {
+ClaimMap claim_view(const gt_storage* st, const Scratch& sc) {
     ClaimMap cm{};
+    cm.gen = sc.claim_gen.as<uint64_t>();
+    if (sc.direct) {
+        cm.vals = sc.claim_direct.as<uint64_t>();
+        cm.cap = 1;
+        cm.direct = 1;
+        uint64_t at = 0;
+        for (uint32_t i = 0; i < st->n_tables; ++i) {
+            cm.dbase[i] = (uint32_t)at;
+            at += st->sizes[i];
+        }
+        return cm;
+    }
     cm.keys = sc.claim_keys.as<uint64_t>();
     cm.vals = sc.claim_vals.as<uint64_t>();
-    cm.gen = sc.claim_gen.as<uint64_t>();
     cm.cap = sc.claim_cap;
     cm.log2cap = log2u(sc.claim_cap);
     return cm;
@@ -601,7 +636,8 @@ Launch make_launch(const gt_storage* st, hipStream_t s) { return make_launch(st-
 // tuned tile shape leaves CUs without waves to hide a window's chain of table
 // accesses behind, so a thread takes four windows together instead (the
 // kernels' kPerSmall form): 500 reads into a 4 x 1e6 Bloom filter went from
-// 365 to 191 us, 4167 reads against 4 x 2^28 counts from 86 to 58 us.
+// 365 to 93 us (with direct claims), 4167 reads against 4 x 2^28 counts from
+// 86 to 58 us.
 constexpr uint64_t kSmallStarts = 1ULL << 22;
 Launch make_launch(const gt_storage* st, uint64_t n_starts, hipStream_t s) {
     Launch L = make_launch(st->kind, s);
@@ -620,7 +656,7 @@ int enqueue_subbatch(gt_storage* st, Scratch& sc, const Launch& L, const Reads& 
     uint64_t* ctr = st->counters.as<uint64_t>();
     uint8_t* fresh = sc.fresh.as<uint8_t>();
     GT_TRY(next_gen(st, sc, s, bumped));
-    const ClaimMap cm = claim_view(sc);
+    const ClaimMap cm = claim_view(st, sc);
     if (st->kind == kExact) {
         const uint64_t nstarts = (uint64_t)(Rs.b1 - Rs.b0);
         if (growth && 2 * (st->ecount_ub + nstarts) > st->ecap) {
@@ -915,7 +951,7 @@ int dbg_insert_impl(gt_storage* st, Scratch& sc, Reads R, uint64_t* n_new, uint8
     uint64_t sub = 0;
     GenBump bump;
     if (!binned) {
-        GT_TRY(prepare_claims(sc, st->kind, st->n_tables, (uint64_t)R.n_bases, &sub, s));
+        GT_TRY(prepare_claims(st, sc, (uint64_t)R.n_bases, &sub, s));
         bump.storage_gen = st->counters.as<uint64_t>() + kGen;
         bump.claim_gen = sc.claim_gen.as<uint64_t>();
     }
@@ -930,7 +966,7 @@ int dbg_insert_impl(gt_storage* st, Scratch& sc, Reads R, uint64_t* n_new, uint8
         sc.bin_dig2.release();
         sc.bin_flags.release();
         sc.bin_vq.release();
-        GT_TRY(prepare_claims(sc, st->kind, st->n_tables, (uint64_t)R.n_bases, &sub, s));
+        GT_TRY(prepare_claims(st, sc, (uint64_t)R.n_bases, &sub, s));
     }
     const Launch L = make_launch(st, std::min<uint64_t>(sub, (uint64_t)R.n_bases), s);
     for (int64_t b0 = 0; b0 < R.n_bases; b0 += (int64_t)sub) {
@@ -958,7 +994,7 @@ int hashes_insert_impl(gt_storage* st, const uint64_t* h, uint64_t n, uint8_t* i
     const Launch L = make_launch(st, s);
     uint64_t* ctr = st->counters.as<uint64_t>();
     uint64_t sub = 0;
-    GT_TRY(prepare_claims(st, n, &sub, s));
+    GT_TRY(prepare_claims(st, st->own, n, &sub, s));
     if (st->kind == kExact) GT_TRY(st->own.fresh.ensure(std::min(sub, n)));
     for (uint64_t i0 = 0; i0 < n; i0 += sub) {
         const uint64_t m = std::min<uint64_t>(sub, n - i0);
@@ -974,7 +1010,7 @@ int hashes_insert_impl(gt_storage* st, const uint64_t* h, uint64_t n, uint8_t* i
             launch_exact_tail(ctr, s);
         } else {
             const Tables T = st->tables_view();
-            const ClaimMap cm = claim_view(st->own);
+            const ClaimMap cm = claim_view(st, st->own);
             launch_hash_claim(L, h + i0, m, T, cm, fresh, ctr);
             launch_hash_apply(L, h + i0, m, T, cm, fresh, is_new ? is_new + i0 : nullptr, ctr);
         }
@@ -2212,7 +2248,7 @@ int gt_autotune(gt_storage* st, uint16_t K, int canonical, int mode, const uint8
     Reads R = make_reads(seq, offsets, n_reads, n_bases, K, mode, canonical);
     GT_TRY(prepare_reads(st, R, true, s));
     uint64_t sub = 0;
-    GT_TRY(prepare_claims(st, n_bases, &sub, s));
+    GT_TRY(prepare_claims(st, st->own, n_bases, &sub, s));
     R.b1 = std::min<int64_t>(R.n_bases, (int64_t)sub);
     DevBuf counts;
     GT_TRY(counts.ensure((size_t)std::max<uint64_t>(n_bases, 1) * sizeof(int16_t)));
@@ -2245,7 +2281,7 @@ int gt_autotune(gt_storage* st, uint16_t K, int canonical, int mode, const uint8
                 if (st->kind == kExact) {
                     launch_exact_lookup(L, R, st->exact_view(), nullptr, ctr);
                 } else {
-                    launch_claim(L, R, st->tables_view(), claim_view(st->own), st->own.fresh.as<uint8_t>(), ctr);
+                    launch_claim(L, R, st->tables_view(), claim_view(st, st->own), st->own.fresh.as<uint8_t>(), ctr);
                 }
                 launch_query(L, R, st->tables_view(), st->exact_or_empty(), counts.as<int16_t>(), nullptr);
                 GT_HIP(hipEventRecord(e1, s));

@@ -70,9 +70,14 @@ __host__ __device__ inline uint64_t* exact_stamp(const ExactSet& es, uint64_t sl
 // gen:28 | table:4 | bin:32, value word = gen:32 | ~ordinal:32 (atomicMax).
 // The generation is a device counter owned with the map (a map may serve
 // several storages, so it cannot use a storage's generation).
+// A direct map has a value word per bin (bin b of table i at
+// vals[dbase[i] + b]) and no keys: a claim is then one atomicMax, with nothing
+// to probe.
 struct ClaimMap {
     uint64_t* keys;
     uint64_t* vals;
+    uint32_t direct;
+    uint32_t dbase[kMaxTables];
     const uint64_t* gen;
     uint64_t cap;
     uint32_t log2cap;

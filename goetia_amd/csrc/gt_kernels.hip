@@ -113,6 +113,11 @@ __device__ __forceinline__ uint32_t claim_gen(const ClaimMap& cm) {
     return (uint32_t)__hip_atomic_load(cm.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A claim in a direct map.
+__device__ __forceinline__ void claim_direct(const ClaimMap& cm, uint32_t table, uint64_t bin, uint64_t stamp) {
+    atomicMax((unsigned long long*)&cm.vals[cm.dbase[table] + bin], (unsigned long long)stamp);
+}
+
 __device__ void claim_insert(const ClaimMap& cm, uint64_t key, uint64_t stamp, uint64_t* errors) {
     const uint64_t mask = cm.cap - 1;
     const uint64_t gen = key >> 36;
@@ -341,7 +346,7 @@ using TileShared = TileSharedT<kTileMax>;
 
 template <class Sh>
 __device__ __forceinline__ void load_char_tables(Sh& sh) {
-    for (int i = threadIdx.x; i < 256; i += kBlock) {
+    for (int i = threadIdx.x; i < 256; i += (int)blockDim.x) {
         sh.tf[i] = c_char_hash[i];
         sh.tr[i] = c_char_hash[gt_complement((unsigned char)i)];
     }
@@ -391,16 +396,15 @@ struct SegScratchT {
     uint64_t pr[N], qr[N];
     uint8_t bf[N], bq[N];   // non-ACGT bytes in the segment / its prefix
 };
-using SegScratch = SegScratchT<kBlock + kSegExtra>;
 
 // The op's LDS for stitched starts (free while the windows are visited), or
 // null for ops without it (those roll K bytes per start).
-template <class Op>
+template <int BLK, class Op>
 __device__ __forceinline__ auto seg_scratch(Op& op, int) -> decltype(op.seg_scratch()) {
     return op.seg_scratch();
 }
-template <class Op>
-__device__ __forceinline__ SegScratch* seg_scratch(Op&, long) {
+template <int BLK, class Op>
+__device__ __forceinline__ SegScratchT<BLK + kSegExtra>* seg_scratch(Op&, long) {
     return nullptr;
 }
 
@@ -508,7 +512,7 @@ __device__ void walk_tiles(const Reads& R, Sh& sh, Op& op) {
         __syncthreads();
 
         op.begin_tile(t0);
-        auto* sg = seg_scratch(op, 0);
+        auto* sg = seg_scratch<BLK>(op, 0);
         const int n_seg = (K + PER - 1) / PER;
         if (sg) {
             static_assert(std::remove_pointer_t<decltype(sg)>::kSegs >= BLK + kSegExtra, "segment scratch too small");
@@ -517,6 +521,7 @@ __device__ void walk_tiles(const Reads& R, Sh& sh, Op& op) {
         if (sg) {
             const int L = K - (n_seg - 1) * PER;
             seg_values<PER>(sh, sg, tid, L);
+            static_assert(BLK >= kSegExtra, "one thread per segment past the tile");
             if (tid < n_seg - 1) seg_values<PER>(sh, sg, BLK + tid, L);
             __syncthreads();
         }
@@ -717,7 +722,10 @@ struct ClaimOp {
             const bool empty = T.kind == kBit ? !bit_get(T.base[i], b) : T.base[i][b] == 0;
             if (empty) {
                 mask |= (uint8_t)(1u << (i < 7 ? i : 7));
-                claim_insert(cm, claim_key(gen, i, b), claim_stamp(gen, ord), errors);
+                if (cm.direct)
+                    claim_direct(cm, i, b, claim_stamp(gen, ord));
+                else
+                    claim_insert(cm, claim_key(gen, i, b), claim_stamp(gen, ord), errors);
             }
         }
         fresh[s - b0] = mask;
@@ -728,9 +736,11 @@ struct ClaimOp {
 };
 
 // The claim pass over a thread's windows together: the bins of four tables of
-// every window are read together, then the claim slots of the empty ones, then
-// the slots are taken, then stamped.  A lookup that meets another key is
-// finished by claim_insert.
+// every window are read together, then the empty ones are claimed in rounds, a
+// probe of each per round.  Bound by the latency of those dependent accesses:
+// finishing a probe that met another key on its own, one after another (a wave
+// nearly always has some), took 112 us for 500 reads into a 4 x 1e6 Bloom
+// filter.
 struct ClaimTogetherOp : ClaimOp {
     static constexpr bool kTogether = true;
     template <int PER>
@@ -755,45 +765,64 @@ struct ClaimTogetherOp : ClaimOp {
                     }
                 }
             }
-            uint64_t slot[4][PER], cur[4][PER];
-            uint32_t empty = 0;                            // bit t * PER + j
+            uint64_t slot[4][PER];
+            uint32_t open = 0;                             // bit t * PER + j: a bin to claim
 #pragma unroll
             for (uint32_t t = 0; t < 4; ++t) {
 #pragma unroll
                 for (int j = 0; j < PER; ++j) {
                     if (T.kind == kBit ? word[t][j] & 1u : word[t][j]) continue;
-                    empty |= 1u << (t * PER + j);
                     mask[j] |= (uint8_t)(1u << (g + t < 7 ? g + t : 7));
+                    if (cm.direct) {
+                        claim_direct(cm, g + t, bin[t][j], claim_stamp(gen, (uint32_t)(w.s0 + j - b0)));
+                        continue;
+                    }
+                    open |= 1u << (t * PER + j);
                     slot[t][j] = claim_slot(cm, claim_key(gen, g + t, bin[t][j]));
-                    cur[t][j] = load_relaxed(&cm.keys[slot[t][j]]);
                 }
             }
-            // as the first steps of claim_insert: a slot of an earlier
-            // generation is free; cur = the key found in it
+            // claim_insert for all of them, a probe of each per round: a slot
+            // of an earlier generation is free, one that changed but still is
+            // one is looked at again
+            for (uint64_t round = 0; open; ++round) {
+                if (round > cm.cap) {
+                    atomicOr((unsigned long long*)errors, (unsigned long long)kErrClaim);
+                    break;
+                }
+                uint64_t cur[4][PER];
 #pragma unroll
-            for (uint32_t t = 0; t < 4; ++t) {
+                for (uint32_t t = 0; t < 4; ++t) {
 #pragma unroll
-                for (int j = 0; j < PER; ++j) {
-                    if (!(empty >> (t * PER + j) & 1u)) continue;
-                    const uint64_t key = claim_key(gen, g + t, bin[t][j]);
-                    if ((cur[t][j] >> 36) != (key >> 36)) {
-                        const uint64_t prev = atomicCAS((unsigned long long*)&cm.keys[slot[t][j]],
-                                                        (unsigned long long)cur[t][j], (unsigned long long)key);
-                        cur[t][j] = prev == cur[t][j] ? key : prev;
+                    for (int j = 0; j < PER; ++j)
+                        if (open >> (t * PER + j) & 1u) cur[t][j] = load_relaxed(&cm.keys[slot[t][j]]);
+                }
+#pragma unroll
+                for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                    for (int j = 0; j < PER; ++j) {
+                        if (!(open >> (t * PER + j) & 1u)) continue;
+                        const uint64_t key = claim_key(gen, g + t, bin[t][j]);
+                        if ((cur[t][j] >> 36) != (key >> 36)) {
+                            const uint64_t prev = atomicCAS((unsigned long long*)&cm.keys[slot[t][j]],
+                                                            (unsigned long long)cur[t][j], (unsigned long long)key);
+                            cur[t][j] = prev == cur[t][j] ? key : prev;
+                        }
                     }
                 }
-            }
 #pragma unroll
-            for (uint32_t t = 0; t < 4; ++t) {
+                for (uint32_t t = 0; t < 4; ++t) {
 #pragma unroll
-                for (int j = 0; j < PER; ++j) {
-                    if (!(empty >> (t * PER + j) & 1u)) continue;
-                    const uint64_t key = claim_key(gen, g + t, bin[t][j]);
-                    const uint64_t stamp = claim_stamp(gen, (uint32_t)(w.s0 + j - b0));
-                    if (cur[t][j] == key)
-                        atomicMax((unsigned long long*)&cm.vals[slot[t][j]], (unsigned long long)stamp);
-                    else
-                        claim_insert(cm, key, stamp, errors);
+                    for (int j = 0; j < PER; ++j) {
+                        if (!(open >> (t * PER + j) & 1u)) continue;
+                        const uint64_t key = claim_key(gen, g + t, bin[t][j]);
+                        if (cur[t][j] == key) {
+                            atomicMax((unsigned long long*)&cm.vals[slot[t][j]],
+                                      (unsigned long long)claim_stamp(gen, (uint32_t)(w.s0 + j - b0)));
+                            open &= ~(1u << (t * PER + j));
+                        } else if ((cur[t][j] >> 36) == (key >> 36)) {
+                            slot[t][j] = (slot[t][j] + 1) & (cm.cap - 1);
+                        }
+                    }
                 }
             }
         }
@@ -856,7 +885,7 @@ struct ApplyOp {
                 if (i == 0 && before == 0) n_occ++;
             }
             if (!is_new && (mask & (1u << (i < 7 ? i : 7)))) {
-                is_new = claim_find(cm, claim_key(gen, i, b)) == stamp;
+                is_new = (cm.direct ? cm.vals[cm.dbase[i] + b] : claim_find(cm, claim_key(gen, i, b))) == stamp;
             }
         }
         n_new += is_new;
@@ -930,33 +959,57 @@ struct ApplyTogetherOp : ApplyOp {
                     if (w.valid >> j & 1u)
                         n_occ += T.kind == kBit ? !(old[0][j] >> (bin[0][j] & 31) & 1u) : old[0][j] == 0;
             }
-            // claimed bins: the home slots together, the rest by claim_find
-            uint64_t slot[4][PER], key[4][PER];
+            // claimed bins: claim_find for all of them, a probe of each per round
+            uint64_t slot[4][PER], stamp[4][PER];
+            uint32_t open = 0;
 #pragma unroll
             for (uint32_t t = 0; t < 4; ++t) {
 #pragma unroll
                 for (int j = 0; j < PER; ++j) {
+                    stamp[t][j] = 0;                       // no window's stamp (generations start at 1)
                     if (g + t >= T.n || !(mask[j] >> (g + t < 7 ? g + t : 7) & 1u)) continue;
+                    if (cm.direct) {
+                        stamp[t][j] = cm.vals[cm.dbase[g + t] + bin[t][j]];
+                        continue;
+                    }
+                    open |= 1u << (t * PER + j);
                     slot[t][j] = claim_slot(cm, claim_key(gen, g + t, bin[t][j]));
-                    key[t][j] = cm.keys[slot[t][j]];
                 }
             }
-            uint64_t val[4][PER];
+            if (cm.direct) {
 #pragma unroll
-            for (uint32_t t = 0; t < 4; ++t) {
+                for (uint32_t t = 0; t < 4; ++t) {
 #pragma unroll
-                for (int j = 0; j < PER; ++j) {
-                    if (g + t >= T.n || !(mask[j] >> (g + t < 7 ? g + t : 7) & 1u)) continue;
-                    const uint64_t k = claim_key(gen, g + t, bin[t][j]);
-                    val[t][j] = key[t][j] == k ? cm.vals[slot[t][j]] : claim_find(cm, k);
+                    for (int j = 0; j < PER; ++j)
+                        if (stamp[t][j] == claim_stamp(gen, (uint32_t)(w.s0 + j - b0))) is_new |= 1u << j;
                 }
             }
+            for (uint64_t round = 0; open && round <= cm.cap; ++round) {
+                uint64_t key[4][PER], val[4][PER];
 #pragma unroll
-            for (uint32_t t = 0; t < 4; ++t) {
+                for (uint32_t t = 0; t < 4; ++t) {
 #pragma unroll
-                for (int j = 0; j < PER; ++j) {
-                    if (g + t >= T.n || !(mask[j] >> (g + t < 7 ? g + t : 7) & 1u)) continue;
-                    if (val[t][j] == claim_stamp(gen, (uint32_t)(w.s0 + j - b0))) is_new |= 1u << j;
+                    for (int j = 0; j < PER; ++j) {
+                        if (!(open >> (t * PER + j) & 1u)) continue;
+                        key[t][j] = cm.keys[slot[t][j]];
+                        val[t][j] = cm.vals[slot[t][j]];
+                    }
+                }
+#pragma unroll
+                for (uint32_t t = 0; t < 4; ++t) {
+#pragma unroll
+                    for (int j = 0; j < PER; ++j) {
+                        if (!(open >> (t * PER + j) & 1u)) continue;
+                        const uint64_t k = claim_key(gen, g + t, bin[t][j]);
+                        if (key[t][j] == k) {
+                            if (val[t][j] == claim_stamp(gen, (uint32_t)(w.s0 + j - b0))) is_new |= 1u << j;
+                            open &= ~(1u << (t * PER + j));
+                        } else if ((key[t][j] >> 36) != (k >> 36)) {
+                            open &= ~(1u << (t * PER + j));    // not claimed
+                        } else {
+                            slot[t][j] = (slot[t][j] + 1) & (cm.cap - 1);
+                        }
+                    }
                 }
             }
         }
@@ -1337,51 +1390,57 @@ struct DegreeOp {
 // ------------------------------------------------------------ kernels
 
 // An op whose windows start from stitched segments (see SegScratchT).
-template <class Op>
+template <class Op, int BLK>
 struct Stitched : Op {
-    SegScratch* seg;
-    __device__ SegScratch* seg_scratch() { return seg; }
+    SegScratchT<BLK + kSegExtra>* seg;
+    __device__ SegScratchT<BLK + kSegExtra>* seg_scratch() { return seg; }
 };
 
-// Windows per thread of the kernels that take them together.
+// Windows per thread of the kernels that take them together, in workgroups of
+// BLK threads: kBlock, or one wave (kSmallBlock) where that spreads a batch
+// over more CUs.
 constexpr int kPerSmall = 4;
+constexpr int kSmallBlock = 64;
 
 template <int PER>
 __global__ __launch_bounds__(kBlock) void claim_kernel(Reads R, Tables T, ClaimMap cm, uint8_t* fresh,
                                                      uint64_t* counters) {
     __shared__ TileSharedT<kBlock * PER> sh;
-    if constexpr (PER == kPerSmall) {
-        __shared__ SegScratch seg;
-        Stitched<ClaimTogetherOp> op{{{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, counters + kErrors}}, &seg};
-        walk_tiles<PER>(R, sh, op);
-        add_counter(counters + kFresh, op.n_fresh);
-    } else {
-        ClaimOp op{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, counters + kErrors};
-        walk_tiles<PER>(R, sh, op);
-        add_counter(counters + kFresh, op.n_fresh);
-    }
+    ClaimOp op{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, counters + kErrors};
+    walk_tiles<PER>(R, sh, op);
+    add_counter(counters + kFresh, op.n_fresh);
+}
+
+template <int BLK>
+__global__ __launch_bounds__(BLK) void claim_together_kernel(Reads R, Tables T, ClaimMap cm, uint8_t* fresh,
+                                                           uint64_t* counters) {
+    __shared__ TileSharedT<BLK * kPerSmall> sh;
+    __shared__ SegScratchT<BLK + kSegExtra> seg;
+    Stitched<ClaimTogetherOp, BLK> op{{{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, counters + kErrors}}, &seg};
+    walk_tiles<kPerSmall, BLK>(R, sh, op);
+    add_counter(counters + kFresh, op.n_fresh);
 }
 
 template <int PER>
 __global__ __launch_bounds__(kBlock) void apply_kernel(Reads R, Tables T, ClaimMap cm, const uint8_t* fresh,
                                                      uint64_t* n_new, uint8_t* new_flags, uint64_t* counters) {
     __shared__ TileSharedT<kBlock * PER> sh;
-    uint64_t nn, occ;
-    if constexpr (PER == kPerSmall) {
-        __shared__ SegScratch seg;
-        Stitched<ApplyTogetherOp> op{
-            {{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, R.kmer_off, new_flags, ReadAcc{n_new}}}, &seg};
-        walk_tiles<PER>(R, sh, op);
-        nn = op.n_new;
-        occ = op.n_occ;
-    } else {
-        ApplyOp op{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, R.kmer_off, new_flags, ReadAcc{n_new}};
-        walk_tiles<PER>(R, sh, op);
-        nn = op.n_new;
-        occ = op.n_occ;
-    }
-    add_counter(counters + kNUnique, nn);
-    add_counter(counters + kNOccupied, occ);
+    ApplyOp op{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, R.kmer_off, new_flags, ReadAcc{n_new}};
+    walk_tiles<PER>(R, sh, op);
+    add_counter(counters + kNUnique, op.n_new);
+    add_counter(counters + kNOccupied, op.n_occ);
+}
+
+template <int BLK>
+__global__ __launch_bounds__(BLK) void apply_together_kernel(Reads R, Tables T, ClaimMap cm, const uint8_t* fresh,
+                                                           uint64_t* n_new, uint8_t* new_flags, uint64_t* counters) {
+    __shared__ TileSharedT<BLK * kPerSmall> sh;
+    __shared__ SegScratchT<BLK + kSegExtra> seg;
+    Stitched<ApplyTogetherOp, BLK> op{
+        {{T, cm, claim_gen(cm), fresh, R.b0, R.canonical, R.kmer_off, new_flags, ReadAcc{n_new}}}, &seg};
+    walk_tiles<kPerSmall, BLK>(R, sh, op);
+    add_counter(counters + kNUnique, op.n_new);
+    add_counter(counters + kNOccupied, op.n_occ);
 }
 
 template <int PER>
@@ -1398,14 +1457,15 @@ __global__ __launch_bounds__(kBlock) void exact_lookup_kernel(Reads R, ExactSet 
 // window's slot).  Looking every window up, then inserting and stamping the
 // absent ones, then looking them up again took 40.2 ms for the 264M bases of
 // 220k uneven reads at 5% substitutions; this takes 20 ms.
-__global__ __launch_bounds__(kBlock) void exact_add_kernel(Reads R, ExactSet E, uint64_t* n_new, uint64_t* counters) {
-    __shared__ TileSharedT<kBlock * kPerSmall> sh;
-    __shared__ SegScratch seg;
+template <int BLK>
+__global__ __launch_bounds__(BLK) void exact_add_kernel(Reads R, ExactSet E, uint64_t* n_new, uint64_t* counters) {
+    __shared__ TileSharedT<BLK * kPerSmall> sh;
+    __shared__ SegScratchT<BLK + kSegExtra> seg;
     uint64_t n_reads;
     int64_t n_bases;
     batch_sizes(R, n_reads, n_bases);      // the reads that are there, not a captured batch's bound
-    Stitched<ExactAddOp> op{{E, R.b0, current_gen(counters), R.off, n_reads, counters + kErrors, n_new}, &seg};
-    walk_tiles<kPerSmall>(R, sh, op);
+    Stitched<ExactAddOp, BLK> op{{E, R.b0, current_gen(counters), R.off, n_reads, counters + kErrors, n_new}, &seg};
+    walk_tiles<kPerSmall, BLK>(R, sh, op);
     add_counter(counters + kNUnique, op.n_new);
     max_counter(counters + kLastIns, op.last_ins);
 }
@@ -1422,15 +1482,18 @@ template <int PER>
 __global__ __launch_bounds__(kBlock) void query_kernel(Reads R, Tables T, ExactSet E, int16_t* counts,
                                                      uint64_t* hashes) {
     __shared__ TileSharedT<kBlock * PER> sh;
-    if constexpr (PER == kPerSmall) {
-        __shared__ SegScratch seg;
-        Stitched<QueryTogetherOp> op{{T, E, R.kmer_off, counts, hashes}, &seg};
-        walk_tiles<PER>(R, sh, op);
-    } else {
-        __shared__ QueryStage<kBlock * PER> st;
-        QueryOp<kBlock * PER> op{T, E, R, kBlock * PER, counts, hashes, &st};
-        walk_tiles<PER>(R, sh, op);
-    }
+    __shared__ QueryStage<kBlock * PER> st;
+    QueryOp<kBlock * PER> op{T, E, R, kBlock * PER, counts, hashes, &st};
+    walk_tiles<PER>(R, sh, op);
+}
+
+template <int BLK>
+__global__ __launch_bounds__(BLK) void query_together_kernel(Reads R, Tables T, ExactSet E, int16_t* counts,
+                                                           uint64_t* hashes) {
+    __shared__ TileSharedT<BLK * kPerSmall> sh;
+    __shared__ SegScratchT<BLK + kSegExtra> seg;
+    Stitched<QueryTogetherOp, BLK> op{{T, E, R.kmer_off, counts, hashes}, &seg};
+    walk_tiles<kPerSmall, BLK>(R, sh, op);
 }
 
 template <int PER>
@@ -1464,7 +1527,10 @@ __global__ __launch_bounds__(kBlock) void hash_claim_kernel(const uint64_t* h, u
             const bool empty = T.kind == kBit ? !bit_get(T.base[t], b) : T.base[t][b] == 0;
             if (empty) {
                 mask |= (uint8_t)(1u << (t < 7 ? t : 7));
-                claim_insert(cm, claim_key(gen, t, b), claim_stamp(gen, (uint32_t)i), counters + kErrors);
+                if (cm.direct)
+                    claim_direct(cm, t, b, claim_stamp(gen, (uint32_t)i));
+                else
+                    claim_insert(cm, claim_key(gen, t, b), claim_stamp(gen, (uint32_t)i), counters + kErrors);
             }
         }
         fresh[i] = mask;
@@ -1491,7 +1557,8 @@ __global__ __launch_bounds__(kBlock) void hash_apply_kernel(const uint64_t* h, u
             } else {
                 if (byte_sat_inc(T.base[t], b) == 0 && t == 0) occ++;
             }
-            if (!nw && (mask & (1u << (t < 7 ? t : 7)))) nw = claim_find(cm, claim_key(gen, t, b)) == stamp;
+            if (!nw && (mask & (1u << (t < 7 ? t : 7))))
+                nw = (cm.direct ? cm.vals[cm.dbase[t] + b] : claim_find(cm, claim_key(gen, t, b))) == stamp;
         }
         nn += nw;
         if (is_new) is_new[i] = nw;
@@ -3207,8 +3274,8 @@ __global__ __launch_bounds__(kBlock) void scan_u32_apply_kernel(uint32_t* a, uin
 
 namespace gt {
 
-static int tile_grid(const Launch& L, const Reads& R) {
-    const int64_t tile = (int64_t)kBlock * L.per;
+static int tile_grid(const Launch& L, const Reads& R, int blk = kBlock) {
+    const int64_t tile = (int64_t)blk * L.per;
     const int64_t tiles = (R.b1 + tile - 1) / tile - R.b0 / tile;
     const int64_t g = tiles < L.grid ? tiles : L.grid;
     return g > 0 ? (int)g : 1;
@@ -3253,14 +3320,21 @@ void launch_fill_u64(uint64_t* p, uint64_t n, uint64_t v, hipStream_t s) {
     fill_u64_kernel<<<(unsigned)(g < 16384 ? g : 16384), 256, 0, s>>>(p, n, v);
 }
 
-// The same with four windows of a thread taken together for launches that ask
-// for it (make_launch).
-#define GT_TILE_LAUNCH_SMALL(L, kernel, ...)                                                  \
-    do {                                                                                      \
-        if ((L).per == kPerSmall)                                                             \
-            kernel<kPerSmall><<<tile_grid(L, R), kBlock, 0, (L).stream>>>(__VA_ARGS__);       \
-        else                                                                                  \
-            GT_TILE_LAUNCH(L, kernel, __VA_ARGS__);                                           \
+// Launches kernel<BLK> of four windows of a thread together for launches that
+// ask for it (make_launch), one wave per workgroup where workgroups of kBlock
+// threads would reach fewer than half of the CUs.  (Past that a workgroup's
+// own work, its tables, halo and counter atomics, costs more than it gives:
+// 500k windows into an exact set took 72 us in 611 workgroups of 256 threads
+// and 126 us in 2441 of 64.)
+static bool small_blocks(const Launch& L, const Reads& R) {
+    return (R.b1 - R.b0) / (kBlock * kPerSmall) < L.grid / 16;
+}
+#define GT_TOGETHER_LAUNCH(L, kernel, ...)                                                          \
+    do {                                                                                            \
+        if (small_blocks(L, R))                                                                     \
+            kernel<kSmallBlock><<<tile_grid(L, R, kSmallBlock), kSmallBlock, 0, (L).stream>>>(__VA_ARGS__); \
+        else                                                                                        \
+            kernel<kBlock><<<tile_grid(L, R), kBlock, 0, (L).stream>>>(__VA_ARGS__);                \
     } while (0)
 
 bool layout_is_small(uint64_t n_reads, int64_t n_bases) {
@@ -3277,12 +3351,18 @@ void launch_layout_small(const int64_t* off, uint64_t n_reads, int64_t n_bases, 
 
 void launch_claim(const Launch& L, const Reads& R, const Tables& T, const ClaimMap& cm, uint8_t* fresh,
                   uint64_t* counters) {
-    GT_TILE_LAUNCH_SMALL(L, claim_kernel, R, T, cm, fresh, counters);
+    if (L.per == kPerSmall)
+        GT_TOGETHER_LAUNCH(L, claim_together_kernel, R, T, cm, fresh, counters);
+    else
+        GT_TILE_LAUNCH(L, claim_kernel, R, T, cm, fresh, counters);
 }
 
 void launch_apply(const Launch& L, const Reads& R, const Tables& T, const ClaimMap& cm, const uint8_t* fresh,
                   uint64_t* n_new, uint8_t* new_flags, uint64_t* counters) {
-    GT_TILE_LAUNCH_SMALL(L, apply_kernel, R, T, cm, fresh, n_new, new_flags, counters);
+    if (L.per == kPerSmall)
+        GT_TOGETHER_LAUNCH(L, apply_together_kernel, R, T, cm, fresh, n_new, new_flags, counters);
+    else
+        GT_TILE_LAUNCH(L, apply_kernel, R, T, cm, fresh, n_new, new_flags, counters);
 }
 
 void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* fresh, uint64_t* counters) {
@@ -3292,7 +3372,7 @@ void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uin
 void launch_exact_add(const Launch& L, const Reads& R, const ExactSet& E, uint64_t* n_new, uint64_t* counters) {
     Launch small = L;
     small.per = kPerSmall;
-    exact_add_kernel<<<tile_grid(small, R), kBlock, 0, L.stream>>>(R, E, n_new, counters);
+    GT_TOGETHER_LAUNCH(small, exact_add_kernel, R, E, n_new, counters);
 }
 
 void launch_exact_flags(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* new_flags,
@@ -3314,7 +3394,10 @@ void launch_exact_tail(uint64_t* counters, hipStream_t s) {
 
 void launch_query(const Launch& L, const Reads& R, const Tables& T, const ExactSet& E, int16_t* counts,
                   uint64_t* hashes) {
-    GT_TILE_LAUNCH_SMALL(L, query_kernel, R, T, E, counts, hashes);
+    if (L.per == kPerSmall)
+        GT_TOGETHER_LAUNCH(L, query_together_kernel, R, T, E, counts, hashes);
+    else
+        GT_TILE_LAUNCH(L, query_kernel, R, T, E, counts, hashes);
 }
 
 void launch_hash(const Launch& L, const Reads& R, uint64_t* fw, uint64_t* rc, uint8_t* valid) {
