@@ -220,7 +220,8 @@ struct Scratch {
     // binned insert: events of the two partition passes, first-pass digit
     // offsets, second-pass counts / starts and their scan sums, new-window
     // flags and the sub-batch's first packed window index
-    DevBuf bin_ent1, bin_ent2, bin_dig2, bin_off1, bin_cnt2, bin_sums, bin_flags, bin_kbase, bin_vq;
+    DevBuf bin_ent1, bin_ent2, bin_dig2, bin_off1, bin_cnt2, bin_sums, bin_flags, bin_kbase;
+    DevBuf bin_res1, bin_win1, bin_tile;   // results per event: result byte, window; per tile and item (res_prepare)
     bool fixed = false;                // buffers preallocated and never moved (captured graphs)
 };
 
@@ -730,9 +731,10 @@ bool use_binned(const gt_storage* st, const Scratch& sc, const Reads& R) {
 }
 
 // Binned sub-batch in start positions, a multiple of kTileMax: 2^27 for an
-// insert, 2^26 for insert_and_query (its four result bytes per window are
-// written scattered, and 2^26 windows keep them in a 256 MiB range), or
-// GOETIA_AMD_BIN_SUB (at most 2^29); capped by GOETIA_AMD_SUB_BATCH.
+// insert, 2^26 for insert_and_query (a first digit's result bytes are then
+// 1 MB, a quarter of an XCD's L2: 22.0 ms for the replays of 4M reads against
+// 24.1 at 2^27 and 27 at 2^25), or GOETIA_AMD_BIN_SUB (at most 2^29); capped
+// by GOETIA_AMD_SUB_BATCH.
 uint64_t bin_sub_batch(uint64_t n_bases, bool iq) {
     uint64_t sb = iq ? 1ULL << 26 : 1ULL << 27;
     if (const char* v = std::getenv("GOETIA_AMD_BIN_SUB")) {
@@ -783,6 +785,28 @@ int bin_prepare(gt_storage* st, Scratch& sc, uint64_t tiles_max, BinPlan& P) {
     return GT_OK;
 }
 
+// Adds the per-event results (BinPlan::res1 and what goes with it) to a plan
+// for sub-batches of up to tiles_max first-pass tiles.
+int res_prepare(const gt_storage* st, Scratch& sc, uint64_t tiles_max, BinPlan& P) {
+    const uint64_t n_ent = tiles_max * st->n_tables * kBinTile;
+    const uint64_t groups_max = (tiles_max + kBinGroup - 1) / kBinGroup;
+    const uint64_t k0_bytes = (tiles_max + 1) * sizeof(uint64_t);
+    const uint64_t run_bytes = tiles_max * kDigits1 * sizeof(uint32_t);
+    const uint64_t item_bytes = kDigits1 * groups_max * sizeof(uint32_t);
+    const uint64_t off_bytes = tiles_max * kDigits1 * sizeof(uint16_t);
+    GT_TRY(sc.bin_res1.ensure(n_ent + 16));                       // the combine reads past a run's end
+    GT_TRY(sc.bin_win1.ensure(n_ent * sizeof(uint16_t) + 16));
+    GT_TRY(sc.bin_tile.ensure(k0_bytes + run_bytes + item_bytes + off_bytes));
+    P.res1 = sc.bin_res1.as<uint8_t>();
+    P.win1 = sc.bin_win1.as<uint16_t>();
+    uint8_t* t = sc.bin_tile.as<uint8_t>();
+    P.tile_k0 = reinterpret_cast<uint64_t*>(t);
+    P.run1 = reinterpret_cast<uint32_t*>(t + k0_bytes);
+    P.item_n = reinterpret_cast<uint32_t*>(t + k0_bytes + run_bytes);
+    P.off1t = reinterpret_cast<uint16_t*>(t + k0_bytes + run_bytes + item_bytes);
+    return GT_OK;
+}
+
 // Routes the (window, table) events of the windows starting in [b0, b1) of
 // prepared reads (at most the prepared tiles_max tiles): by bucket, in
 // window order within a bucket (first pass, second-pass count and scan,
@@ -797,7 +821,7 @@ void bin_route(const Reads& R, const Tables& T, BinPlan& P, Scratch& sc, int64_t
     const uint64_t cnt_len = ((uint64_t)P.n_d1 << P.shift2) * P.n_groups;
     const int grid_l1 = std::max(1, g_dev.cus * 2);     // 70 KB of LDS per workgroup
     const int grid = std::max(1, g_dev.cus * 8);
-    launch_bin_kbase(R, b0, sc.bin_kbase.as<uint64_t>(), s);
+    launch_bin_kbase(R, b0, sc.bin_kbase.as<uint64_t>(), b1, P.tile_k0 ? P.tile_k0 + P.tiles1 : nullptr, s);
     {
         ProfScope ps("bin_hash", s);
         launch_bin_l1(Rs, T, P, grid_l1, s);
@@ -821,15 +845,13 @@ void bin_route(const Reads& R, const Tables& T, BinPlan& P, Scratch& sc, int64_t
 // (count-min only), the insert_and_query count of every window.
 int binned_insert_impl(gt_storage* st, Scratch& sc, const Reads& R, uint64_t* n_new, uint8_t* new_flags,
                        int16_t* iq_counts, hipStream_t s) {
-    const uint32_t nt = st->n_tables;
     const bool iq = iq_counts != nullptr;
     const uint64_t sub = bin_sub_batch((uint64_t)R.n_bases, iq);
     BinPlan P;
     GT_TRY(bin_prepare(st, sc, sub / kBinTile, P));
     uint8_t* flags = new_flags;
     if (iq) {
-        GT_TRY(sc.bin_vq.ensure((size_t)R.n_bases * kBinMaxTables));
-        launch_zero_words(sc.bin_vq.as<uint32_t>(), R.kmer_off + R.n_reads, (uint64_t)R.n_bases, s);
+        GT_TRY(res_prepare(st, sc, sub / kBinTile, P));
         flags = nullptr;
     } else {
         if (!flags) {
@@ -839,7 +861,6 @@ int binned_insert_impl(gt_storage* st, Scratch& sc, const Reads& R, uint64_t* n_
         launch_zero_bytes(flags, R.kmer_off + R.n_reads, (uint64_t)R.n_bases, s);
     }
     P.flags = flags;
-    P.vq = iq ? sc.bin_vq.as<uint8_t>() : nullptr;
     P.unordered = iq ? 0u : 1u;        // a plain insert's replay does not depend on event order
 
     const Tables T = st->tables_view();
@@ -852,15 +873,15 @@ int binned_insert_impl(gt_storage* st, Scratch& sc, const Reads& R, uint64_t* n_
             // per CU, by LDS), each walking its buckets with the next one prefetched
             // (35.9 ms per full step against 36.6 with eight launched per CU)
             ProfScope ps("bin_apply", s);
-            launch_bin_apply(P, T, ctr, P.unordered && !P.vq ? std::max(1, g_dev.cus * 2) : grid, s);
+            launch_bin_apply(P, T, ctr, std::max(1, g_dev.cus * (P.unordered ? 2 : 4)), s);
+        }
+        if (iq) {
+            ProfScope ps("bin_iq", s);
+            launch_bin_iq_combine(P, iq_counts, ctr, grid, s);
         }
         GT_HIP(hipGetLastError());
     }
-    if (iq) {
-        ProfScope ps("bin_iq", s);
-        launch_bin_iq_combine(sc.bin_vq.as<uint32_t>(), R.kmer_off + R.n_reads, (uint64_t)R.n_bases, nt, iq_counts,
-                              ctr, s);
-    } else {
+    if (!iq) {
         ProfScope ps("bin_new", s);
         launch_bin_read_new(R.kmer_off, R.n_reads, flags, n_new, ctr, s);
     }
@@ -965,7 +986,8 @@ int dbg_insert_impl(gt_storage* st, Scratch& sc, Reads R, uint64_t* n_new, uint8
         sc.bin_ent2.release();
         sc.bin_dig2.release();
         sc.bin_flags.release();
-        sc.bin_vq.release();
+        sc.bin_res1.release();
+        sc.bin_win1.release();
         GT_TRY(prepare_claims(st, sc, (uint64_t)R.n_bases, &sub, s));
     }
     const Launch L = make_launch(st, std::min<uint64_t>(sub, (uint64_t)R.n_bases), s);
@@ -1716,7 +1738,8 @@ int gt_dbg_insert_and_query_dev(gt_storage* st, uint16_t K, int canonical, int m
         st->own.bin_ent1.release();     // no room for the event buffers: strict order below
         st->own.bin_ent2.release();
         st->own.bin_dig2.release();
-        st->own.bin_vq.release();
+        st->own.bin_res1.release();
+        st->own.bin_win1.release();
     }
     if (st->kind == kByte) {
         // More than four tables or 2^30 bins: hash the batch, then apply it
@@ -1884,8 +1907,8 @@ int gt_diginorm_dev(gt_storage* st, uint16_t K, int canonical, int mode, const u
     uint32_t* ctl = st->dn_ctl.as<uint32_t>();
     uint8_t* flags = sc.bin_flags.as<uint8_t>();
     P.flags = flags;
-    P.vq = nullptr;
     P.rid = rid;
+    P.wread = wread;
     P.keep = state;
     const Tables T = st->tables_view();
     uint64_t* ctr = st->counters.as<uint64_t>();
@@ -1903,7 +1926,6 @@ int gt_diginorm_dev(gt_storage* st, uint16_t K, int canonical, int mode, const u
             P.hasev = hasev;
             bin_route(R, T, P, sc, off[r0], off[r1], s);
             P.hasev = nullptr;
-            launch_dn_event_reads(P, wread, rid, n_win * st->n_tables, s);
             bool settled = false;
             uint32_t h_ctl[2] = {0, 0};
             for (int g = 1; g <= cap && !settled; ++g) {

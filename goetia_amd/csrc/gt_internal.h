@@ -124,11 +124,24 @@ struct BinPlan {
     uint32_t* cnt2;                       // (n_d1 << shift2) x n_groups (+1): counts, then exclusive starts
     const uint64_t* kbase;                // packed index of the sub-batch's first window
     uint8_t* flags;                       // per packed window: 1 = new k-mer
-    uint8_t* vq;                          // insert_and_query: per packed window, kBinMaxTables
-                                          // counts just after the event (flags unused then)
+    // Results per event (insert_and_query; flags unused then): res1 has a byte
+    // per event, by first digit and within it in event order, and an ent2
+    // event's low word is its index there.  item_n: events of each
+    // second-pass item; per tile, run1 the res1 index and off1t the ent1
+    // position of each first digit's run; win1: the window within its tile of
+    // every ent1 event; tile_k0 (one more entry at the end): the packed index
+    // of the tile's first window
+    uint8_t* res1;
+    uint32_t* item_n;
+    uint32_t* run1;
+    uint16_t* off1t;
+    uint16_t* win1;
+    uint64_t* tile_k0;
     // masked replay (batched diginorm): only events of reads r < r_end with
     // keep[r] & 1 are applied; rid[i] is the read of ent2 event i
-    const uint32_t* rid;
+    uint32_t* rid;
+    const uint32_t* wread;                // read of every window of the sub-batch: the ordered scatter
+                                          // then writes rid
     const uint8_t* keep;
     uint32_t r_end;
     uint8_t* hasev;                       // optional, per window of the sub-batch: the first pass

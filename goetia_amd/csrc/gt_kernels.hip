@@ -1900,6 +1900,10 @@ __global__ void exact_keys_kernel(ExactSet E, uint64_t* out, uint64_t cap_out, u
 // per bin, then settles each bin from its smallest-ordinal event.
 // insert_and_query and diginorm keep the ordered kernels.
 
+// XCDs of the device, each with an L2 of its own; consecutive workgroups go to
+// consecutive XCDs.
+constexpr uint32_t kXcds = 8;
+
 // Mask of the lanes whose v equals this lane's (all 64 lanes must be active).
 template <int BITS>
 __device__ __forceinline__ uint64_t match_mask(uint32_t v) {
@@ -1931,10 +1935,16 @@ __device__ __forceinline__ uint64_t match_lds(uint64_t* slots, uint32_t key, boo
     return m;
 }
 
-// Packed index of the first window starting at or after b0 (one lane).
+// Packed index of the first window starting at or after b0, and at or after
+// b1 when out1 is given (one lane each).
 __global__ void bin_kbase_kernel(const int64_t* off, const int64_t* kmer_off, uint64_t n_reads, int K, int64_t b0,
-                                 uint64_t* out) {
-    if (blockIdx.x || threadIdx.x) return;
+                                 uint64_t* out, int64_t b1, uint64_t* out1) {
+    if (blockIdx.x || threadIdx.x > 1) return;
+    if (threadIdx.x) {
+        b0 = b1;
+        out = out1;
+    }
+    if (!out) return;
     uint64_t lo = 0, hi = n_reads - 1;
     while (lo < hi) {
         const uint64_t mid = (lo + hi + 1) >> 1;
@@ -1989,6 +1999,7 @@ struct BinL1Shared {
     uint32_t cnt[kU ? kDigits1 : 1];                 // order-free: events per digit, then starts
     uint32_t wpos[kU ? 1 : kRankWaves][kDigits1 + 1];  // stable: per ranking wave, digit counts then positions
     uint32_t part[BLK / 64];
+    uint32_t ord0;                                   // insert_and_query: ordinal of the tile's first window
 };
 static_assert(sizeof(int64_t) * (kReadCache + 1) >= sizeof(uint64_t) * kRankWaves * kDigits1,
               "the stable sort borrows the walker's read-offset cache for its match slots");
@@ -2016,6 +2027,9 @@ struct BinL1Op {
     uint64_t* slots;          // kRankWaves x kDigits1 match slots (the walker's read-offset cache, idle here)
     int64_t b_lo;             // first start of the sub-batch (tiles may begin before it)
     int64_t t0 = 0;
+    const TileSharedT<kBinTile>* tile_sh;   // the walker's tile (its first read), and that read's layout
+    const int64_t* off;
+    int K;
     uint32_t kr = 0xFFFFFFFFu;  // read whose packed-index offset is cached in kd
     int64_t kd = 0;             // kmer_off[kr] - start of read kr - kbase
 
@@ -2025,6 +2039,17 @@ struct BinL1Op {
         for (uint32_t t = 0; t < P.n_tables; ++t)
             for (int j = 0; j < PER; ++j) sh->g[t * kBinTile + w0 + j] = kNoBin;
         if (kU && threadIdx.x < kDigits1) sh->cnt[threadIdx.x] = 0;      // digit counters
+        if (P.win1 && threadIdx.x == 0) {
+            // packed index of the first window at or after the tile's start (read
+            // after the barrier of the stitched starts)
+            const uint32_t r = tile_sh->r_lo;
+            const int64_t a = off[r], wins = off[r + 1] - a - K + 1;
+            int64_t d = tile_base - a;
+            d = d < 0 || wins <= 0 ? 0 : (d > wins ? wins : d);
+            const int64_t k0 = kmer_off[r] + d;
+            sh->ord0 = (uint32_t)(k0 - (int64_t)kbase);
+            P.tile_k0[tile_base / kBinTile - P.tile0] = (uint64_t)k0;
+        }
     }
 
     __device__ void operator()(int64_t s, uint32_t r, int64_t rstart, uint64_t fw, uint64_t rc, bool valid) {
@@ -2105,8 +2130,10 @@ struct BinL1Op {
                 const uint32_t i = i0 + q * BLK + threadIdx.x;
                 if (i < n_ev) {
                     const uint32_t g = sh->g[e[q]];
-                    dst[i] = ((uint64_t)g << 32) | sh->ord[e[q] & (kBinTile - 1)];
+                    const uint32_t ord = sh->ord[e[q] & (kBinTile - 1)];
+                    dst[i] = ((uint64_t)g << 32) | ord;
                     dst2[i] = (uint16_t)((g >> kBinBits) & mask2);
+                    if (P.win1) P.win1[r0 + i] = (uint16_t)((ord - sh->ord0) & (kBinTile - 1));
                 }
             }
         }
@@ -2154,6 +2181,7 @@ struct BinL1Op {
         const uint32_t start = block_exclusive_u32<BLK>(tot, sh->part, &n_ev);
         if (d < kDigits1) {
             P.off1[(size_t)d * P.tiles1 + lt1] = (uint16_t)start;
+            if (P.off1t) P.off1t[(size_t)lt1 * kDigits1 + d] = (uint16_t)start;
             uint32_t p = start;
             for (int w = 0; w < kRankWaves; ++w) {
                 const uint32_t c = sh->wpos[w][d];
@@ -2190,7 +2218,8 @@ __global__ __launch_bounds__(kBinL1Block) void bin_l1_kernel(Reads R, Tables T, 
     constexpr int PER = kBinTile / BLK;
     __shared__ TileSharedT<kBinTile> sh;
     __shared__ BinL1Shared<BLK, kU> bs;
-    BinL1Op<kU, BLK, PER> op{T, P, R.kmer_off, R.canonical, *P.kbase, &bs, reinterpret_cast<uint64_t*>(sh.roff), R.b0};
+    BinL1Op<kU, BLK, PER> op{T, P, R.kmer_off, R.canonical, *P.kbase, &bs, reinterpret_cast<uint64_t*>(sh.roff), R.b0,
+                           0, &sh, R.off, R.K};
     walk_tiles<PER, BLK>(R, sh, op);
 }
 
@@ -2324,6 +2353,7 @@ __global__ __launch_bounds__(kCountBlock) void bin_l2_count_kernel(BinPlan P) {
         for (uint32_t gi = 0; gi < ng; ++gi) {
             uint32_t* h = hist[gi];
             const uint32_t n = bin_load_runs<BLK>(P, d1, grp0 + gi, sh);
+            if (P.item_n && threadIdx.x == 0) P.item_n[d1 * P.n_groups + grp0 + gi] = n;
             auto chunk_len = [&](uint32_t c) {
                 return c < n ? (n - c < (uint32_t)kBinChunk ? n - c : (uint32_t)kBinChunk) : 0u;
             };
@@ -2383,6 +2413,17 @@ __global__ __launch_bounds__(kBlock) void bin_l2_scatter_kernel(BinPlan P) {
         for (uint32_t d2 = threadIdx.x; d2 < (uint32_t)kDigits2; d2 += kBlock)
             sh.cur[d2] = d2 <= mask2 ? P.cnt2[(size_t)((d1 << P.shift2) | d2) * P.n_groups + grp] : 0u;
         const uint32_t n = bin_load_runs(P, d1, grp, sh.runs);
+        uint32_t item0 = 0;                                // res1 index of the item's first event
+        if (P.res1) {
+            // the events of earlier first digits, then of this digit's earlier items
+            uint32_t before = 0;
+            for (uint32_t q = threadIdx.x; q < grp; q += kBlock) before += P.item_n[d1 * P.n_groups + q];
+            uint32_t all;
+            block_exclusive_u32(before, sh.runs.part, &all);
+            item0 = P.cnt2[(size_t)(d1 << P.shift2) * P.n_groups] + all;
+            for (uint32_t j = threadIdx.x; j < kBinGroup && grp * kBinGroup + j < P.tiles1; j += kBlock)
+                P.run1[(size_t)(grp * kBinGroup + j) * kDigits1 + d1] = item0 + sh.runs.rpre[j];
+        }
         // chunk c's events are loaded while chunk c - 1 is sorted
         uint64_t v[kBinChunk / kBlock];
         {
@@ -2443,10 +2484,29 @@ __global__ __launch_bounds__(kBlock) void bin_l2_scatter_kernel(BinPlan P) {
                 __builtin_amdgcn_wave_barrier();
             }
             __syncthreads();
-            for (uint32_t i = threadIdx.x; i < m; i += kBlock) {
-                const uint64_t e = sh.ev[sh.perm[i]];
-                const uint32_t d = bin_d2(e, mask2);
-                P.ent2[sh.cur[d] + (i - sh.lstart[d])] = e;
+            for (uint32_t i0 = 0; i0 < m; i0 += 4 * kBlock) {
+                uint64_t e[4];
+                uint32_t at[4], rd[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t i = i0 + q * kBlock + threadIdx.x;
+                    if (i >= m) continue;
+                    const uint32_t j = sh.perm[i];
+                    e[q] = sh.ev[j];
+                    const uint32_t d = bin_d2(e[q], mask2);
+                    at[q] = sh.cur[d] + (i - sh.lstart[d]);
+                    // the events of a chunk come from a few hundred tiles, whose
+                    // windows' reads are near one another (gathered from bucket
+                    // order they were random lines: 2.0 ms per 2^25 starts)
+                    if (P.wread) rd[q] = P.wread[(uint32_t)e[q]];
+                    if (P.res1) e[q] = (e[q] & ~0xFFFFFFFFULL) | (item0 + c0 + j);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (i0 + q * kBlock + threadIdx.x >= m) continue;
+                    P.ent2[at[q]] = e[q];
+                    if (P.wread) P.rid[at[q]] = rd[q];
+                }
             }
             __syncthreads();
             for (uint32_t dd = threadIdx.x; dd < (uint32_t)kDigits2; dd += kBlock)
@@ -2551,6 +2611,25 @@ __device__ __forceinline__ uint64_t bin_match(uint64_t* slots, uint32_t key, boo
     return m;
 }
 
+// Whether two active lanes of the wavefront are on one bin of a slice of byte
+// counts; *pre gets each active lane's count.  Every active lane writes its
+// number over its count and reads it back, so the caller has to write each
+// active bin again.  64 random events of kBucketBins bins share none 78 times
+// of 100, and then need no ranking: three LDS accesses in a row in place of
+// bin_match's three and its ballots.
+__device__ __forceinline__ bool bins_shared(uint8_t* sb, uint32_t key, bool active, uint32_t* pre) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t p = 0, back = lane;
+    if (active) p = sb[key];
+    __builtin_amdgcn_wave_barrier();
+    if (active) sb[key] = (uint8_t)lane;
+    __builtin_amdgcn_wave_barrier();
+    if (active) back = sb[key];
+    __builtin_amdgcn_wave_barrier();
+    *pre = p;
+    return __ballot(back != lane) != 0;
+}
+
 // Stages the bins of bucket b of byte tables in LDS (sw: kBucketBins / 4
 // words); returns the table of the bucket and the staged words' source.
 __device__ __forceinline__ uint32_t* bin_stage_slice(const BinPlan& P, const Tables& T, uint32_t b, uint32_t* sw,
@@ -2592,17 +2671,31 @@ __device__ __forceinline__ uint32_t* bin_stage_slice(const BinPlan& P, const Tab
 
 // Replay: one wavefront per bucket (four per workgroup).  Masked: only the
 // events of kept reads before P.r_end take part (batched diginorm).
+//
+// insert_and_query's result bytes go to res1, where a first digit's events
+// are one dense range (2 MB per 2^27 starts), and the workgroups of one XCD
+// (every eighth) take the buckets of one digit at a time: the range stays in
+// that XCD's L2 and its bytes leave it as whole lines.  Stores of random
+// bytes run at 232 G/s into 2 MB per XCD and at about 90 past the L2, so what
+// has no second use there (events, table slices) goes past it.  Writing each
+// byte to its window's place took 3.56 ms per 2^26 starts, of which 1.5 is the
+// replay without results; to its place in the tile's region (32 bytes per tile
+// and digit) 4.6, since the lines of a digit then span 8 MB; this takes 2.44.
 template <bool kMasked>
 __device__ __forceinline__ void bin_apply_body(const BinPlan& P, const Tables& T, uint64_t* counters,
                                                uint32_t (*slice)[kBucketBins / 4], uint64_t (*slots)[256]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint64_t lt = lanes_below();
     const uint64_t kb = *P.kbase;
-    const bool bytes = T.kind == kByte;
     uint32_t* sw = slice[wave];
     uint8_t* sb = reinterpret_cast<uint8_t*>(sw);
     uint64_t occ = 0;
-    for (uint32_t b = blockIdx.x * 4u + (uint32_t)wave; b < P.n_buckets; b += gridDim.x * 4u) {
+    // this XCD's buckets are those of every eighth first digit, digit by digit
+    const uint32_t xcd = blockIdx.x % kXcds, n_d1 = P.n_d1 > xcd ? (P.n_d1 - xcd + kXcds - 1) / kXcds : 0u;
+    const uint32_t first = blockIdx.x / kXcds * 4u + (uint32_t)wave, step = gridDim.x / kXcds * 4u;
+    for (uint32_t x = first; x < n_d1 << P.shift2; x += step) {
+        const uint32_t b = ((xcd + kXcds * (x >> P.shift2)) << P.shift2) | (x & ((1u << P.shift2) - 1u));
+        if (b >= P.n_buckets) continue;
         const uint32_t lo_e = P.cnt2[(size_t)b * P.n_groups];
         const uint32_t hi_e = P.cnt2[(size_t)(b + 1) * P.n_groups];
         if (lo_e == hi_e) continue;
@@ -2620,14 +2713,14 @@ __device__ __forceinline__ void bin_apply_body(const BinPlan& P, const Tables& T
         const uint64_t bin0 = (uint64_t)(b - P.bfirst[t]) << kBinBits;
         const uint64_t left = pt - bin0;
         const uint32_t nb = (uint32_t)(left < (uint64_t)kBucketBins ? left : (uint64_t)kBucketBins);
-        const uint32_t nw = bytes ? (nb + 3u) / 4u : (nb + 31u) / 32u;
-        uint32_t* src = reinterpret_cast<uint32_t*>(bytes ? base + bin0 : base + bin0 / 8);
+        const uint32_t nw = (nb + 3u) / 4u;
+        uint32_t* src = reinterpret_cast<uint32_t*>(base + bin0);
         for (uint32_t w0 = 0; w0 < nw; w0 += 8 * 64) {
             uint32_t x[8];
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
                 const uint32_t w = w0 + (uint32_t)q * 64 + (uint32_t)lane;
-                x[q] = w < nw ? src[w] : 0u;
+                x[q] = w < nw ? __builtin_nontemporal_load(src + w) : 0u;
             }
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
@@ -2636,60 +2729,65 @@ __device__ __forceinline__ void bin_apply_body(const BinPlan& P, const Tables& T
             }
         }
         __builtin_amdgcn_wave_barrier();
-        // events are loaded four chunks ahead
-        constexpr int kAhead = 4;
+        // Events are loaded kAhead steps ahead (with their reads, whose states
+        // follow kAhead / 2 steps later).  Loads and stores of a wave complete in
+        // order, so a step waits for the result stores of the step that issued
+        // its loads too: it is the depth of this pipeline that hides them.
+        constexpr int kAhead = 8;
         uint64_t pf[kAhead];
+        uint32_t pr[kMasked ? kAhead : 1];
+        uint8_t pk[kMasked ? kAhead : 1];
+        auto load = [&](uint32_t at, int q) {
+            const uint32_t i = at + (uint32_t)lane;
+            pf[q] = i < hi_e ? __builtin_nontemporal_load(P.ent2 + i) : 0;
+            if (kMasked) pr[kMasked ? q : 0] = i < hi_e ? P.rid[i] : 0xFFFFFFFFu;
+        };
+        auto load_state = [&](int q) {
+            if (kMasked) pk[q] = pr[q] < P.r_end ? P.keep[pr[q]] : (uint8_t)0;
+        };
 #pragma unroll
-        for (int q = 0; q < kAhead; ++q) {
-            const uint32_t i = lo_e + (uint32_t)q * 64 + (uint32_t)lane;
-            pf[q] = i < hi_e ? P.ent2[i] : 0;
+        for (int q = 0; q < kAhead; ++q) load(lo_e + (uint32_t)q * 64, q);
+        if (kMasked) {
+#pragma unroll
+            for (int q = 0; q < kAhead / 2; ++q) load_state(q);
         }
-        for (uint32_t c = lo_e; c < hi_e; c += 64) {
-            const uint32_t i = c + (uint32_t)lane;
-            bool v = i < hi_e;
-            if (kMasked && v) {
-                const uint32_t r = P.rid[i];
-                v = r < P.r_end && (P.keep[r] & 1u);
-            }
-            const uint64_t e = pf[0];
+        for (uint32_t c0 = lo_e; c0 < hi_e; c0 += kAhead * 64) {
 #pragma unroll
-            for (int q = 0; q + 1 < kAhead; ++q) pf[q] = pf[q + 1];
-            {
-                const uint32_t nx = c + (uint32_t)kAhead * 64 + (uint32_t)lane;
-                pf[kAhead - 1] = nx < hi_e ? P.ent2[nx] : 0;
-            }
-            const uint32_t key = v ? ((uint32_t)(e >> 32) & (kBucketBins - 1)) : 0u;
-            const uint64_t m = bin_match(slots[wave], key, v);
-            const uint32_t rank = (uint32_t)__popcll(m & lt);
-            if (v) {
-                if (bytes) {
-                    const uint32_t pre = sb[key];
-                    if (P.vq) {
+            for (int q = 0; q < kAhead; ++q) {
+                const uint32_t c = c0 + (uint32_t)q * 64;
+                if (c >= hi_e) break;
+                bool v = c + (uint32_t)lane < hi_e;
+                if (kMasked) v = v && (pk[kMasked ? q : 0] & 1u);
+                const uint64_t e = pf[q];
+                if (kMasked) load_state((q + kAhead / 2) % kAhead);
+                load(c + kAhead * 64, q);
+                const uint32_t key = v ? ((uint32_t)(e >> 32) & (kBucketBins - 1)) : 0u;
+                uint32_t pre;
+                uint32_t rank = 0, hits = 1;
+                if (bins_shared(sb, key, v, &pre)) {
+                    const uint64_t m = bin_match(slots[wave], key, v);
+                    rank = (uint32_t)__popcll(m & lt);
+                    hits = (uint32_t)__popcll(m);
+                }
+                if (v) {
+                    if (P.res1) {
                         // insert_and_query (bytestorage.cc:142-150): this table's
                         // count just after the event
                         const uint32_t after = pre + rank + 1;
-                        P.vq[(kb + (uint32_t)e) * kBinMaxTables + t] = (uint8_t)(after < 255u ? after : 255u);
+                        P.res1[(uint32_t)e] = (uint8_t)(after < 255u ? after : 255u);
                     } else if (pre + rank == 0) {
                         P.flags[kb + (uint32_t)e] = 1;
                     }
                     if (rank == 0) {
-                        const uint32_t post = pre + (uint32_t)__popcll(m);
+                        const uint32_t post = pre + hits;
                         sb[key] = (uint8_t)(post < 255u ? post : 255u);
                         occ += (t == 0 && pre == 0);
                     }
-                } else {
-                    const uint32_t bit = 1u << (key & 31u);
-                    const bool pre = (sw[key >> 5] & bit) != 0;
-                    if (!pre && rank == 0) {
-                        P.flags[kb + (uint32_t)e] = 1;
-                        atomicOr(&sw[key >> 5], bit);
-                        occ += (t == 0);
-                    }
                 }
+                __builtin_amdgcn_wave_barrier();
             }
-            __builtin_amdgcn_wave_barrier();
         }
-        for (uint32_t w = lane; w < nw; w += 64) src[w] = sw[w];
+        for (uint32_t w = lane; w < nw; w += 64) __builtin_nontemporal_store(sw[w], src + w);
         __builtin_amdgcn_wave_barrier();
     }
     add_counter(counters + kNOccupied, occ);
@@ -2898,28 +2996,55 @@ __global__ void seg_gather_kernel(const uint64_t* nb, const uint8_t* mask, const
     }
 }
 
-// insert_and_query results from the per-table counts after each event:
+// insert_and_query results of a tile's windows from its events' result bytes:
 // count = min over tables (the reference returns 1 for a new k-mer, and a
 // k-mer is new exactly when that minimum is 1); windows without events (N
-// holding, skipped) read -1.  Adds the new k-mers to n_unique.
-__global__ void bin_iq_combine_kernel(const uint32_t* vq, const int64_t* nk, uint32_t n_tables, int16_t* counts,
-                                      uint64_t* counters) {
-    const uint64_t n = (uint64_t)*nk;
-    const uint32_t mask = n_tables >= 4 ? 0xFFFFFFFFu : ((1u << (8 * n_tables)) - 1u);
+// holding, skipped) read -1.  Adds the new k-mers to n_unique.  The minimum
+// is taken in LDS, kRunLanes lanes per run of one first digit (about 32
+// events), three bytes read per event: bound by those bytes.  (A thread per
+// run, each on lines of its own, took 848 us per 2^27 starts.)
+constexpr int kRunLanes = 8;
+
+__global__ __launch_bounds__(kBlock) void bin_iq_combine_kernel(BinPlan P, int16_t* counts, uint64_t* counters) {
+    __shared__ uint32_t least[kBinTile];
+    __shared__ uint32_t run[kDigits1];
+    __shared__ uint16_t off[kDigits1 + 1];
+    static_assert(kBlock == kDigits1, "a thread per first digit");
+    constexpr uint32_t kNone = 0x100u;
     uint64_t n_new = 0;
-    for (uint64_t k = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; k < n; k += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t w = vq[k] & mask;
-        int16_t c = -1;
-        if (w) {
-            uint32_t mn = 255;
-            for (uint32_t t = 0; t < n_tables; ++t) {
-                const uint32_t b = (w >> (8 * t)) & 0xFFu;
-                mn = b < mn ? b : mn;
+    const uint32_t sub = threadIdx.x % kRunLanes;
+    for (uint32_t lt1 = blockIdx.x; lt1 < P.tiles1; lt1 += gridDim.x) {
+        const uint64_t k0 = P.tile_k0[lt1];
+        const uint32_t n_win = (uint32_t)(P.tile_k0[lt1 + 1] - k0);
+        run[threadIdx.x] = P.run1[(size_t)lt1 * kDigits1 + threadIdx.x];
+        off[threadIdx.x] = P.off1t[(size_t)lt1 * kDigits1 + threadIdx.x];
+        if (threadIdx.x == 0) off[kDigits1] = P.off1[(size_t)kDigits1 * P.tiles1 + lt1];
+        for (uint32_t i = threadIdx.x; i < (uint32_t)kBinTile; i += kBlock) least[i] = kNone;
+        __syncthreads();
+        const uint16_t* win = P.win1 + (size_t)lt1 * P.n_tables * kBinTile;
+#pragma unroll 4
+        for (uint32_t d = threadIdx.x / kRunLanes; d < P.n_d1; d += kBlock / kRunLanes) {
+            const uint32_t a = off[d], n = off[d + 1] - a;
+            for (uint32_t i = 4 * sub; i < n; i += 4 * kRunLanes) {
+                // up to 3 entries past the run are read and left out; both buffers
+                // end in that much room
+                uint32_t c4;
+                uint64_t w4;
+                __builtin_memcpy(&c4, P.res1 + run[d] + i, 4);
+                __builtin_memcpy(&w4, win + a + i, 8);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (i + q < n)
+                        atomicMin(&least[(uint32_t)(w4 >> (16 * q)) & (kBinTile - 1)], c4 >> (8 * q) & 0xFFu);
             }
-            c = (int16_t)mn;
-            n_new += mn == 1;
         }
-        if (counts) counts[k] = c;
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < n_win && i < (uint32_t)kBinTile; i += kBlock) {
+            const uint32_t c = least[i];
+            counts[k0 + i] = c == kNone ? (int16_t)-1 : (int16_t)c;
+            n_new += c == 1;
+        }
+        __syncthreads();
     }
     add_counter(counters + kNUnique, n_new);
 }
@@ -2997,13 +3122,6 @@ __global__ void dn_init_kernel(const int64_t* off, const int64_t* kmer_off, uint
     }
 }
 
-// Read of every event of the chunk (rid, aligned with ent2).
-__global__ void dn_event_reads_kernel(BinPlan P, const uint32_t* wread, uint32_t* rid) {
-    const uint32_t n = P.cnt2[(size_t)P.n_buckets * P.n_groups];
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        rid[i] = wread[(uint32_t)P.ent2[i]];
-}
-
 // The events [pos, ...) of one read rr that runs past a 64-event step: each
 // sees its bin as it was before the read; a kept read then raises its bins.
 // Returns the end of the read's events.
@@ -3064,22 +3182,32 @@ __global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, 
         uint32_t t, nw;
         bin_stage_slice(P, T, b, sw, &t, &nw);
         __builtin_amdgcn_wave_barrier();
-        // the events of the next two steps are loaded ahead: [pos, pos + 64)
-        // in (e, r), [pos + 64, pos + 128) in (eb, rb)
-        auto load = [&](uint32_t at, uint64_t& ex, uint32_t& rx) {
+        // Blocks of 64 events from pos are loaded kAhead ahead, the states of
+        // their reads kStates ahead; block 0 is the one taken.  (A state loaded
+        // in its own step waited a whole memory latency, and for the marks
+        // stored before it.)
+        constexpr int kAhead = 6, kStates = 4;
+        uint64_t ev[kAhead];
+        uint32_t rd[kAhead];
+        uint8_t sv[kStates];
+        auto load = [&](uint32_t at, int q) {
             const uint32_t i = at + (uint32_t)lane;
-            ex = i < hi_e ? P.ent2[i] : 0;
-            rx = i < hi_e ? rid[i] : 0xFFFFFFFFu;
+            ev[q] = i < hi_e ? __builtin_nontemporal_load(P.ent2 + i) : 0;
+            rd[q] = i < hi_e ? rid[i] : 0xFFFFFFFFu;
+        };
+        auto load_state = [&](int q) { sv[q] = rd[q] != 0xFFFFFFFFu ? state[rd[q]] : (uint8_t)0; };
+        auto refill = [&](uint32_t at) {
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q) load(at + (uint32_t)q * 64, q);
+#pragma unroll
+            for (int q = 0; q < kStates; ++q) load_state(q);
         };
         uint32_t pos = lo_e;
-        uint64_t e, eb;
-        uint32_t r, rb;
-        load(pos, e, r);
-        load(pos + 64u, eb, rb);
+        refill(pos);
         while (pos < hi_e) {
-            uint64_t ec;
-            uint32_t rc;
-            load(pos + 128u, ec, rc);
+            const uint64_t e = ev[0];
+            const uint32_t r = rd[0], rb = rd[1];
+            const uint8_t st0 = sv[0];
             const bool v = pos + (uint32_t)lane < hi_e;
             const uint32_t rn = __shfl(rb, 0);                              // read of event pos + 64
             const uint32_t rp = __shfl_up(r, 1);
@@ -3091,38 +3219,46 @@ __global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, 
                 if (s63 == 0) {
                     pos = dn_long_read(P, rid, state[__shfl(r, 0)], cutoff, fails, sb, slots[wave], pos, hi_e,
                                        __shfl(r, 0));
-                    load(pos, e, r);
-                    load(pos + 64u, eb, rb);
+                    refill(pos);
                     continue;
                 }
                 np = s63;
             }
             const bool act = (uint32_t)lane < np;
             const uint32_t key = act ? ((uint32_t)(e >> 32) & (kBucketBins - 1)) : 0u;
-            const uint64_t m = bin_match(slots[wave], key, act);
-            const uint8_t st = act ? state[r] : (uint8_t)0;
-            const uint64_t km = __ballot(act && (st & kDnKept));
-            const uint32_t first = 63u - (uint32_t)__clzll(bmask & le);      // first lane of my read
-            if (act) {
-                uint32_t seen = sb[key] + (uint32_t)__popcll(m & km & ((1ULL << first) - 1ULL));
-                seen = seen < 255u ? seen : 255u;
-                if (!(st & kDnSettled) && seen < cutoff) fails[(uint32_t)e] = 1;
+            const uint8_t st = act ? st0 : (uint8_t)0;
+            const bool kept = act && (st & kDnKept);
+            uint32_t pre, seen, hits = kept ? 1u : 0u;
+            bool writes = act;                              // the lane that writes its bin
+            if (bins_shared(sb, key, act, &pre)) {
+                const uint64_t m = bin_match(slots[wave], key, act);
+                const uint64_t km = m & __ballot(kept);
+                const uint32_t first = 63u - (uint32_t)__clzll(bmask & le);  // first lane of my read
+                seen = pre + (uint32_t)__popcll(km & ((1ULL << first) - 1ULL));
+                hits = (uint32_t)__popcll(km);
+                writes = act && !(m & lt);
+            } else {
+                seen = pre;
             }
-            __builtin_amdgcn_wave_barrier();
-            if (act && (st & kDnKept) && !(m & km & lt)) {
-                const uint32_t post = sb[key] + (uint32_t)__popcll(m & km);
+            if (act && !(st & kDnSettled) && (seen < 255u ? seen : 255u) < cutoff) fails[(uint32_t)e] = 1;
+            if (writes) {
+                const uint32_t post = pre + hits;
                 sb[key] = (uint8_t)(post < 255u ? post : 255u);
             }
             __builtin_amdgcn_wave_barrier();
             pos += np;
             if (np == 64u) {
-                e = eb;
-                r = rb;
-                eb = ec;
-                rb = rc;
+#pragma unroll
+                for (int q = 0; q + 1 < kAhead; ++q) {
+                    ev[q] = ev[q + 1];
+                    rd[q] = rd[q + 1];
+                }
+#pragma unroll
+                for (int q = 0; q + 1 < kStates; ++q) sv[q] = sv[q + 1];
+                load_state(kStates - 1);
+                load(pos + (uint32_t)(kAhead - 1) * 64, kAhead - 1);
             } else {
-                load(pos, e, r);
-                load(pos + 64u, eb, rb);
+                refill(pos);
             }
         }
     }
@@ -3199,13 +3335,6 @@ __global__ void dn_passed_kernel(const uint8_t* state, uint32_t r0, uint32_t r1,
 __global__ void fill_u8_kernel(uint8_t* p, uint64_t n, uint8_t v) {
     for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
         p[i] = v;
-}
-
-// Zeroes p[0, *n) (32-bit words).
-__global__ void zero_words_kernel(uint32_t* p, const int64_t* n) {
-    const uint64_t len = (uint64_t)*n;
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < len; i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = 0;
 }
 
 // Zeroes p[0, *n).
@@ -3462,8 +3591,8 @@ void launch_exact_keys(const ExactSet& E, uint64_t* out, uint64_t cap_out, unsig
 
 namespace gt {
 
-void launch_bin_kbase(const Reads& R, int64_t b0, uint64_t* out, hipStream_t s) {
-    bin_kbase_kernel<<<1, 64, 0, s>>>(R.off, R.kmer_off, R.n_reads, R.K, b0, out);
+void launch_bin_kbase(const Reads& R, int64_t b0, uint64_t* out, int64_t b1, uint64_t* out1, hipStream_t s) {
+    bin_kbase_kernel<<<1, 64, 0, s>>>(R.off, R.kmer_off, R.n_reads, R.K, b0, out, b1, out1);
 }
 
 void launch_bin_l1(const Reads& R, const Tables& T, const BinPlan& P, int grid, hipStream_t s) {
@@ -3488,8 +3617,14 @@ void launch_bin_l2_scatter(const BinPlan& P, int grid, hipStream_t s) {
         bin_l2_scatter_kernel<<<g, kBlock, 0, s>>>(P);
 }
 
+// Workgroups of the ordered replay: a wave per bucket, a multiple of the XCDs.
+static int ordered_grid(const BinPlan& P, int grid) {
+    const int64_t g = std::min<int64_t>(((int64_t)P.n_buckets + 3) / 4, grid);
+    return (int)((std::max<int64_t>(g, 1) + kXcds - 1) / kXcds * kXcds);
+}
+
 void launch_bin_apply(const BinPlan& P, const Tables& T, uint64_t* counters, int grid, hipStream_t s) {
-    if (P.unordered && !P.vq) {
+    if (P.unordered) {
         const int g = (int)std::min<int64_t>(std::max<int64_t>(P.n_buckets, 1), grid);
         if (T.kind == kByte)
             bin_apply_u_kernel<true><<<g, kApplyBlock, 0, s>>>(P, T, counters);
@@ -3497,8 +3632,7 @@ void launch_bin_apply(const BinPlan& P, const Tables& T, uint64_t* counters, int
             bin_apply_u_kernel<false><<<g, kApplyBlock, 0, s>>>(P, T, counters);
         return;
     }
-    const int g = (int)std::min<int64_t>(std::max<int64_t>((P.n_buckets + 3) / 4, 1), grid);
-    bin_apply_kernel<<<g, kBlock, 0, s>>>(P, T, counters);
+    bin_apply_kernel<<<ordered_grid(P, grid), kBlock, 0, s>>>(P, T, counters);
 }
 
 void launch_bin_read_new(const int64_t* kmer_off, uint64_t n_reads, const uint8_t* flags, uint64_t* n_new,
@@ -3522,11 +3656,6 @@ void launch_dn_init(const int64_t* off, const int64_t* kmer_off, uint32_t r0, ui
     dn_init_kernel<<<grid_of(r1 - r0, 4, 65535), 256, 0, s>>>(off, kmer_off, r0, r1, K, wread, state);
 }
 
-void launch_dn_event_reads(const BinPlan& P, const uint32_t* wread, uint32_t* rid, uint64_t max_events,
-                           hipStream_t s) {
-    dn_event_reads_kernel<<<grid_of(max_events, 256 * 4, 16384), 256, 0, s>>>(P, wread, rid);
-}
-
 void launch_dn_replay(const BinPlan& P, const Tables& T, const uint32_t* rid, const uint8_t* state, uint32_t cutoff,
                       uint8_t* fails, int grid, hipStream_t s) {
     const int g = (int)std::min<int64_t>(std::max<int64_t>((P.n_buckets + 3) / 4, 1), grid);
@@ -3547,8 +3676,7 @@ void launch_dn_passed(const uint8_t* state, uint32_t r0, uint32_t r1, uint8_t* p
 }
 
 void launch_dn_apply(const BinPlan& P, const Tables& T, uint64_t* counters, int grid, hipStream_t s) {
-    const int g = (int)std::min<int64_t>(std::max<int64_t>((P.n_buckets + 3) / 4, 1), grid);
-    dn_apply_kernel<<<g, kBlock, 0, s>>>(P, T, counters);
+    dn_apply_kernel<<<ordered_grid(P, grid), kBlock, 0, s>>>(P, T, counters);
 }
 
 void launch_zero_bytes(uint8_t* p, const int64_t* n, uint64_t max_n, hipStream_t s) {
@@ -3563,16 +3691,9 @@ void launch_seg_gather(const uint64_t* nb, const uint8_t* mask, const uint64_t* 
                                                                                out_mask);
 }
 
-void launch_bin_iq_combine(const uint32_t* vq, const int64_t* nk, uint64_t max_n, uint32_t n_tables, int16_t* counts,
-                           uint64_t* counters, hipStream_t s) {
-    const uint64_t g = (max_n + 255) / 256;
-    bin_iq_combine_kernel<<<(unsigned)(g < 16384 ? (g ? g : 1) : 16384), 256, 0, s>>>(vq, nk, n_tables, counts,
-                                                                                   counters);
-}
-
-void launch_zero_words(uint32_t* p, const int64_t* n, uint64_t max_n, hipStream_t s) {
-    const uint64_t g = (max_n + 255) / 256;
-    zero_words_kernel<<<(unsigned)(g < 16384 ? (g ? g : 1) : 16384), 256, 0, s>>>(p, n);
+void launch_bin_iq_combine(const BinPlan& P, int16_t* counts, uint64_t* counters, int grid, hipStream_t s) {
+    const int g = (int)std::min<int64_t>(std::max<int64_t>(P.tiles1, 1), grid);
+    bin_iq_combine_kernel<<<g, kBlock, 0, s>>>(P, counts, counters);
 }
 
 void launch_solid_reads(const int64_t* off, const int64_t* kmer_off, uint64_t n_reads, int K, const int16_t* counts,

@@ -82,7 +82,7 @@ void launch_exact_keys(const ExactSet& E, uint64_t* out, uint64_t cap_out, unsig
 
 // Binned insert of Bloom / count-min tables (one sub-batch = kbase, l1,
 // l2_count, scan, l2_scatter, apply; read_new once per call).
-void launch_bin_kbase(const Reads& R, int64_t b0, uint64_t* out, hipStream_t s);
+void launch_bin_kbase(const Reads& R, int64_t b0, uint64_t* out, int64_t b1, uint64_t* out1, hipStream_t s);
 void launch_bin_l1(const Reads& R, const Tables& T, const BinPlan& P, int grid, hipStream_t s);
 void launch_bin_l2_count(const BinPlan& P, int grid, hipStream_t s);
 void launch_bin_l2_scatter(const BinPlan& P, int grid, hipStream_t s);
@@ -90,22 +90,18 @@ void launch_bin_apply(const BinPlan& P, const Tables& T, uint64_t* counters, int
 void launch_bin_read_new(const int64_t* kmer_off, uint64_t n_reads, const uint8_t* flags, uint64_t* n_new,
                          uint64_t* counters, hipStream_t s);
 void launch_zero_bytes(uint8_t* p, const int64_t* n, uint64_t max_n, hipStream_t s);
-void launch_zero_words(uint32_t* p, const int64_t* n, uint64_t max_n, hipStream_t s);
 void launch_solid_reads(const int64_t* off, const int64_t* kmer_off, uint64_t n_reads, int K, const int16_t* counts,
                         uint32_t threshold, float min_prop_solid, uint8_t* passed, hipStream_t s);
 void launch_seg_gather(const uint64_t* nb, const uint8_t* mask, const uint64_t* idx, uint64_t n, uint64_t* out_nb,
                        uint8_t* out_mask, hipStream_t s);
-void launch_bin_iq_combine(const uint32_t* vq, const int64_t* nk, uint64_t max_n, uint32_t n_tables, int16_t* counts,
-                           uint64_t* counters, hipStream_t s);
+void launch_bin_iq_combine(const BinPlan& P, int16_t* counts, uint64_t* counters, int grid, hipStream_t s);
 void launch_fill_u8(uint8_t* p, uint64_t n, uint8_t v, hipStream_t s);
 
 // Batched diginorm over one chunk of reads [r0, r1) whose events are routed
-// (init, event_reads once; replay, ctl_reset, decide per guess; apply of the
+// (init before the routing; replay, ctl_reset, decide per guess; apply of the
 // kept reads and passed at the end).
 void launch_dn_init(const int64_t* off, const int64_t* kmer_off, uint32_t r0, uint32_t r1, int K, uint32_t* wread,
                     uint8_t* state, hipStream_t s);
-void launch_dn_event_reads(const BinPlan& P, const uint32_t* wread, uint32_t* rid, uint64_t max_events,
-                           hipStream_t s);
 void launch_dn_replay(const BinPlan& P, const Tables& T, const uint32_t* rid, const uint8_t* state, uint32_t cutoff,
                       uint8_t* fails, int grid, hipStream_t s);
 void launch_dn_decide(const int64_t* off, const int64_t* kmer_off, uint32_t r0, uint32_t r1, int K,

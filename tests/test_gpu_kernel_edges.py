@@ -155,3 +155,25 @@ def test_exact_set_moves_newness_and_grows(oracle):
     np.testing.assert_array_equal(g.insert_sequences(b), e_new)
     assert not g.S.insert(2 ** 64 - 1) and not o.insert(2 ** 64 - 1)
     assert g.n_unique() == o.n_unique
+
+
+@pytest.mark.parametrize('n_tables,sizes', [(1, [8191]), (2, [8192 * 3 + 1, 20011]), (3, [97, 101, 103]),
+                                            (4, [2_100_001, 2_100_011, 2_100_017, 2_100_019])])
+@pytest.mark.parametrize('sub', ['', '8192'])
+def test_insert_and_query_results_by_event_position(oracle, monkeypatch, n_tables, sizes, sub):
+    """Tiles whose first window lies in a short read, in a gap between reads or
+    mid-read, N bases, counts past 255, a last partial tile; one sub-batch and
+    several."""
+    monkeypatch.setenv('GOETIA_AMD_SUB_BATCH', sub)
+    K = 31
+    for seed, lengths in ((1, [40]), (2, [2048, 30, 2047, 31, 1]), (3, [5, 9000, 12, 0, 0, 3000]), (4, [150] * 700)):
+        g, o = _pair(oracle, 2, sizes, K, mode=N.MODE_SKIP_N)
+        b = _reads(seed, lengths, genome=max(1500, max(lengths)), n_rate=0.002)
+        hot = np.frombuffer(b'AC' * 400, np.uint8)
+        b = ReadBatch(np.concatenate([b.seq, hot]), np.append(b.offsets, b.n_bases + len(hot)))
+        for _ in range(2):
+            exp = o.insert_and_query_reads(b.seq, b.offsets, K, True, N.MODE_SKIP_N)
+            np.testing.assert_array_equal(g.insert_and_query_sequences(b), exp)
+        for x, y in zip(g.get_raw(), o.tables()):
+            np.testing.assert_array_equal(x, y)
+        assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
