@@ -245,7 +245,7 @@ struct gt_storage {
     DevBuf solid_counts;               // insert_and_query counts of a solid-filter batch
     // batched diginorm: read of every routed event and window, windows with
     // events, windows failing the cutoff, per-read state, iteration control
-    DevBuf dn_rid, dn_wread, dn_hasev, dn_fails, dn_state, dn_ctl;
+    DevBuf dn_rid, dn_wread, dn_hasev, dn_fails, dn_state, dn_ctl, dn_ends;
     uint64_t gen_issued = 0;           // generation bumps enqueued so far (device kGen follows it)
     uint64_t epoch = 0;                // bumped when device table pointers change (exact-set growth)
     std::vector<struct gt_pipeline*> pipelines;   // attached pipelines
@@ -1898,6 +1898,7 @@ int gt_diginorm_dev(gt_storage* st, uint16_t K, int canonical, int mode, const u
     GT_TRY(st->dn_fails.ensure(win_max));
     GT_TRY(st->dn_state.ensure(n_reads));
     GT_TRY(st->dn_ctl.ensure(2 * sizeof(uint32_t)));
+    GT_TRY(st->dn_ends.ensure((uint64_t)P.n_buckets * sizeof(uint32_t)));
     GT_TRY(sc.bin_flags.ensure(std::max<uint64_t>((uint64_t)kof[n_reads], 1)));
     uint32_t* rid = st->dn_rid.as<uint32_t>();
     uint32_t* wread = st->dn_wread.as<uint32_t>();
@@ -1924,6 +1925,7 @@ int gt_diginorm_dev(gt_storage* st, uint16_t K, int canonical, int mode, const u
         const uint64_t n_win = (uint64_t)(kof[r1] - kof[r0]);
         if (n_win) {
             P.hasev = hasev;
+            P.ends = nullptr;
             bin_route(R, T, P, sc, off[r0], off[r1], s);
             P.hasev = nullptr;
             bool settled = false;
@@ -1932,7 +1934,10 @@ int gt_diginorm_dev(gt_storage* st, uint16_t K, int canonical, int mode, const u
                 {
                     ProfScope ps("dn_replay", s);
                     launch_fill_u8(fails, n_win, 0, s);
-                    launch_dn_replay(P, T, rid, state, cutoff, fails, grid, s);
+                    // an odd guess makes drops final: the next replay leaves their events out
+                    uint32_t* ends = g % 2 == 0 ? st->dn_ends.as<uint32_t>() : nullptr;
+                    launch_dn_replay(P, T, rid, state, cutoff, fails, ends, grid, s);
+                    if (ends) P.ends = ends;
                 }
                 {
                     ProfScope ps("dn_decide", s);

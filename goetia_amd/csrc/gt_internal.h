@@ -143,6 +143,7 @@ struct BinPlan {
     const uint32_t* wread;                // read of every window of the sub-batch: the ordered scatter
                                           // then writes rid
     const uint8_t* keep;
+    const uint32_t* ends;                 // diginorm, optional: end of each bucket's remaining events
     uint32_t r_end;
     uint8_t* hasev;                       // optional, per window of the sub-batch: the first pass
                                           // writes 1 for windows with events, 0 for skipped ones

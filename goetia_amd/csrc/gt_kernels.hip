@@ -2697,7 +2697,7 @@ __device__ __forceinline__ void bin_apply_body(const BinPlan& P, const Tables& T
         const uint32_t b = ((xcd + kXcds * (x >> P.shift2)) << P.shift2) | (x & ((1u << P.shift2) - 1u));
         if (b >= P.n_buckets) continue;
         const uint32_t lo_e = P.cnt2[(size_t)b * P.n_groups];
-        const uint32_t hi_e = P.cnt2[(size_t)(b + 1) * P.n_groups];
+        const uint32_t hi_e = kMasked && P.ends ? P.ends[b] : P.cnt2[(size_t)(b + 1) * P.n_groups];
         if (lo_e == hi_e) continue;
         uint32_t t = 0;
         uint64_t pt = T.p[0];
@@ -2945,7 +2945,6 @@ __global__ __launch_bounds__(kBlock) void dn_apply_kernel(BinPlan P, Tables T, u
 // bytes.  (A thread per read over flags staged in LDS spent 225 us on 1M
 // reads of 120 windows, most of it on one counter atomic per wave.)
 constexpr int kReadLanes = 16;
-constexpr int kReadNewStage = 32768;
 
 // Sum of v over the kReadLanes lanes of a read.
 __device__ __forceinline__ uint32_t read_lanes_sum(uint32_t v) {
@@ -3166,8 +3165,16 @@ __device__ uint32_t dn_long_read(const BinPlan& P, const uint32_t* rid, uint8_t 
 // guessed-kept read then raise their bins, saturating at 255
 // (bytestorage.cc:60-113).  The events of one read are consecutive within a
 // bucket; a step takes the whole reads among the next 64 events.
-__global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, const uint32_t* rid,
-                                                           const uint8_t* state, uint32_t cutoff, uint8_t* fails) {
+//
+// The events of a read that is finally dropped say nothing more: they mark no
+// window and raise no bin.  With kCompact (guesses after one whose drops are
+// final) a wave moves the events that still matter to the front of its bucket
+// as it goes, in order, and leaves their end in P.ends: past the cutoff's
+// coverage most reads are dropped by the first guess, and the guesses that
+// follow, and the insert of the kept reads, then take a fraction of the events.
+template <bool kCompact>
+__global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, uint32_t* rid, const uint8_t* state,
+                                                           uint32_t cutoff, uint8_t* fails, uint32_t* ends) {
     __shared__ uint32_t slice[4][kBucketBins / 4];
     __shared__ uint64_t slots[4][256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -3177,8 +3184,11 @@ __global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, 
     uint8_t* sb = reinterpret_cast<uint8_t*>(sw);
     for (uint32_t b = blockIdx.x * 4u + (uint32_t)wave; b < P.n_buckets; b += gridDim.x * 4u) {
         const uint32_t lo_e = P.cnt2[(size_t)b * P.n_groups];
-        const uint32_t hi_e = P.cnt2[(size_t)(b + 1) * P.n_groups];
-        if (lo_e == hi_e) continue;
+        const uint32_t hi_e = P.ends ? P.ends[b] : P.cnt2[(size_t)(b + 1) * P.n_groups];
+        if (lo_e == hi_e) {
+            if (kCompact && lane == 0) ends[b] = hi_e;
+            continue;
+        }
         uint32_t t, nw;
         bin_stage_slice(P, T, b, sw, &t, &nw);
         __builtin_amdgcn_wave_barrier();
@@ -3203,6 +3213,7 @@ __global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, 
             for (int q = 0; q < kStates; ++q) load_state(q);
         };
         uint32_t pos = lo_e;
+        uint32_t kept_end = lo_e;                           // kCompact: end of the events moved so far
         refill(pos);
         while (pos < hi_e) {
             const uint64_t e = ev[0];
@@ -3217,8 +3228,21 @@ __global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, 
                 // the last read of the step goes on past it
                 const uint32_t s63 = 63u - (uint32_t)__clzll(bmask);
                 if (s63 == 0) {
-                    pos = dn_long_read(P, rid, state[__shfl(r, 0)], cutoff, fails, sb, slots[wave], pos, hi_e,
-                                       __shfl(r, 0));
+                    const uint32_t from = pos;
+                    const uint8_t st = state[__shfl(r, 0)];
+                    pos = dn_long_read(P, rid, st, cutoff, fails, sb, slots[wave], pos, hi_e, __shfl(r, 0));
+                    if (kCompact && (st & (kDnKept | kDnSettled)) != kDnSettled) {
+                        for (uint32_t c = from; c < pos; c += 64) {
+                            const uint32_t i = c + (uint32_t)lane;
+                            const uint64_t x = i < pos ? P.ent2[i] : 0;
+                            const uint32_t y = i < pos ? rid[i] : 0;
+                            if (i < pos) {
+                                P.ent2[kept_end + lane] = x;
+                                rid[kept_end + lane] = y;
+                            }
+                            kept_end += pos - c < 64u ? pos - c : 64u;
+                        }
+                    }
                     refill(pos);
                     continue;
                 }
@@ -3246,6 +3270,17 @@ __global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, 
                 sb[key] = (uint8_t)(post < 255u ? post : 255u);
             }
             __builtin_amdgcn_wave_barrier();
+            if (kCompact) {
+                // at or before the events of this step, all of them read
+                const bool stays = act && (st & (kDnKept | kDnSettled)) != kDnSettled;
+                const uint64_t sm = __ballot(stays);
+                if (stays) {
+                    const uint32_t to = kept_end + (uint32_t)__popcll(sm & lt);
+                    P.ent2[to] = e;
+                    rid[to] = r;
+                }
+                kept_end += (uint32_t)__popcll(sm);
+            }
             pos += np;
             if (np == 64u) {
 #pragma unroll
@@ -3261,6 +3296,7 @@ __global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, 
                 refill(pos);
             }
         }
+        if (kCompact && lane == 0) ends[b] = kept_end;
     }
 }
 
@@ -3269,44 +3305,48 @@ __global__ __launch_bounds__(kBlock) void dn_replay_kernel(BinPlan P, Tables T, 
 // computed as the reference does (diginorm.hh:43).  With `upper` set the new
 // guess is an upper bound of the kept set (the one replayed was a lower
 // bound), so its drops are final; otherwise its keeps are.  ctl[0] counts
-// reads whose guess changed, ctl[1] is the first read not yet final.  A
-// thread per read; a workgroup's kBlock reads have one contiguous window
-// range, staged in LDS when it fits.
+// reads whose guess changed, ctl[1] is the first read not yet final.
+// kReadLanes lanes share a read and take its windows four at a time; reads
+// that are final cost their state byte (a thread per read over windows staged
+// in LDS took 131 us per guess of 2^25 starts, settled reads or not).
 __global__ __launch_bounds__(kBlock) void dn_decide_kernel(const int64_t* off, const int64_t* kmer_off, uint32_t r0,
                                                            uint32_t r1, int K, const uint8_t* hasev,
                                                            const uint8_t* fails, int upper, uint8_t* state,
                                                            uint32_t* ctl) {
-    __shared__ uint8_t ok[kReadNewStage];
+    constexpr uint64_t kReads = kBlock / kReadLanes;
+    const int sub = threadIdx.x % kReadLanes;
     const int64_t kb = kmer_off[r0];
     uint32_t changed = 0, first_open = 0xFFFFFFFFu;
-    for (uint64_t q0 = r0 + (uint64_t)blockIdx.x * kBlock; q0 < r1; q0 += (uint64_t)gridDim.x * kBlock) {
-        const uint64_t q1 = q0 + kBlock < r1 ? q0 + kBlock : r1;
-        const int64_t w0 = kmer_off[q0] - kb, w1 = kmer_off[q1] - kb;
-        const bool staged = w1 - w0 <= kReadNewStage;
-        __syncthreads();
-        if (staged)
-            for (int64_t i = threadIdx.x; i < w1 - w0; i += kBlock) ok[i] = hasev[w0 + i] && !fails[w0 + i];
-        __syncthreads();
-        const uint64_t r = q0 + threadIdx.x;
-        if (r >= q1) continue;
-        const uint8_t st = state[r];
-        if (st & kDnSettled) continue;
-        const int64_t a = kmer_off[r] - kb, b = kmer_off[r + 1] - kb;
+    for (uint64_t q0 = r0 + (uint64_t)blockIdx.x * kReads; q0 < r1; q0 += (uint64_t)gridDim.x * kReads) {
+        const uint64_t r = q0 + threadIdx.x / kReadLanes;
+        const uint8_t st = r < r1 ? state[r] : kDnSettled;
         uint32_t c = 0;
-        if (staged) {
-            for (int64_t w = a; w < b; ++w) c += ok[w - w0];
-        } else {
-            for (int64_t w = a; w < b; ++w) c += (hasev[w] && !fails[w]) ? 1u : 0u;
+        if (!(st & kDnSettled)) {
+            const int64_t a = kmer_off[r] - kb, b = kmer_off[r + 1] - kb;
+            for (int64_t w = a + 4 * sub; w < b; w += 4 * kReadLanes) {
+                if (w + 4 <= b) {
+                    uint32_t h, f;                          // bytes of 0 or 1
+                    __builtin_memcpy(&h, hasev + w, 4);
+                    __builtin_memcpy(&f, fails + w, 4);
+                    c += (uint32_t)__popc(h & ~f);
+                } else {
+                    for (int64_t i = w; i < b; ++i) c += (hasev[i] && !fails[i]) ? 1u : 0u;
+                }
+            }
         }
-        const uint64_t n_kmers = (uint64_t)(off[r + 1] - off[r]) - (uint64_t)K + 1u;
-        const uint32_t min_req = (uint32_t)(0.5 + (double)((float)n_kmers / 2));
-        const bool keep = c < min_req;
-        const bool settled = upper ? !keep : keep;
-        changed += keep != ((st & kDnKept) != 0);
-        state[r] = (uint8_t)((keep ? kDnKept : 0) | (settled ? kDnSettled : 0));
-        if (!settled && (uint32_t)r < first_open) first_open = (uint32_t)r;
+        c = read_lanes_sum(c);
+        if (sub == 0 && !(st & kDnSettled)) {
+            const uint64_t n_kmers = (uint64_t)(off[r + 1] - off[r]) - (uint64_t)K + 1u;
+            const uint32_t min_req = (uint32_t)(0.5 + (double)((float)n_kmers / 2));
+            const bool keep = c < min_req;
+            const bool settled = upper ? !keep : keep;
+            changed += keep != ((st & kDnKept) != 0);
+            state[r] = (uint8_t)((keep ? kDnKept : 0) | (settled ? kDnSettled : 0));
+            if (!settled && (uint32_t)r < first_open) first_open = (uint32_t)r;
+        }
     }
-    // one atomic per wavefront
+    // one atomic per workgroup
+    __shared__ uint32_t part[2][kBlock / 64];
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
         changed += __shfl_xor(changed, d);
@@ -3314,6 +3354,15 @@ __global__ __launch_bounds__(kBlock) void dn_decide_kernel(const int64_t* off, c
         first_open = o < first_open ? o : first_open;
     }
     if ((threadIdx.x & 63) == 0) {
+        part[0][threadIdx.x >> 6] = changed;
+        part[1][threadIdx.x >> 6] = first_open;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / 64; ++w) {
+            changed += part[0][w];
+            first_open = part[1][w] < first_open ? part[1][w] : first_open;
+        }
         if (changed) atomicAdd(&ctl[0], changed);
         if (first_open != 0xFFFFFFFFu) atomicMin(&ctl[1], first_open);
     }
@@ -3656,16 +3705,19 @@ void launch_dn_init(const int64_t* off, const int64_t* kmer_off, uint32_t r0, ui
     dn_init_kernel<<<grid_of(r1 - r0, 4, 65535), 256, 0, s>>>(off, kmer_off, r0, r1, K, wread, state);
 }
 
-void launch_dn_replay(const BinPlan& P, const Tables& T, const uint32_t* rid, const uint8_t* state, uint32_t cutoff,
-                      uint8_t* fails, int grid, hipStream_t s) {
+void launch_dn_replay(const BinPlan& P, const Tables& T, uint32_t* rid, const uint8_t* state, uint32_t cutoff,
+                      uint8_t* fails, uint32_t* ends, int grid, hipStream_t s) {
     const int g = (int)std::min<int64_t>(std::max<int64_t>((P.n_buckets + 3) / 4, 1), grid);
-    dn_replay_kernel<<<g, kBlock, 0, s>>>(P, T, rid, state, cutoff, fails);
+    if (ends)
+        dn_replay_kernel<true><<<g, kBlock, 0, s>>>(P, T, rid, state, cutoff, fails, ends);
+    else
+        dn_replay_kernel<false><<<g, kBlock, 0, s>>>(P, T, rid, state, cutoff, fails, nullptr);
 }
 
 void launch_dn_decide(const int64_t* off, const int64_t* kmer_off, uint32_t r0, uint32_t r1, int K,
                       const uint8_t* hasev, const uint8_t* fails, int upper, uint8_t* state, uint32_t* ctl,
                       hipStream_t s) {
-    dn_decide_kernel<<<grid_of(r1 - r0, kBlock, 16384), kBlock, 0, s>>>(off, kmer_off, r0, r1, K, hasev, fails,
+    dn_decide_kernel<<<grid_of(r1 - r0, kBlock / kReadLanes, 2048), kBlock, 0, s>>>(off, kmer_off, r0, r1, K, hasev, fails,
                                                                           upper, state, ctl);
 }
 

@@ -177,3 +177,27 @@ def test_insert_and_query_results_by_event_position(oracle, monkeypatch, n_table
         for x, y in zip(g.get_raw(), o.tables()):
             np.testing.assert_array_equal(x, y)
         assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+
+
+@pytest.mark.parametrize('K,cutoff,chunk,guesses', [(21, 3, '', ''), (31, 5, '2048', ''), (31, 5, '16384', '3'),
+                                                    (17, 20, '', '2')])
+def test_diginorm_leaves_out_events_of_dropped_reads(oracle, monkeypatch, K, cutoff, chunk, guesses):
+    """High coverage over small tables (several events of a step on one bin),
+    reads that fill a bucket's step with their own events (tandem repeats),
+    N bases, short reads; chunks cut by the guess cap; two batches."""
+    monkeypatch.setenv('GOETIA_AMD_DIGINORM_CHUNK', chunk)
+    monkeypatch.setenv('GOETIA_AMD_DIGINORM_GUESSES', guesses)
+    g, o = _pair(oracle, 2, [9001, 9011, 9013], K, mode=N.MODE_SKIP_N)
+    f = lg.DiginormFilter.build(g, cutoff)
+    for seed in (1, 2):
+        b = _reads(seed, [90, K - 1, K, 150, 70] * 260, genome=1500, sub=0.01, n_rate=0.001)
+        rep = np.frombuffer((b'ACGTT' * 60 + b'A' * 90) * 3, np.uint8)
+        off = b.offsets
+        for _ in range(6):
+            off = np.append(off, off[-1] + len(rep))
+        b = ReadBatch(np.concatenate([b.seq] + [rep] * 6), off)
+        exp = o.diginorm_reads(b.seq, b.offsets, K, cutoff, True, N.MODE_SKIP_N)
+        np.testing.assert_array_equal(f.filter_sequences(b), np.asarray(exp, bool))
+        for x, y in zip(g.get_raw(), o.tables()):
+            np.testing.assert_array_equal(x, y)
+        assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
