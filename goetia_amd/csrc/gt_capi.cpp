@@ -716,18 +716,29 @@ uint32_t bin_buckets(const gt_storage* st) {
 }
 
 // Whether an insert goes through the binned path.  GOETIA_AMD_BINNED=0 / 1
-// forces it off / on (where the tables allow it); by default it is used for
-// batches of at least 2^20 bases with at least one base per 256 table bins,
-// where replaying buckets in LDS beats random atomics on the tables (on
-// 4 x 2^28 count-min bins, 4.5M-base batches insert 3.7e9 k-mers/s binned
-// against 2.2e9 with atomics, 1.2M-base batches 1.4e9 against 1.8e9).
+// forces it off / on (where the tables allow it); by default it is used from
+// 2^14 bases plus 5 per bucket on, about where the two paths cross: it passes
+// over every bucket that has an event (up to 6 ns each), and the atomic insert
+// takes 0.3 to 0.9 ns more per base.  Reset and insert of 150-base reads, us
+// (atomic / binned):
+//   4 x 1e6 bits       500 reads  101 /   75    2000 reads  170 /   95
+//   4 x 3e7 counts     500 reads  240 /  165    2000 reads  401 /  178
+//   4 x 2^28 bits     2000 reads  374 /  566    6000 reads  878 /  594
+//   4 x 2^28 counts   2000 reads  622 /  964    6000 reads 1178 / 1024
 bool use_binned(const gt_storage* st, const Scratch& sc, const Reads& R) {
-    if (R.dyn || sc.fixed || !bin_buckets(st)) return false;
+    const uint32_t buckets = bin_buckets(st);
+    if (R.dyn || sc.fixed || !buckets) return false;
     const char* v = std::getenv("GOETIA_AMD_BINNED");
     if (v && *v) return v[0] != '0';
-    uint64_t bins = 0;
-    for (uint64_t p : st->sizes) bins += p;
-    return (uint64_t)R.n_bases >= (1ULL << 20) && (uint64_t)R.n_bases * 256 >= bins;
+    return (uint64_t)R.n_bases >= (1ULL << 14) + 5 * (uint64_t)buckets;
+}
+
+// First-pass tiles per second-pass work item: kBinGroup, or fewer when that
+// leaves the second pass fewer than four items per CU.
+uint32_t bin_group(uint32_t n_d1, uint64_t tiles) {
+    uint32_t g = kBinGroup;
+    while (g > 64 && (uint64_t)n_d1 * ((tiles + g - 1) / g) < 4 * (uint64_t)g_dev.cus) g /= 2;
+    return g;
 }
 
 // Binned sub-batch in start positions, a multiple of kTileMax: 2^27 for an
@@ -765,7 +776,8 @@ int bin_prepare(gt_storage* st, Scratch& sc, uint64_t tiles_max, BinPlan& P) {
     P.shift2 = bits > (uint32_t)kDigitBits1 ? bits - (uint32_t)kDigitBits1 : 0u;
     P.n_d1 = (nb + (1u << P.shift2) - 1) >> P.shift2;
 
-    const uint64_t groups_max = (tiles_max + kBinGroup - 1) / kBinGroup;
+    P.group = bin_group(P.n_d1, tiles_max);
+    const uint64_t groups_max = (tiles_max + P.group - 1) / P.group;
     const uint64_t n_ent = tiles_max * nt * kBinTile;
     const uint64_t cnt_max = ((uint64_t)P.n_d1 << P.shift2) * groups_max;
     int rc = sc.bin_ent1.ensure(n_ent * sizeof(uint64_t));
@@ -789,7 +801,7 @@ int bin_prepare(gt_storage* st, Scratch& sc, uint64_t tiles_max, BinPlan& P) {
 // for sub-batches of up to tiles_max first-pass tiles.
 int res_prepare(const gt_storage* st, Scratch& sc, uint64_t tiles_max, BinPlan& P) {
     const uint64_t n_ent = tiles_max * st->n_tables * kBinTile;
-    const uint64_t groups_max = (tiles_max + kBinGroup - 1) / kBinGroup;
+    const uint64_t groups_max = (tiles_max + P.group - 1) / P.group;
     const uint64_t k0_bytes = (tiles_max + 1) * sizeof(uint64_t);
     const uint64_t run_bytes = tiles_max * kDigits1 * sizeof(uint32_t);
     const uint64_t item_bytes = kDigits1 * groups_max * sizeof(uint32_t);
@@ -817,11 +829,14 @@ void bin_route(const Reads& R, const Tables& T, BinPlan& P, Scratch& sc, int64_t
     Rs.b1 = b1;
     P.tile0 = b0 / kBinTile;
     P.tiles1 = (uint32_t)((b1 + kBinTile - 1) / kBinTile - P.tile0);
-    P.n_groups = (P.tiles1 + kBinGroup - 1) / kBinGroup;
+    P.n_groups = (P.tiles1 + P.group - 1) / P.group;
     const uint64_t cnt_len = ((uint64_t)P.n_d1 << P.shift2) * P.n_groups;
     const int grid_l1 = std::max(1, g_dev.cus * 2);     // 70 KB of LDS per workgroup
     const int grid = std::max(1, g_dev.cus * 8);
-    launch_bin_kbase(R, b0, sc.bin_kbase.as<uint64_t>(), b1, P.tile_k0 ? P.tile_k0 + P.tiles1 : nullptr, s);
+    // (a plain insert's first sub-batch starts at packed index 0, which the
+    // flags' zeroing has stored)
+    if (b0 != 0 || !P.unordered)
+        launch_bin_kbase(R, b0, sc.bin_kbase.as<uint64_t>(), b1, P.tile_k0 ? P.tile_k0 + P.tiles1 : nullptr, s);
     {
         ProfScope ps("bin_hash", s);
         launch_bin_l1(Rs, T, P, grid_l1, s);
@@ -858,7 +873,7 @@ int binned_insert_impl(gt_storage* st, Scratch& sc, const Reads& R, uint64_t* n_
             GT_TRY(sc.bin_flags.ensure((size_t)R.n_bases));
             flags = sc.bin_flags.as<uint8_t>();
         }
-        launch_zero_bytes(flags, R.kmer_off + R.n_reads, (uint64_t)R.n_bases, s);
+        launch_zero_bytes(flags, R.kmer_off + R.n_reads, (uint64_t)R.n_bases, sc.bin_kbase.as<uint64_t>(), s);
     }
     P.flags = flags;
     P.unordered = iq ? 0u : 1u;        // a plain insert's replay does not depend on event order

@@ -98,7 +98,7 @@ constexpr int kDigitBits2 = 9;
 constexpr int kDigits2 = 1 << kDigitBits2;        // largest second-pass fan-out
 constexpr int kBinTile = 2048;                    // starts per first-pass tile (512 threads x 4)
 constexpr uint32_t kBinMaxTables = 4;
-constexpr uint32_t kBinGroup = 1024;              // first-pass tiles per second-pass work item
+constexpr uint32_t kBinGroup = 1024;              // most first-pass tiles per second-pass work item
 constexpr int kBinChunk = 4096;                   // events staged in LDS per second-pass step
 constexpr uint32_t kMaxBuckets = 1u << (kDigitBits1 + kDigitBits2);
 constexpr uint32_t kNoBin = 0xFFFFFFFFu;
@@ -116,7 +116,8 @@ struct BinPlan {
     uint32_t n_d1;                        // first-pass digits in use
     int64_t tile0;                        // first first-pass tile (absolute) of the sub-batch
     uint32_t tiles1;                      // first-pass tiles of the sub-batch
-    uint32_t n_groups;                    // ceil(tiles1 / kBinGroup)
+    uint32_t group;                       // first-pass tiles per second-pass work item
+    uint32_t n_groups;                    // ceil(tiles1 / group)
     uint64_t* ent1;                       // per tile a region of n_tables * kBinTile events, by d1
     uint16_t* dig2;                       // second digit of each ent1 event (same index)
     uint64_t* ent2;                       // events by bucket, event order within a bucket

@@ -2241,10 +2241,10 @@ __device__ uint32_t bin_load_runs(const BinPlan& P, uint32_t d1, uint32_t grp, B
 #pragma unroll
     for (int k = 0; k < kRunsPerThread; ++k) {
         const uint32_t j = threadIdx.x * kRunsPerThread + k;
-        const uint32_t lt = grp * kBinGroup + j;
+        const uint32_t lt = grp * P.group + j;
         uint32_t st = 0;
         len[k] = 0;
-        if (lt < P.tiles1) {
+        if (j < P.group && lt < P.tiles1) {
             const uint32_t a = P.off1[(size_t)d1 * P.tiles1 + lt];
             const uint32_t b = P.off1[(size_t)(d1 + 1) * P.tiles1 + lt];
             st = lt * P.n_tables * kBinTile + a;
@@ -2327,29 +2327,31 @@ __device__ __forceinline__ void bin_chunk_load_d2(const BinPlan& P, const BinRun
 
 // For each (first digit, group) item: events per second digit, from the
 // first pass's digit array; a chunk's loads are issued two chunks ahead.  A
-// workgroup counts kCountGroups consecutive groups of one first digit, so
-// each second digit's counts for them (adjacent in cnt2) go out as one write.
+// workgroup counts up to kCountGroups consecutive groups (`per`) of one first
+// digit, so each second digit's counts for them (adjacent in cnt2) go out as
+// one write; a small sub-batch takes fewer, since 8 of a 13M-window batch's 8
+// groups left one workgroup per digit: 241 us, as much as hashing the batch.
 constexpr uint32_t kCountGroups = 8;
 
 // 512 threads: the count's chains of dependent loads (run offsets, then
 // digits) overlap across eight waves per workgroup.
 constexpr int kCountBlock = 2 * kBlock;
 
-__global__ __launch_bounds__(kCountBlock) void bin_l2_count_kernel(BinPlan P) {
+__global__ __launch_bounds__(kCountBlock) void bin_l2_count_kernel(BinPlan P, uint32_t per) {
     constexpr int BLK = kCountBlock;
     __shared__ BinRuns sh;
     __shared__ uint32_t hist[kCountGroups][kDigits2];
     __shared__ uint32_t first[kBinChunk / 64];
     constexpr int kQ = kBinChunk / BLK;
-    const uint32_t g_blocks = (P.n_groups + kCountGroups - 1) / kCountGroups;
+    const uint32_t g_blocks = (P.n_groups + per - 1) / per;
     const uint32_t n_blocks = P.n_d1 * g_blocks;
     const uint32_t mask2 = (1u << P.shift2) - 1u;
     uint32_t da[kQ], db[kQ];
     for (uint32_t blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
-        const uint32_t d1 = blk / g_blocks, grp0 = (blk % g_blocks) * kCountGroups;
-        const uint32_t ng = P.n_groups - grp0 < kCountGroups ? P.n_groups - grp0 : kCountGroups;
+        const uint32_t d1 = blk / g_blocks, grp0 = (blk % g_blocks) * per;
+        const uint32_t ng = P.n_groups - grp0 < per ? P.n_groups - grp0 : per;
         __syncthreads();
-        for (uint32_t x = threadIdx.x; x < kCountGroups * (uint32_t)kDigits2; x += BLK) (&hist[0][0])[x] = 0;
+        for (uint32_t x = threadIdx.x; x < per * (uint32_t)kDigits2; x += BLK) (&hist[0][0])[x] = 0;
         for (uint32_t gi = 0; gi < ng; ++gi) {
             uint32_t* h = hist[gi];
             const uint32_t n = bin_load_runs<BLK>(P, d1, grp0 + gi, sh);
@@ -2378,8 +2380,8 @@ __global__ __launch_bounds__(kCountBlock) void bin_l2_count_kernel(BinPlan P) {
             __syncthreads();                               // bin_load_runs of the next group reuses sh
         }
         // lanes take (digit, group) pairs group-fastest: a digit's groups are adjacent words of cnt2
-        for (uint32_t x = threadIdx.x; x < kCountGroups * (mask2 + 1u); x += BLK) {
-            const uint32_t d2 = x / kCountGroups, gi = x % kCountGroups;
+        for (uint32_t x = threadIdx.x; x < per * (mask2 + 1u); x += BLK) {
+            const uint32_t d2 = x / per, gi = x % per;
             if (gi < ng) P.cnt2[(size_t)((d1 << P.shift2) | d2) * P.n_groups + grp0 + gi] = hist[gi][d2];
         }
     }
@@ -2421,8 +2423,8 @@ __global__ __launch_bounds__(kBlock) void bin_l2_scatter_kernel(BinPlan P) {
             uint32_t all;
             block_exclusive_u32(before, sh.runs.part, &all);
             item0 = P.cnt2[(size_t)(d1 << P.shift2) * P.n_groups] + all;
-            for (uint32_t j = threadIdx.x; j < kBinGroup && grp * kBinGroup + j < P.tiles1; j += kBlock)
-                P.run1[(size_t)(grp * kBinGroup + j) * kDigits1 + d1] = item0 + sh.runs.rpre[j];
+            for (uint32_t j = threadIdx.x; j < P.group && grp * P.group + j < P.tiles1; j += kBlock)
+                P.run1[(size_t)(grp * P.group + j) * kDigits1 + d1] = item0 + sh.runs.rpre[j];
         }
         // chunk c's events are loaded while chunk c - 1 is sorted
         uint64_t v[kBinChunk / kBlock];
@@ -3386,9 +3388,10 @@ __global__ void fill_u8_kernel(uint8_t* p, uint64_t n, uint8_t v) {
         p[i] = v;
 }
 
-// Zeroes p[0, *n).
-__global__ void zero_bytes_kernel(uint8_t* p, const int64_t* n) {
+// Zeroes p[0, *n), and *also when given.
+__global__ void zero_bytes_kernel(uint8_t* p, const int64_t* n, uint64_t* also) {
     const uint64_t len = (uint64_t)*n;
+    if (also && blockIdx.x == 0 && threadIdx.x == 0) *also = 0;
     for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < len; i += (uint64_t)gridDim.x * blockDim.x)
         p[i] = 0;
 }
@@ -3653,9 +3656,12 @@ void launch_bin_l1(const Reads& R, const Tables& T, const BinPlan& P, int grid, 
 }
 
 void launch_bin_l2_count(const BinPlan& P, int grid, hipStream_t s) {
-    const int64_t blocks = (int64_t)P.n_d1 * ((P.n_groups + kCountGroups - 1) / kCountGroups);
+    // as many groups a workgroup as leave half of the grid busy, at most kCountGroups
+    const int64_t items = (int64_t)P.n_d1 * P.n_groups;
+    const uint32_t per = (uint32_t)std::min<int64_t>(kCountGroups, std::max<int64_t>(items / (grid / 2 > 0 ? grid / 2 : 1), 1));
+    const int64_t blocks = (int64_t)P.n_d1 * ((P.n_groups + per - 1) / per);
     const int g = (int)std::min<int64_t>(std::max<int64_t>(blocks, 1), grid);
-    bin_l2_count_kernel<<<g, kCountBlock, 0, s>>>(P);
+    bin_l2_count_kernel<<<g, kCountBlock, 0, s>>>(P, per);
 }
 
 void launch_bin_l2_scatter(const BinPlan& P, int grid, hipStream_t s) {
@@ -3731,9 +3737,9 @@ void launch_dn_apply(const BinPlan& P, const Tables& T, uint64_t* counters, int 
     dn_apply_kernel<<<ordered_grid(P, grid), kBlock, 0, s>>>(P, T, counters);
 }
 
-void launch_zero_bytes(uint8_t* p, const int64_t* n, uint64_t max_n, hipStream_t s) {
+void launch_zero_bytes(uint8_t* p, const int64_t* n, uint64_t max_n, uint64_t* also, hipStream_t s) {
     const uint64_t g = (max_n + 255) / 256;
-    zero_bytes_kernel<<<(unsigned)(g < 16384 ? (g ? g : 1) : 16384), 256, 0, s>>>(p, n);
+    zero_bytes_kernel<<<(unsigned)(g < 16384 ? (g ? g : 1) : 16384), 256, 0, s>>>(p, n, also);
 }
 
 void launch_seg_gather(const uint64_t* nb, const uint8_t* mask, const uint64_t* idx, uint64_t n, uint64_t* out_nb,
@@ -3755,9 +3761,38 @@ void launch_solid_reads(const int64_t* off, const int64_t* kmer_off, uint64_t n_
                                                                                 threshold, min_prop_solid, passed);
 }
 
+// The same for a short array by one workgroup.
+constexpr int kScanSmallBlock = 1024;
+constexpr uint64_t kScanSmall = 16 * kScanSmallBlock;
+
+__global__ __launch_bounds__(kScanSmallBlock) void scan_u32_small_kernel(uint32_t* a, uint32_t n) {
+    __shared__ uint32_t part[kScanSmallBlock / 64];
+    const uint32_t per = (n + kScanSmallBlock - 1) / kScanSmallBlock;
+    const uint32_t i0 = threadIdx.x * per < n ? threadIdx.x * per : n, i1 = i0 + per < n ? i0 + per : n;
+    uint32_t v[16];
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 16; ++j) {
+        v[j] = i0 + j < i1 ? a[i0 + j] : 0u;
+        sum += v[j];
+    }
+    uint32_t total;
+    uint32_t run = block_exclusive_u32<kScanSmallBlock>(sum, part, &total);
+#pragma unroll
+    for (uint32_t j = 0; j < 16; ++j) {
+        if (i0 + j < i1) a[i0 + j] = run;
+        run += v[j];
+    }
+    if (threadIdx.x == 0) a[n] = total;
+}
+
 uint64_t scan_u32_block_count(uint64_t n) { return (n + kScanU32Chunk - 1) / kScanU32Chunk; }
 
 void launch_scan_u32(uint32_t* a, uint64_t n, uint32_t* sums, hipStream_t s) {
+    if (n <= kScanSmall) {
+        scan_u32_small_kernel<<<1, kScanSmallBlock, 0, s>>>(a, (uint32_t)n);
+        return;
+    }
     const uint64_t nb = scan_u32_block_count(n);
     if (nb) scan_u32_sums_kernel<<<(unsigned)nb, kBlock, 0, s>>>(a, n, sums);
     scan_u32_blocks_kernel<<<1, kBlock, 0, s>>>(sums, nb, a + n);

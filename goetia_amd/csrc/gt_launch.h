@@ -89,7 +89,7 @@ void launch_bin_l2_scatter(const BinPlan& P, int grid, hipStream_t s);
 void launch_bin_apply(const BinPlan& P, const Tables& T, uint64_t* counters, int grid, hipStream_t s);
 void launch_bin_read_new(const int64_t* kmer_off, uint64_t n_reads, const uint8_t* flags, uint64_t* n_new,
                          uint64_t* counters, hipStream_t s);
-void launch_zero_bytes(uint8_t* p, const int64_t* n, uint64_t max_n, hipStream_t s);
+void launch_zero_bytes(uint8_t* p, const int64_t* n, uint64_t max_n, uint64_t* also, hipStream_t s);
 void launch_solid_reads(const int64_t* off, const int64_t* kmer_off, uint64_t n_reads, int K, const int16_t* counts,
                         uint32_t threshold, float min_prop_solid, uint8_t* passed, hipStream_t s);
 void launch_seg_gather(const uint64_t* nb, const uint8_t* mask, const uint64_t* idx, uint64_t n, uint64_t* out_nb,

@@ -97,10 +97,13 @@ def test_per_read_sums_and_solid_reads_at_every_length(oracle, monkeypatch, spre
 
 @pytest.mark.parametrize('kind,n_tables', [(1, 1), (1, 4), (1, 6), (2, 2), (2, 4), (2, 9), (3, 0)])
 @pytest.mark.parametrize('K,mode', [(21, N.MODE_RAW), (31, N.MODE_SKIP_N), (255, N.MODE_RAW)])
-def test_small_batches_take_windows_together(oracle, kind, n_tables, K, mode):
+@pytest.mark.parametrize('binned', ['0', '1'])
+def test_small_batches_take_windows_together(oracle, monkeypatch, kind, n_tables, K, mode, binned):
     """Batches around one tile of 1024 starts, hot k-mers (several windows of a
     thread on one bin or slot), reads below K, N bases, and a second batch over
-    the first one's keys: n_new, flags, counts, counters, tables."""
+    the first one's keys: n_new, flags, counts, counters, tables; through the
+    atomic insert and, where the tables allow it, the binned one."""
+    monkeypatch.setenv('GOETIA_AMD_BINNED', binned)
     sizes = [4001, 4003, 4007, 4013, 4019, 4021, 4027, 4049, 4051][:n_tables]
     for lengths in ([K], [K - 1, K + 3], [300, 0, 421, 300, 3], [1024], [1025], [257] * 40, [150] * 300):
         g, o = _pair(oracle, kind, sizes, K, mode=mode)
@@ -122,9 +125,11 @@ def test_small_batches_take_windows_together(oracle, kind, n_tables, K, mode):
 
 
 @pytest.mark.parametrize('n_reads', [1, 1023, 1025, 16384, 16385])
-def test_layout_of_small_batches(oracle, n_reads):
+@pytest.mark.parametrize('binned', ['0', '1'])
+def test_layout_of_small_batches(oracle, monkeypatch, n_reads, binned):
     """Either side of the one-launch layout's limit: packed results of reads of
     0 to 60 bases, and one long read over many tiles."""
+    monkeypatch.setenv('GOETIA_AMD_BINNED', binned)
     K = 21
     rng = np.random.default_rng(n_reads)
     lengths = rng.integers(0, 60, n_reads)
@@ -201,3 +206,24 @@ def test_diginorm_leaves_out_events_of_dropped_reads(oracle, monkeypatch, K, cut
         for x, y in zip(g.get_raw(), o.tables()):
             np.testing.assert_array_equal(x, y)
         assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+
+
+@pytest.mark.parametrize('kind,max_table', [(1, 40_009), (2, 2_000_003), (2, 60_000_011)])
+@pytest.mark.parametrize('n_reads', [130, 900, 9000])
+def test_binned_insert_in_small_groups(oracle, monkeypatch, kind, max_table, n_reads):
+    """Batches whose second pass takes 64 to 1024 tiles per item and one or
+    more of them per counting workgroup, and whose counts are scanned by one
+    workgroup or several."""
+    monkeypatch.setenv('GOETIA_AMD_BINNED', '1')
+    K, sizes = 31, oracle.primes_near_x(4, max_table)
+    g, o = _pair(oracle, kind, sizes, K)
+    for seed in (1, 2):
+        b = _reads(seed, [150] * n_reads, genome=20_000)
+        _, e_new = o.insert_reads(b.seq, b.offsets, K)
+        np.testing.assert_array_equal(g.insert_sequences(b), e_new)
+        if kind == 2:
+            exp = o.insert_and_query_reads(b.seq, b.offsets, K)
+            np.testing.assert_array_equal(g.insert_and_query_sequences(b), exp)
+    for x, y in zip(g.get_raw(), o.tables()):
+        np.testing.assert_array_equal(x, y)
+    assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
