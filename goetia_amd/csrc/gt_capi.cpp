@@ -355,8 +355,7 @@ int alloc_exact(gt_storage* st, uint64_t cap, hipStream_t s) {
 
 int zero_tables(gt_storage* st, hipStream_t s) {
     if (st->kind == kExact) {
-        launch_fill_u64(st->ekv.as<uint64_t>(), 2 * (st->ecap + 1), ~0ULL, s);
-        launch_fill_u64(st->eones.as<uint64_t>(), 1, 0, s);
+        launch_exact_clear(st->exact_view(), st->counters.as<uint64_t>(), s);
     } else {
         launch_fill_u64(st->tables.as<uint64_t>(), st->tables.bytes / 8, 0, s);
     }
@@ -741,13 +740,18 @@ uint32_t bin_group(uint32_t n_d1, uint64_t tiles) {
     return g;
 }
 
-// Binned sub-batch in start positions, a multiple of kTileMax: 2^27 for an
-// insert, 2^26 for insert_and_query (a first digit's result bytes are then
-// 1 MB, a quarter of an XCD's L2: 22.0 ms for the replays of 4M reads against
-// 24.1 at 2^27 and 27 at 2^25), or GOETIA_AMD_BIN_SUB (at most 2^29); capped
-// by GOETIA_AMD_SUB_BATCH.
+// Binned sub-batch in start positions, a multiple of kTileMax: even parts of
+// the batch of at most 2^27 for an insert and 2^26 for insert_and_query (a
+// first digit's result bytes are then 1 MB, a quarter of an XCD's L2: 22.0 ms
+// for the replays of 4M reads against 24.1 at 2^27 and 27 at 2^25), or the
+// whole batch when that is at most a quarter over: every sub-batch passes over
+// the tables, and the 16M starts that 1M reads of 150 leave past 2^27 took as
+// long to replay (2.1 ms) as the rest.  GOETIA_AMD_BIN_SUB sets the size (at
+// most 2^29); GOETIA_AMD_SUB_BATCH caps it.
 uint64_t bin_sub_batch(uint64_t n_bases, bool iq) {
-    uint64_t sb = iq ? 1ULL << 26 : 1ULL << 27;
+    const uint64_t most = iq ? 1ULL << 26 : 1ULL << 27;
+    uint64_t sb = n_bases;
+    if (n_bases > most + most / 4) sb = (n_bases + (n_bases + most - 1) / most - 1) / ((n_bases + most - 1) / most);
     if (const char* v = std::getenv("GOETIA_AMD_BIN_SUB")) {
         const unsigned long long x = std::strtoull(v, nullptr, 10);
         if (x) sb = std::min<uint64_t>(x, 1ULL << 29);
@@ -1291,10 +1295,7 @@ int gt_storage_reset(gt_storage* st) {
     StorageLock lk(st);
     GT_TRY(lk.rc);
     GT_TRY(zero_tables(st, nullptr));
-    if (st->kind == kExact) {
-        launch_fill_u64(st->counters.as<uint64_t>() + kNUnique, 2, 0, nullptr);   // n_unique, last-was-present
-        st->ecount_ub = 0;
-    }
+    if (st->kind == kExact) st->ecount_ub = 0;
     GT_HIP(hipStreamSynchronize(nullptr));
     return GT_OK;
 }

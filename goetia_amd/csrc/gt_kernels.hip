@@ -1827,6 +1827,20 @@ __global__ void fill_u64_kernel(uint64_t* p, uint64_t n, uint64_t v) {
         p[i] = v;
 }
 
+// An empty exact set: every key and stamp word all ones, the all-ones key
+// absent, n_unique and last-was-present 0 (one launch; a small set's reset is
+// its launches).
+__global__ void exact_clear_kernel(ExactSet E, uint64_t* counters) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *E.ones = 0;
+        counters[kNUnique] = 0;
+        counters[kNOccupied] = 0;
+    }
+    ulonglong2* p = reinterpret_cast<ulonglong2*>(E.kv);
+    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i <= E.cap; i += (uint64_t)gridDim.x * blockDim.x)
+        p[i] = make_ulonglong2(~0ULL, ~0ULL);
+}
+
 // Bloom union (bitstorage.cc:103-137): me |= other, counting table-0 bits
 // that become set.
 __global__ void bit_union_kernel(uint32_t* me, const uint32_t* other, uint64_t n_words, int count_bits,
@@ -3625,6 +3639,11 @@ void launch_bit_union(uint32_t* me, const uint32_t* other, uint64_t n_words, int
     const uint64_t g = (n_words + 255) / 256;
     bit_union_kernel<<<(unsigned)(g < 2048 ? (g ? g : 1) : 2048), 256, 0, s>>>(me, other, n_words, count_bits,
                                                                               counters);
+}
+
+void launch_exact_clear(const ExactSet& E, uint64_t* counters, hipStream_t s) {
+    const uint64_t g = E.cap / 256 + 1;
+    exact_clear_kernel<<<(unsigned)(g < 16384 ? g : 16384), 256, 0, s>>>(E, counters);
 }
 
 void launch_exact_rehash(const ExactSet& from, const ExactSet& to, uint64_t* counters, hipStream_t s) {

@@ -58,6 +58,7 @@ void launch_hash_query(const Launch& L, const uint64_t* h, uint64_t n, const Tab
 
 void launch_bit_union(uint32_t* me, const uint32_t* other, uint64_t n_words, int count_bits, uint64_t* counters,
                       hipStream_t s);
+void launch_exact_clear(const ExactSet& E, uint64_t* counters, hipStream_t s);
 void launch_exact_rehash(const ExactSet& from, const ExactSet& to, uint64_t* counters, hipStream_t s);
 // Count-min insert_and_query of n values in index order (fw[k], or
 // min(fw, rc) when rc is set and canonical), sort-based (gt_sorted_iq.hip);
