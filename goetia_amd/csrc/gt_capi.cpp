@@ -858,6 +858,112 @@ void bin_route(const Reads& R, const Tables& T, BinPlan& P, Scratch& sc, int64_t
     }
 }
 
+// ------------------------------------------------------------ routed query
+
+// Digits of a routed query over a storage's tables (0: not eligible).
+uint32_t route_digits(const gt_storage* st) {
+    if ((st->kind != kByte && st->kind != kBit) || st->n_tables == 0 || st->n_tables > kBinMaxTables) return 0;
+    uint64_t nd = 0;
+    for (uint64_t p : st->sizes) {
+        if (p >= (1ULL << 30)) return 0;                 // the passes' fast modulus
+        nd += (p + (1ULL << kRouteShift) - 1) >> kRouteShift;
+    }
+    return nd <= (uint64_t)kRouteDigits ? (uint32_t)nd : 0;
+}
+
+// Whether a query goes through the routed passes (GOETIA_AMD_ROUTED=0 / 1
+// forces it off / on where the tables allow it): by default on two tables or
+// more of 30 MiB together (smaller ones are read mostly out of the L2s as they
+// are; one table's reads cost less than their routing), from 2^23 bases plus
+// one per 64 table bytes on (every slice is read into an L2 once per
+// sub-batch).  150-base reads, us (direct / routed):
+//   4 x 2^21 counts   300k reads 1332 / 3278
+//   4 x 2^23 counts   30k reads  247 /  382    100k  792 /  729     1M 7431 / 6016
+//   4 x 2^25 counts   30k reads  293 /  333    100k  937 /  848     1M 8852 / 5473
+//   4 x 2^28 counts   100k reads 980 / 1002    300k 2790 / 2316     1M 8947 / 6931
+//   4 x 2^28 bits     30k reads  270 /  267    100k  859 /  670     1M 8076 / 5984
+//   2 x 2^28 bits     30k reads  152 /  188    100k  458 /  414     1M 4183 / 3707
+//   1 x 2^28 counts   1M reads  2468 / 3255
+bool use_routed(const gt_storage* st, const Scratch& sc, const Reads& R) {
+    if (R.dyn || sc.fixed || !route_digits(st)) return false;
+    const char* v = std::getenv("GOETIA_AMD_ROUTED");
+    if (v && *v) return v[0] != '0';
+    uint64_t bytes = 0;
+    for (uint64_t nb : st->nbytes) bytes += nb;
+    return st->n_tables >= 2 && bytes >= (30ULL << 20) && (uint64_t)R.n_bases >= (1ULL << 23) + bytes / 64;
+}
+
+// Query of prepared reads through the routed passes, in sub-batches of 2^27
+// starts (GOETIA_AMD_BIN_SUB and GOETIA_AMD_SUB_BATCH as the binned insert).
+int routed_query_impl(gt_storage* st, Scratch& sc, const Reads& R, int16_t* counts, uint64_t* hashes, hipStream_t s) {
+    const uint64_t sub = bin_sub_batch((uint64_t)R.n_bases, false);
+    const uint64_t tiles_max = sub / kBinTile;
+    const uint32_t stride = route_stride(st->n_tables);
+    RoutePlan P{};
+    P.n_tables = st->n_tables;
+    for (uint32_t i = 0; i < st->n_tables; ++i) {
+        P.dfirst[i] = P.n_digits;
+        P.n_digits += (uint32_t)((st->sizes[i] + (1ULL << kRouteShift) - 1) >> kRouteShift);
+    }
+    P.dfirst[st->n_tables] = P.n_digits;
+    // the insert's event buffers: a storage that was filled in batches has them
+    const uint64_t blocks = (uint64_t)P.n_digits * ((tiles_max + 63) / 64);
+    const uint64_t next_bytes = 16 * kRouteNextStep * sizeof(uint32_t), k0_bytes = (tiles_max + 1) * sizeof(uint64_t);
+    const uint64_t off_bytes = ((P.n_digits + 1) * tiles_max * sizeof(uint16_t) + 15) / 16 * 16;
+    GT_TRY(sc.bin_ent1.ensure(tiles_max * stride * sizeof(uint32_t)));
+    GT_TRY(sc.bin_res1.ensure(tiles_max * stride + 16));          // the combine reads past a run's end
+    GT_TRY(sc.bin_tile.ensure(next_bytes + k0_bytes + off_bytes));
+    GT_TRY(sc.bin_ent2.ensure((uint64_t)P.n_digits * tiles_max * sizeof(uint32_t)));
+    GT_TRY(sc.bin_cnt2.ensure((blocks + 1) * sizeof(uint32_t)));
+    GT_TRY(sc.bin_sums.ensure((scan_u32_block_count(blocks) + 1) * sizeof(uint32_t)));
+    P.ent = sc.bin_ent1.as<uint32_t>();
+    P.res = sc.bin_res1.as<uint8_t>();
+    P.next = sc.bin_tile.as<uint32_t>();
+    P.tile_k0 = reinterpret_cast<uint64_t*>(sc.bin_tile.as<uint8_t>() + next_bytes);
+    P.off = reinterpret_cast<uint16_t*>(sc.bin_tile.as<uint8_t>() + next_bytes + k0_bytes);
+    P.run = sc.bin_ent2.as<uint32_t>();
+    P.blk = sc.bin_cnt2.as<uint32_t>();
+    const Tables T = st->tables_view();
+    for (int64_t b0 = 0; b0 < R.n_bases; b0 += (int64_t)sub) {
+        Reads Rs = R;
+        Rs.b0 = b0;
+        Rs.b1 = std::min<int64_t>(R.n_bases, b0 + (int64_t)sub);
+        P.tile0 = b0 / kBinTile;
+        P.tiles = (uint32_t)((Rs.b1 + kBinTile - 1) / kBinTile - P.tile0);
+        launch_bin_kbase(R, b0, nullptr, Rs.b1, P.tile_k0 + P.tiles, s);
+        {
+            ProfScope ps("query_route", s);
+            launch_route(Rs, T, P, hashes, g_dev.cus, s);
+        }
+        {
+            ProfScope ps("query_gather", s);
+            launch_route_count(P, s);
+            launch_scan_u32(P.blk, route_blocks(P), sc.bin_sums.as<uint32_t>(), s);
+            launch_route_gather(T, P, g_dev.cus, s);
+        }
+        {
+            ProfScope ps("query_combine", s);
+            launch_route_combine(P, counts, g_dev.cus, s);
+        }
+        GT_HIP(hipGetLastError());
+    }
+    return GT_OK;
+}
+
+// Query of prepared reads.
+int query_impl(gt_storage* st, Scratch& sc, const Reads& R, int16_t* counts, uint64_t* hashes, hipStream_t s) {
+    if (counts && use_routed(st, sc, R)) {
+        const int rc = routed_query_impl(st, sc, R, counts, hashes, s);
+        if (rc != GT_ERR_OUT_OF_MEMORY) return rc;
+        sc.bin_ent1.release();          // no room for the lookups: read the tables window by window
+        sc.bin_res1.release();
+    }
+    ProfScope ps("query", s);
+    launch_query(make_launch(st, (uint64_t)R.n_bases, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
+    GT_HIP(hipGetLastError());
+    return GT_OK;
+}
+
 // Binned insert of prepared reads (tile_read and kmer_off set): per
 // sub-batch, route the (window, table) events by bin and replay each bucket
 // in LDS; then per-read new counts from the window flags, or, with iq_counts
@@ -1682,11 +1788,7 @@ int gt_dbg_query_dev(gt_storage* st, uint16_t K, int canonical, int mode, const 
     hipStream_t s = (hipStream_t)stream;
     Reads R = make_reads(seq, offsets, n_reads, n_bases, K, mode, canonical);
     GT_TRY(prepare_reads(st, R, true, s));
-    {
-        ProfScope ps("query", s);
-        launch_query(make_launch(st, n_bases, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
-    }
-    GT_HIP(hipGetLastError());
+    GT_TRY(query_impl(st, st->own, R, counts, hashes, s));
     if (st->use_bigcount && st->big.aux) {
         // ByteStorage::query's bigcount step for counts of 255 (bytestorage.cc:130-137)
         int64_t nk = 0;
@@ -1782,9 +1884,7 @@ int gt_dbg_insert_and_query_dev(gt_storage* st, uint16_t K, int canonical, int m
     // sparseppstorage.cc:21-25); a query after the batch gives exactly that
     // (and -1 for skipped windows).
     GT_TRY(prepare_reads(st, R, true, s));
-    launch_query(make_launch(st, n_bases, s), R, st->tables_view(), st->exact_or_empty(), counts, nullptr);
-    GT_HIP(hipGetLastError());
-    return GT_OK;
+    return query_impl(st, st->own, R, counts, nullptr, s);
 }
 
 int gt_dbg_insert_and_query(gt_storage* st, uint16_t K, int canonical, int mode, const uint8_t* seq,
@@ -2711,11 +2811,7 @@ int gt_dbg_query_ws_dev(gt_storage* st, gt_workspace* ws, uint16_t K, int canoni
     hipStream_t s = (hipStream_t)stream;
     Reads R = make_reads(seq, offsets, n_reads, n_bases, K, mode, canonical);
     GT_TRY(prepare_reads(ws->sc, R, true, s));
-    {
-        ProfScope ps("query", s);
-        launch_query(make_launch(st, n_bases, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
-    }
-    GT_HIP(hipGetLastError());
+    GT_TRY(query_impl(st, ws->sc, R, counts, hashes, s));
     return GT_OK;
 }
 

@@ -152,6 +152,34 @@ struct BinPlan {
                                           // inserts); 0: window order (insert_and_query, diginorm)
 };
 
+// Routed query of Bloom / count-min tables: the (window, table) lookups of a
+// sub-batch are sorted per tile by digit, a slice of 2^shift consecutive bins
+// of one table, so that one XCD at a time reads a slice out of its L2.  A
+// lookup is the u32 bin within its digit << kRouteWinBits | window within its
+// tile; tile lt's lookups start at lt * route_stride().
+constexpr int kRouteDigits = 512;
+constexpr int kRouteWinBits = 11;                 // log2(kBinTile)
+constexpr uint32_t kRouteShift = 32 - kRouteWinBits;
+struct RoutePlan {
+    uint32_t n_tables;
+    uint32_t n_digits;
+    uint32_t dfirst[kBinMaxTables + 1];   // first digit of each table
+    int64_t tile0;                        // first tile (absolute) of the sub-batch
+    uint32_t tiles;
+    uint32_t* ent;
+    uint8_t* res;                         // the table's answer to each lookup: by digit, then by tile
+    uint32_t* blk;                        // n_digits x blocks of 64 tiles (+1): lookups, then first index in res
+    uint32_t* run;                        // n_digits x tiles: index in res of a digit's lookups of a tile
+    uint16_t* off;                        // (kRouteDigits + 1) x tiles, digit-major: start of a digit in its tile
+    uint64_t* tile_k0;                    // per tile and one past: packed index of its first window
+    uint32_t* next;                       // per XCD, kRouteNextStep words apart: blocks handed out by the gather
+};
+constexpr uint32_t kRouteNextStep = 64;
+// Lookups per tile region, with a pad of one L2 channel (256 bytes): a digit's
+// lookups lie at about the same place of every region, and regions a power of
+// two apart would put them all into one channel.
+__host__ __device__ inline uint32_t route_stride(uint32_t n_tables) { return n_tables * kBinTile + 64; }
+
 // One call's view of the reads.  Starts s in [b0, b1) are processed; the
 // ordinal of the k-mer at s is s - b0.  With `dyn` set, n_reads and n_bases
 // are upper bounds and the actual sizes are read from device memory, so one

@@ -3104,6 +3104,277 @@ __global__ __launch_bounds__(kBlock) void solid_reads_kernel(const int64_t* off,
     }
 }
 
+// ------------------------------------------------------------ routed query
+//
+// A query's table reads are random 128-byte lines, 55.7e9 a second past the
+// L2s, but 255e9 from lines that an XCD's 4 MB L2 holds.  Large batches over
+// large tables therefore go through three passes:
+//
+//   route    hash a tile's windows, sort its (window, table) lookups by slice
+//            of 2 MB (a digit) in LDS and write them to the tile's region;
+//   gather   the workgroups of one XCD take the lookups of one digit at a time,
+//            read its slice through their L2 and write a byte per lookup;
+//   combine  per tile, the minimum over the tables in LDS, written as counts.
+//
+// 20M reads of 150 bases against 4 x 2^28 counts: 172 ms window by window,
+// 139 ms so (route 43, gather 70, combine 24, the counts between them 1.5).
+
+// Route pass over one tile: BLK threads of PER windows each, whose lookups
+// stay in registers until their places are known.
+constexpr int kRouteBlock = 512;
+constexpr int kRoutePer = kBinTile / kRouteBlock;
+static_assert(kBinTile == 1 << kRouteWinBits, "a lookup holds its window's place in its tile");
+
+struct RouteShared {
+    union {
+        uint32_t sorted[kBinMaxTables * kBinTile];
+        SegScratchT<kRouteBlock + kSegExtra> seg;     // stitched window starts (before end_tile)
+    };
+    uint32_t cnt[kRouteDigits];                       // lookups per digit, then their starts
+    uint32_t part[kRouteBlock / 64];
+    uint64_t k0;                                      // packed index of the tile's first window
+};
+
+struct RouteOp {
+    Tables T;
+    RoutePlan P;
+    const int64_t* kmer_off;
+    const int64_t* off;
+    int K;
+    uint64_t* hashes;
+    RouteShared* sh;
+    const TileSharedT<kBinTile>* tile_sh;
+    uint32_t ev[kBinMaxTables][kRoutePer];
+    uint32_t at[kBinMaxTables][kRoutePer];            // digit << 16 | place among the tile's of that digit
+    uint32_t have;                                    // valid windows
+    static constexpr bool kTogether = true;
+    static_assert(kRouteBlock >= kRouteDigits, "one thread per digit");
+
+    __device__ SegScratchT<kRouteBlock + kSegExtra>* seg_scratch() { return &sh->seg; }
+    __device__ void begin_tile(int64_t t0) {
+        have = 0;
+        if (threadIdx.x < kRouteDigits) sh->cnt[threadIdx.x] = 0;
+        if (threadIdx.x == 0) {
+            // (read after the barrier of the stitched starts)
+            const uint32_t r = tile_sh->r_lo;
+            const int64_t a = off[r], wins = off[r + 1] - a - K + 1;
+            int64_t d = t0 - a;
+            d = d < 0 || wins <= 0 ? 0 : (d > wins ? wins : d);
+            sh->k0 = (uint64_t)(kmer_off[r] + d);
+            P.tile_k0[t0 / kBinTile - P.tile0] = sh->k0;
+        }
+    }
+    template <int PER>
+    __device__ void together(const Windows<PER>& w) {
+        have = w.valid;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (!(w.in >> j & 1u)) continue;
+            const int64_t k = kmer_off[w.r[j]] + (w.s0 + j - w.rstart[j]);
+            const bool valid = w.valid >> j & 1u;
+            if (hashes) hashes[k] = valid ? w.h[j] : 0;
+            if (!valid) continue;
+            const uint32_t win = (uint32_t)((uint64_t)k - sh->k0) & (kBinTile - 1);
+#pragma unroll
+            for (uint32_t t = 0; t < kBinMaxTables; ++t) {
+                if (t >= P.n_tables) continue;
+                const uint32_t bin = gt_fastmod30(w.h[j], (uint32_t)T.p[t], T.m[t]);
+                const uint32_t d = P.dfirst[t] + (bin >> kRouteShift);
+                ev[t][j] = bin << kRouteWinBits | win;         // the digit's bits shift out
+                at[t][j] = d << 16 | atomicAdd(&sh->cnt[d], 1u);
+            }
+        }
+    }
+    __device__ void flush() {}
+    __device__ void end_tile(int64_t tile) {
+        __syncthreads();
+        const uint32_t lt = (uint32_t)(tile - P.tile0);
+        const uint32_t d = threadIdx.x;
+        uint32_t n_ev;
+        const uint32_t start = block_exclusive_u32<kRouteBlock>(d < kRouteDigits ? sh->cnt[d] : 0u, sh->part, &n_ev);
+        if (d < kRouteDigits) {
+            if (d < P.n_digits) P.off[(size_t)d * P.tiles + lt] = (uint16_t)start;
+            sh->cnt[d] = start;
+        }
+        if (d == 0) P.off[(size_t)P.n_digits * P.tiles + lt] = (uint16_t)n_ev;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t t = 0; t < kBinMaxTables; ++t) {
+#pragma unroll
+            for (int j = 0; j < kRoutePer; ++j)
+                if (t < P.n_tables && (have >> j & 1u)) sh->sorted[sh->cnt[at[t][j] >> 16] + (at[t][j] & 0xFFFFu)] = ev[t][j];
+        }
+        __syncthreads();
+        uint32_t* dst = P.ent + (size_t)lt * route_stride(P.n_tables);
+        for (uint32_t i = 4 * threadIdx.x; i < n_ev; i += 4 * kRouteBlock)   // past n_ev: inside the region, never read
+            *reinterpret_cast<uint4*>(dst + i) = *reinterpret_cast<const uint4*>(sh->sorted + i);
+    }
+};
+
+__global__ __launch_bounds__(kRouteBlock, 4) void route_kernel(Reads R, Tables T, RoutePlan P, uint64_t* hashes) {
+    __shared__ TileSharedT<kBinTile> sh;
+    __shared__ RouteShared rs;
+    if (blockIdx.x == 0 && threadIdx.x < kXcds) P.next[threadIdx.x * kRouteNextStep] = 0;   // for the gather after it
+    RouteOp op{T, P, R.kmer_off, R.off, R.K, hashes, &rs, &sh, {}, {}, 0};
+    walk_tiles<kRoutePer, kRouteBlock>(R, sh, op);
+}
+
+// Lookups of every digit in every block of 64 tiles (a wave each).
+__global__ __launch_bounds__(kBlock) void route_count_kernel(RoutePlan P) {
+    const uint32_t n_blk = (P.tiles + 63) / 64, n = P.n_digits * n_blk;
+    const uint32_t lane = threadIdx.x & 63;
+    for (uint32_t x = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); x < n; x += gridDim.x * (kBlock / 64)) {
+        const uint32_t d = x / n_blk, lt = x % n_blk * 64 + lane;
+        uint32_t c = 0;
+        if (lt < P.tiles) c = P.off[(size_t)(d + 1) * P.tiles + lt] - P.off[(size_t)d * P.tiles + lt];
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+        if (lane == 0) P.blk[x] = c;
+    }
+}
+
+// Gather pass.  LPR lanes take one tile's run of a digit, so 64 / LPR tiles
+// at a time of a wave's 64; the reads of several tiles are in flight together.
+// Bound by the L2's random reads; lookups go past it, and a wave's answers are
+// one run of whole lines (16 bytes per tile and digit, left in the tiles' own
+// regions, took 26 of 95 ms for 20M reads).  An XCD's waves take
+// blocks of 64 tiles in order from one counter, digit by digit: walking fixed
+// shares they drifted apart until their slices no longer fit the L2 together
+// (139 ms for 20M reads, against 102 with the counter alone).
+template <bool kBytes, int LPR>
+__global__ __launch_bounds__(kBlock) void route_gather_kernel(Tables T, RoutePlan P) {
+    constexpr int kAt = 64 / LPR;                     // tiles at a time
+    constexpr int kDeep = 8;                          // rounds of them in flight
+    const int lane = threadIdx.x & 63;
+    const uint32_t xcd = blockIdx.x % kXcds;
+    const uint32_t n_blk = (P.tiles + 63) / 64;
+    const uint32_t n_d = P.n_digits > xcd ? (P.n_digits - xcd + kXcds - 1) / kXcds : 0u;
+    const uint32_t stride = route_stride(P.n_tables);
+    auto take = [&]() {
+        uint32_t x = 0;
+        if (lane == 0) x = atomicAdd(&P.next[xcd * kRouteNextStep], 1u);
+        return x;
+    };
+    uint32_t ahead = take();
+    for (;;) {
+        const uint32_t x = (uint32_t)__builtin_amdgcn_readfirstlane((int)ahead);
+        if (x >= n_d * n_blk) break;
+        ahead = take();
+        const uint32_t d = xcd + kXcds * (x / n_blk), lt0 = x % n_blk * 64;
+        uint32_t t = 0;
+        const uint8_t* base = T.base[0];
+#pragma unroll
+        for (uint32_t i = 1; i < kBinMaxTables; ++i) {
+            if (i < P.n_tables && d >= P.dfirst[i]) {
+                t = i;
+                base = T.base[i];
+            }
+        }
+        uint32_t first = P.dfirst[0];
+#pragma unroll
+        for (uint32_t i = 1; i < kBinMaxTables; ++i)
+            if (i == t) first = P.dfirst[i];
+        const uint8_t* slice = base + ((uint64_t)(d - first) << kRouteShift) / (kBytes ? 1 : 8);
+        const uint32_t lt = lt0 + (uint32_t)lane;
+        uint32_t a = 0, n = 0;
+        if (lt < P.tiles) {
+            a = P.off[(size_t)d * P.tiles + lt];
+            n = P.off[(size_t)(d + 1) * P.tiles + lt] - a;
+        }
+        const uint64_t at = (uint64_t)lt * stride + a;
+        uint32_t to = n;                                  // index in res of the tile's lookups
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(to, o, 64);
+            if (lane >= o) to += y;
+        }
+        to += P.blk[d * n_blk + x % n_blk] - n;
+        if (lt < P.tiles) P.run[(size_t)d * P.tiles + lt] = to;
+        auto answer = [&](uint32_t e) -> uint8_t {
+            const uint32_t bin = e >> kRouteWinBits;
+            if (kBytes) return slice[bin];
+            return (uint8_t)(slice[bin >> 3] >> (bin & 7u) & 1u);
+        };
+#pragma unroll 1
+        for (int r0 = 0; r0 < LPR; r0 += kDeep) {
+            uint64_t from[kDeep];
+            uint32_t len[kDeep], dst[kDeep], e[kDeep][2];
+#pragma unroll
+            for (int q = 0; q < kDeep; ++q) {
+                const int src = (r0 + q) * kAt + lane / LPR;
+                from[q] = (uint64_t)__shfl((unsigned long long)at, src, 64) + (uint32_t)(lane % LPR);
+                const uint32_t len_all = __shfl(n, src, 64);
+                dst[q] = __shfl(to, src, 64) + (uint32_t)(lane % LPR);
+                len[q] = len_all > (uint32_t)(lane % LPR) ? len_all - (uint32_t)(lane % LPR) : 0u;
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (len[q] > (uint32_t)(h * LPR)) e[q][h] = P.ent[from[q] + h * LPR];
+            }
+            uint8_t c[kDeep][2];
+#pragma unroll
+            for (int q = 0; q < kDeep; ++q) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (len[q] > (uint32_t)(h * LPR)) c[q][h] = answer(e[q][h]);
+            }
+#pragma unroll
+            for (int q = 0; q < kDeep; ++q) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (len[q] > (uint32_t)(h * LPR)) P.res[dst[q] + h * LPR] = c[q][h];
+                for (uint32_t i = 2 * LPR; i < len[q]; i += LPR) P.res[dst[q] + i] = answer(P.ent[from[q] + i]);
+            }
+        }
+    }
+}
+
+// Combine pass: counts of a tile's windows, -1 for windows without lookups
+// (N holding, skipped).  kRouteLanes lanes per run; an XCD takes consecutive
+// tiles, whose runs of a digit share lines of res, run and off.
+constexpr int kRouteLanes = 4;
+
+__global__ __launch_bounds__(kBlock) void route_combine_kernel(RoutePlan P, int16_t* counts) {
+    __shared__ uint32_t least[kBinTile];
+    __shared__ uint32_t run[kRouteDigits];
+    __shared__ uint16_t off[kRouteDigits + 1];
+    constexpr uint32_t kNone = 0x100u;
+    const uint32_t stride = route_stride(P.n_tables);
+    const uint32_t per_xcd = (P.tiles + kXcds - 1) / kXcds;
+    const uint32_t sub = threadIdx.x % kRouteLanes;
+    for (uint32_t y = blockIdx.x / kXcds; y < per_xcd; y += gridDim.x / kXcds) {
+        const uint32_t lt = blockIdx.x % kXcds * per_xcd + y;
+        if (lt >= P.tiles) break;                          // uniform
+        const uint64_t k0 = P.tile_k0[lt];
+        const uint32_t n_win = (uint32_t)(P.tile_k0[lt + 1] - k0);
+        for (uint32_t d = threadIdx.x; d <= P.n_digits; d += kBlock) {
+            off[d] = P.off[(size_t)d * P.tiles + lt];
+            if (d < P.n_digits) run[d] = P.run[(size_t)d * P.tiles + lt];
+        }
+        for (uint32_t i = threadIdx.x; i < (uint32_t)kBinTile; i += kBlock) least[i] = kNone;
+        __syncthreads();
+        const uint32_t* ent = P.ent + (size_t)lt * stride;
+#pragma unroll 4
+        for (uint32_t d = threadIdx.x / kRouteLanes; d < P.n_digits; d += kBlock / kRouteLanes) {
+            const uint32_t a = off[d], n = off[d + 1] - a;
+            for (uint32_t i = 4 * sub; i < n; i += 4 * kRouteLanes) {
+                // up to 3 entries past the run are read and left out; both buffers
+                // end in that much room
+                uint32_t e[4], c;
+                __builtin_memcpy(e, ent + a + i, 16);
+                __builtin_memcpy(&c, P.res + run[d] + i, 4);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (i + q < n) atomicMin(&least[e[q] & (kBinTile - 1)], c >> (8 * q) & 0xFFu);
+            }
+        }
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < n_win && i < (uint32_t)kBinTile; i += kBlock) {
+            const uint32_t c = least[i];
+            counts[k0 + i] = c == kNone ? (int16_t)-1 : (int16_t)c;
+        }
+        __syncthreads();
+    }
+}
+
 // ------------------------------------------------------------ batched diginorm
 //
 // DiginormFilter::Filter::filter_sequence (diginorm.hh:105-119) drops a read
@@ -3766,6 +4037,41 @@ void launch_seg_gather(const uint64_t* nb, const uint8_t* mask, const uint64_t* 
     const uint64_t g = (n + 255) / 256;
     seg_gather_kernel<<<(unsigned)(g < 16384 ? (g ? g : 1) : 16384), 256, 0, s>>>(nb, mask, idx, n, out_nb,
                                                                                out_mask);
+}
+
+void launch_route(const Reads& R, const Tables& T, const RoutePlan& P, uint64_t* hashes, int cus, hipStream_t s) {
+    const int g = (int)std::min<int64_t>(std::max<int64_t>(P.tiles, 1), (int64_t)cus * 3);
+    route_kernel<<<g, kRouteBlock, 0, s>>>(R, T, P, hashes);
+}
+
+template <bool kBytes>
+static void launch_gather(const Tables& T, const RoutePlan& P, int grid, hipStream_t s) {
+    // a tile's run of a digit has about n_tables * kBinTile / n_digits lookups
+    if (P.n_digits > 256)
+        route_gather_kernel<kBytes, 16><<<grid, kBlock, 0, s>>>(T, P);
+    else if (P.n_digits > 128)
+        route_gather_kernel<kBytes, 32><<<grid, kBlock, 0, s>>>(T, P);
+    else
+        route_gather_kernel<kBytes, 64><<<grid, kBlock, 0, s>>>(T, P);
+}
+
+uint64_t route_blocks(const RoutePlan& P) { return (uint64_t)P.n_digits * ((P.tiles + 63) / 64); }
+
+void launch_route_count(const RoutePlan& P, hipStream_t s) {
+    route_count_kernel<<<grid_of(route_blocks(P), kBlock / 64, 8192), kBlock, 0, s>>>(P);
+}
+
+void launch_route_gather(const Tables& T, const RoutePlan& P, int cus, hipStream_t s) {
+    const int grid = std::max(1, cus) * 4;           // more drift apart (eight a CU: 102 ms for 20M reads, four 95), fewer wait
+    if (T.kind == kByte)
+        launch_gather<true>(T, P, grid, s);
+    else
+        launch_gather<false>(T, P, grid, s);
+}
+
+void launch_route_combine(const RoutePlan& P, int16_t* counts, int cus, hipStream_t s) {
+    const int64_t g = std::min<int64_t>(P.tiles, (int64_t)cus * 8);
+    route_combine_kernel<<<(unsigned)((g + kXcds - 1) / kXcds * kXcds), kBlock, 0, s>>>(P, counts);
 }
 
 void launch_bin_iq_combine(const BinPlan& P, int16_t* counts, uint64_t* counters, int grid, hipStream_t s) {

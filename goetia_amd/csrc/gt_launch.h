@@ -95,6 +95,13 @@ void launch_solid_reads(const int64_t* off, const int64_t* kmer_off, uint64_t n_
                         uint32_t threshold, float min_prop_solid, uint8_t* passed, hipStream_t s);
 void launch_seg_gather(const uint64_t* nb, const uint8_t* mask, const uint64_t* idx, uint64_t n, uint64_t* out_nb,
                        uint8_t* out_mask, hipStream_t s);
+// Routed query (one sub-batch = kbase of its end, route, count and scan of
+// route_blocks() entries of RoutePlan::blk, gather, combine).
+uint64_t route_blocks(const RoutePlan& P);
+void launch_route_count(const RoutePlan& P, hipStream_t s);
+void launch_route(const Reads& R, const Tables& T, const RoutePlan& P, uint64_t* hashes, int cus, hipStream_t s);
+void launch_route_gather(const Tables& T, const RoutePlan& P, int cus, hipStream_t s);
+void launch_route_combine(const RoutePlan& P, int16_t* counts, int cus, hipStream_t s);
 void launch_bin_iq_combine(const BinPlan& P, int16_t* counts, uint64_t* counters, int grid, hipStream_t s);
 void launch_fill_u8(uint8_t* p, uint64_t n, uint8_t v, hipStream_t s);
 

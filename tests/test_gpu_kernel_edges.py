@@ -227,3 +227,35 @@ def test_binned_insert_in_small_groups(oracle, monkeypatch, kind, max_table, n_r
     for x, y in zip(g.get_raw(), o.tables()):
         np.testing.assert_array_equal(x, y)
     assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+
+
+@pytest.mark.parametrize('kind,sizes', [(1, [97]), (1, [1 << 21, (1 << 21) + 1]), (2, [8191, 8209, 8219, 8221]),
+                                        (2, [(1 << 21) - 1, 1 << 21, (1 << 21) + 1, 5_000_011]),
+                                        (2, [1 << 28, 3, 70_000_001]), (1, [(1 << 30) - 35, 11])])
+@pytest.mark.parametrize('K,mode', [(1, N.MODE_RAW), (31, N.MODE_SKIP_N), (64, N.MODE_RAW), (255, N.MODE_SKIP_N)])
+def test_routed_query_equals_the_direct_one(oracle, monkeypatch, kind, sizes, K, mode):
+    """Slices of one bin to 2^21, digits of 1 to several hundred per table (16,
+    32 and 64 lanes to a run), runs longer than two rounds of their lanes, N
+    bases, gaps, sub-batches, hashes; present and absent windows."""
+    g, o = _pair(oracle, kind, [min(s, 5_000_011) for s in sizes], K, mode=mode)
+    if max(sizes) > 5_000_011:                          # too large for the oracle here: the direct query is its stand-in
+        g, o = _pair(oracle, kind, sizes, K, mode=mode)[0], None
+    fill = _reads(1, [300] * 60, genome=6000)
+    if o is not None:
+        o.insert_reads(fill.seq, fill.offsets, K, True, mode)
+    g.insert_sequences(fill)
+    for seed, lengths in ((1, [K]), (1, [300] * 60), (2, [K + 1, 0, 5000, 3, 2048, 2047, 1, 400])):
+        b = _reads(seed, lengths, genome=6000, n_rate=0.002)
+        hot = np.frombuffer(b'A' * 3000, np.uint8)
+        b = ReadBatch(np.concatenate([b.seq, hot]), np.append(b.offsets, b.n_bases + len(hot)))
+        for sub in ('', '8192'):
+            monkeypatch.setenv('GOETIA_AMD_SUB_BATCH', sub)
+            monkeypatch.setenv('GOETIA_AMD_ROUTED', '0')
+            direct, dh = g.query_sequences(b, with_hashes=True)
+            monkeypatch.setenv('GOETIA_AMD_ROUTED', '1')
+            routed, rh = g.query_sequences(b, with_hashes=True)
+            np.testing.assert_array_equal(routed, direct)
+            np.testing.assert_array_equal(rh, dh)
+            np.testing.assert_array_equal(g.query_sequences(b), direct)
+        if o is not None:
+            np.testing.assert_array_equal(routed, o.query_reads(b.seq, b.offsets, K, True, mode))
