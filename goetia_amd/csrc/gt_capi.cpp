@@ -740,18 +740,18 @@ uint32_t bin_group(uint32_t n_d1, uint64_t tiles) {
     return g;
 }
 
-// Binned sub-batch in start positions, a multiple of kTileMax: even parts of
-// the batch of at most 2^27 for an insert and 2^26 for insert_and_query (a
-// first digit's result bytes are then 1 MB, a quarter of an XCD's L2: 22.0 ms
-// for the replays of 4M reads against 24.1 at 2^27 and 27 at 2^25), or the
-// whole batch when that is at most a quarter over: every sub-batch passes over
-// the tables, and the 16M starts that 1M reads of 150 leave past 2^27 took as
-// long to replay (2.1 ms) as the rest.  GOETIA_AMD_BIN_SUB sets the size (at
-// most 2^29); GOETIA_AMD_SUB_BATCH caps it.
+// Binned sub-batch in start positions, a multiple of kTileMax: 2^27 for an
+// insert and 2^26 for insert_and_query (a first digit's result bytes are then
+// 1 MB, a quarter of an XCD's L2: 22.0 ms for the replays of 4M reads against
+// 24.1 at 2^27 and 27 at 2^25), or the whole batch when that is at most a
+// quarter over: every sub-batch passes over the tables, and the 16M starts
+// that 1M reads of 150 leave past 2^27 took as long to replay (2.1 ms) as the
+// rest.  (Even parts of a large batch cost its scatter 59.1 ms against 56.3
+// for 20M reads: 2^27 starts are a whole number of its rounds.)
+// GOETIA_AMD_BIN_SUB sets the size (at most 2^29); GOETIA_AMD_SUB_BATCH caps it.
 uint64_t bin_sub_batch(uint64_t n_bases, bool iq) {
     const uint64_t most = iq ? 1ULL << 26 : 1ULL << 27;
-    uint64_t sb = n_bases;
-    if (n_bases > most + most / 4) sb = (n_bases + (n_bases + most - 1) / most - 1) / ((n_bases + most - 1) / most);
+    uint64_t sb = n_bases <= most + most / 4 ? n_bases : most;
     if (const char* v = std::getenv("GOETIA_AMD_BIN_SUB")) {
         const unsigned long long x = std::strtoull(v, nullptr, 10);
         if (x) sb = std::min<uint64_t>(x, 1ULL << 29);
@@ -924,6 +924,7 @@ int routed_query_impl(gt_storage* st, Scratch& sc, const Reads& R, int16_t* coun
     P.run = sc.bin_ent2.as<uint32_t>();
     P.blk = sc.bin_cnt2.as<uint32_t>();
     const Tables T = st->tables_view();
+    ProfScope all("query", s);
     for (int64_t b0 = 0; b0 < R.n_bases; b0 += (int64_t)sub) {
         Reads Rs = R;
         Rs.b0 = b0;
