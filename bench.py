@@ -36,15 +36,17 @@ KERNELS = ['bin_hash', 'bin_count', 'bin_route', 'bin_apply', 'bin_new', 'claim'
 # granule per table (twice for a read-modify-write).  The binned passes move
 # 8-byte events, one per table per k-mer: write once when routed, read once
 # by the next pass; the replay also reads and writes each table slice once per
-# sub-batch (2 x 1.07 GB per 2^27 starts, 16 B per k-mer).
-BYTES_PER_KMER = {'claim': 4 * 64, 'apply': 4 * 2 * 64, 'query': 4 * 64,
+# sub-batch (2 x 1.07 GB per 2^27 starts, 16 B per k-mer).  The query of a
+# large batch writes a 4-byte lookup per table and reads it twice, writes and
+# reads a 1-byte answer to each, writes a 2-byte count and reads every table
+# slice once per sub-batch (8 B per k-mer).
+BYTES_PER_KMER = {'claim': 4 * 64, 'apply': 4 * 2 * 64, 'query': 4 * (3 * 4 + 2) + 2 + 8,
                   'bin_hash': 4 * 8, 'bin_count': 4 * 8, 'bin_route': 2 * 4 * 8,
                   'bin_apply': 4 * 8 + 16, 'bin_new': 1}
 # HBM bytes per k-mer (read + write) measured with rocprofv3 FETCH_SIZE /
 # WRITE_SIZE on this workload and scaled by a 1 GiB copy (the table and the
 # commands are in profiles/cms_20m_hbm_traffic.md).
-MEASURED_BYTES_PER_KMER = {'bin_hash': 36.3, 'bin_count': 37.1, 'bin_route': 93.6, 'bin_apply': 64.0, 'bin_new': 1.2,
-                           'query': 515.5}
+MEASURED_BYTES_PER_KMER = {'bin_hash': 36.3, 'bin_count': 37.1, 'bin_route': 93.6, 'bin_apply': 64.0, 'bin_new': 1.2}
 
 
 def log(*a):
@@ -296,7 +298,7 @@ def main():
     cpu = None if args.no_cpu_baseline else cpu_baseline(cfg, batch, args.cpu_sample_reads)
 
     # the query against the measured random-read roofline: one random table
-    # byte per k-mer and table
+    # byte per k-mer and table (above 1 where the reads come out of the L2s)
     if roofline is not None and not args.no_random_access:
         ra = random_access(N, sum(store.table_bytes(i) for i in range(store.n_tables())),
                            sweep=args.random_access_sweep)

@@ -438,7 +438,8 @@ int gt_server_free(gt_server* S);
  * library launches is bracketed by a pair of hipEvents recorded on the
  * kernel's own stream; gt_profile_get synchronizes and returns, for one
  * kernel name ("claim", "apply", "exact_lookup", "exact_insert",
- * "exact_resolve", "query", "hash", "degrees", "seq_insert_query", the binned
+ * "exact_resolve", "query" (a large batch's passes within it: "query_route",
+ * "query_gather", "query_combine"), "hash", "degrees", "seq_insert_query", the binned
  * insert's "bin_hash", "bin_count", "bin_route", "bin_apply", "bin_new",
  * "bin_iq", diginorm's "dn_replay", "dn_decide", "dn_apply"), the number of
  * launches and their summed duration in milliseconds since the last reset. */
