@@ -30,7 +30,8 @@ enum Mode : int { kRaw = 0, kSkipN = 1 };
 // first-touch generation (exact-set stamps): bumped on the device once per
 // sub-batch, so replays of a captured batch never reuse a generation.
 // For the exact set, kNOccupied holds 1 when the last value inserted was
-// already present (its bucket count depends on it), and kLastIns / kLastNew
+// already present (its bucket count depends on it), and kLastIns (for per-hash
+// inserts also kLastNew)
 // the position + 1 of a sub-batch's last inserted and last new window.
 enum Counter : int {
     kNUnique = 0, kNOccupied = 1, kFresh = 2, kErrors = 3, kGen = 4, kLastIns = 5, kLastNew = 6, kNCounters = 7

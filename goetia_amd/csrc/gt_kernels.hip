@@ -6,8 +6,11 @@
 // windows per thread, and hand every window to an operation functor:
 //
 //   Bloom / count-min insert  = claim pass + apply pass (first-touch exact)
-//   exact-set insert          = lookup pass + insert pass + resolve pass
+//   exact-set insert          = one pass (and one more for new flags)
 //   query, degrees            = one read-only pass
+//
+// Large Bloom / count-min batches take the binned insert and the routed query
+// below instead.
 //
 // "First touch": goetia inserts k-mers one at a time in read order, so a
 // k-mer is new iff, for some table, its bin was empty before it
@@ -1896,7 +1899,7 @@ __global__ void exact_keys_kernel(ExactSet E, uint64_t* out, uint64_t cap_out, u
 //
 // Both partitions are stable, so a bucket holds its events in window order.
 // The replay takes 64 events at a time: lanes that hit the same bin are found
-// with one ballot per bin bit, and a lane's rank among them is the number of
+// in LDS and by ballots, and a lane's rank among them is the number of
 // earlier events of the chunk on that bin, so the value the bin held just
 // before the event is (slice value at chunk start) + rank.  That is goetia's
 // sequential insert, event by event (bytestorage.cc:60-113,
