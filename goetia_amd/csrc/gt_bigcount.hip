@@ -224,6 +224,7 @@ struct Tmp {
     int alloc(size_t n) {
         if (hipMalloc(&p, n ? n : 1) != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();       // not the next launch's error
             return set_error(GT_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(n) + " bytes failed");
         }
         return GT_OK;
@@ -242,6 +243,7 @@ int big_alloc(BigMapDev& M, uint64_t cap, hipStream_t s) {
         if (k) (void)hipFree(k);
         if (v) (void)hipFree(v);
         if (p) (void)hipFree(p);
+        (void)hipGetLastError();
         return set_error(GT_ERR_OUT_OF_MEMORY, "bigcount map of " + std::to_string(cap) + " slots");
     }
     M.keys = static_cast<uint64_t*>(k);
@@ -262,8 +264,10 @@ int read_aux(const BigMapDev& M, uint32_t* host, hipStream_t s) {
 int big_init(BigMapDev& M, hipStream_t s) {
     if (M.aux) return GT_OK;
     void* a = nullptr;
-    if (hipMalloc(&a, kBigAux * sizeof(uint32_t)) != hipSuccess)
+    if (hipMalloc(&a, kBigAux * sizeof(uint32_t)) != hipSuccess) {
+        (void)hipGetLastError();
         return set_error(GT_ERR_OUT_OF_MEMORY, "bigcount map counters");
+    }
     M.aux = static_cast<uint32_t*>(a);
     BIG_TRY(hip_check(hipMemsetAsync(M.aux, 0, kBigAux * sizeof(uint32_t), s), "bigcount map counters"));
     return big_alloc(M, 64, s);

@@ -88,6 +88,16 @@ int ensure_device(int device = -1) {
 
 // ------------------------------------------------------------ device buffers
 
+// What hipMalloc is asked for in place of sz bytes: the same, or, past the
+// bytes that GOETIA_AMD_ALLOC_LIMIT names, more than any device has, so that
+// the runtime refuses it as it does on a full one (the tests of what a call
+// does then).
+size_t alloc_request(size_t sz) {
+    const char* v = std::getenv("GOETIA_AMD_ALLOC_LIMIT");
+    if (!v || !*v || sz <= std::strtoull(v, nullptr, 10)) return sz;
+    return (size_t)1 << 60;
+}
+
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
@@ -115,9 +125,12 @@ struct DevBuf {
                                                 std::to_string(bytes) + "-byte fixed scratch region");
         release();
         size_t sz = std::max<size_t>(need, 256);
-        hipError_t e = hipMalloc(&p, sz);
+        hipError_t e = hipMalloc(&p, alloc_request(sz));
         if (e != hipSuccess) {
             p = nullptr;
+            // the runtime keeps the error, and the next launch's check would report
+            // it: a caller that goes another way without the buffer would fail
+            (void)hipGetLastError();
             return fail(GT_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(sz) + " bytes failed: " +
                                                   hipGetErrorString(e));
         }
@@ -223,6 +236,14 @@ struct Scratch {
     DevBuf bin_ent1, bin_ent2, bin_dig2, bin_off1, bin_cnt2, bin_sums, bin_flags, bin_kbase;
     DevBuf bin_res1, bin_win1, bin_tile;   // results per event: result byte, window; per tile and item (res_prepare)
     bool fixed = false;                // buffers preallocated and never moved (captured graphs)
+
+    // Gives back the buffers that grow with a batch's events, for a call that
+    // found no room for all of them and goes on without.
+    void release_events() {
+        for (DevBuf* b : {&bin_ent1, &bin_ent2, &bin_dig2, &bin_off1, &bin_cnt2, &bin_sums, &bin_flags, &bin_res1,
+                          &bin_win1, &bin_tile})
+            b->release();
+    }
 };
 
 // ------------------------------------------------------------ storage
@@ -488,6 +509,7 @@ uint64_t sub_batch_cap() {
 
 // Allocates a claim map of `want` slots (zeroed) with its generation counter.
 int alloc_claims(Scratch& sc, uint64_t want, hipStream_t s) {
+    sc.claim_cap = 0;                  // no map while its buffers move (one of them may not fit)
     GT_TRY(sc.claim_keys.ensure(want * sizeof(uint64_t)));
     GT_TRY(sc.claim_vals.ensure(want * sizeof(uint64_t)));
     GT_TRY(sc.claim_gen.ensure(sizeof(uint64_t)));
@@ -956,8 +978,7 @@ int query_impl(gt_storage* st, Scratch& sc, const Reads& R, int16_t* counts, uin
     if (counts && use_routed(st, sc, R)) {
         const int rc = routed_query_impl(st, sc, R, counts, hashes, s);
         if (rc != GT_ERR_OUT_OF_MEMORY) return rc;
-        sc.bin_ent1.release();          // no room for the lookups: read the tables window by window
-        sc.bin_res1.release();
+        sc.release_events();            // no room for the lookups: read the tables window by window
     }
     ProfScope ps("query", s);
     launch_query(make_launch(st, (uint64_t)R.n_bases, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
@@ -1108,12 +1129,7 @@ int dbg_insert_impl(gt_storage* st, Scratch& sc, Reads R, uint64_t* n_new, uint8
         if (rc != GT_ERR_OUT_OF_MEMORY) return rc;
         // not enough device memory for the event buffers: release them and
         // insert with atomics on the tables instead (same results)
-        sc.bin_ent1.release();
-        sc.bin_ent2.release();
-        sc.bin_dig2.release();
-        sc.bin_flags.release();
-        sc.bin_res1.release();
-        sc.bin_win1.release();
+        sc.release_events();
         GT_TRY(prepare_claims(st, sc, (uint64_t)R.n_bases, &sub, s));
     }
     const Launch L = make_launch(st, std::min<uint64_t>(sub, (uint64_t)R.n_bases), s);
@@ -1854,11 +1870,7 @@ int gt_dbg_insert_and_query_dev(gt_storage* st, uint16_t K, int canonical, int m
         GT_TRY(prepare_reads(st, R, true, s));
         const int rc = binned_insert_impl(st, st->own, R, nullptr, nullptr, counts, s);
         if (rc != GT_ERR_OUT_OF_MEMORY) return rc;
-        st->own.bin_ent1.release();     // no room for the event buffers: strict order below
-        st->own.bin_ent2.release();
-        st->own.bin_dig2.release();
-        st->own.bin_res1.release();
-        st->own.bin_win1.release();
+        st->own.release_events();       // no room for the event buffers: strict order below
     }
     if (st->kind == kByte) {
         // More than four tables or 2^30 bins: hash the batch, then apply it

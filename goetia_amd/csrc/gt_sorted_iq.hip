@@ -132,6 +132,7 @@ struct Buf {
     int alloc(size_t n) {
         if (hipMalloc(&p, n ? n : 1) != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();       // not the next launch's error
             return set_error(GT_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(n) + " bytes failed");
         }
         return GT_OK;

@@ -259,3 +259,49 @@ def test_routed_query_equals_the_direct_one(oracle, monkeypatch, kind, sizes, K,
             np.testing.assert_array_equal(g.query_sequences(b), direct)
         if o is not None:
             np.testing.assert_array_equal(routed, o.query_reads(b.seq, b.offsets, K, True, mode))
+
+
+def _launches(name):
+    """Times a kernel's timer ran since the last reset."""
+    import ctypes as C
+    n, ms = C.c_uint64(), C.c_double()
+    N.call('gt_profile_get', name.encode(), C.byref(n), C.byref(ms))
+    return n.value
+
+
+@pytest.fixture
+def launches():
+    N.call('gt_profile_enable', 1)
+    N.call('gt_profile_reset')
+    yield _launches
+    N.call('gt_profile_enable', 0)
+
+
+@pytest.mark.parametrize('kind', [1, 2])
+def test_calls_without_room_for_their_events(oracle, monkeypatch, launches, kind):
+    """A device that has no room for the event buffers of the binned insert,
+    the routed query and insert_and_query: each goes its other way, with the
+    same results, and the calls after it are not told of the refusal."""
+    K, sizes = 31, [20011, 20021, 20023, 20029]
+    monkeypatch.setenv('GOETIA_AMD_BINNED', '1')
+    monkeypatch.setenv('GOETIA_AMD_ROUTED', '1')
+    g, o = _pair(oracle, kind, sizes, K)
+    b = _reads(3, [150] * 2000, genome=20_000)           # 0.3 MB of reads, 10 MB of events
+    c = _reads(4, [150] * 2000, genome=20_000)
+    monkeypatch.setenv('GOETIA_AMD_ALLOC_LIMIT', str(2 << 20))
+    for batch in (b, c, b):
+        _, e_new = o.insert_reads(batch.seq, batch.offsets, K)
+        np.testing.assert_array_equal(g.insert_sequences(batch), e_new)
+        np.testing.assert_array_equal(g.query_sequences(batch), o.query_reads(batch.seq, batch.offsets, K))
+    if kind == 2:
+        exp = o.insert_and_query_reads(c.seq, c.offsets, K)
+        np.testing.assert_array_equal(g.insert_and_query_sequences(c), exp)
+    assert launches('bin_hash') == 0 and launches('query_route') == 0
+    monkeypatch.delenv('GOETIA_AMD_ALLOC_LIMIT')
+    _, e_new = o.insert_reads(c.seq, c.offsets, K)
+    np.testing.assert_array_equal(g.insert_sequences(c), e_new)
+    np.testing.assert_array_equal(g.query_sequences(c), o.query_reads(c.seq, c.offsets, K))
+    assert launches('bin_hash') > 0 and launches('query_route') > 0
+    for x, y in zip(g.get_raw(), o.tables()):
+        np.testing.assert_array_equal(x, y)
+    assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
