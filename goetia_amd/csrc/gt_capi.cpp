@@ -524,16 +524,30 @@ int alloc_claims(Scratch& sc, uint64_t want, hipStream_t s) {
     return GT_OK;
 }
 
+constexpr uint64_t kMaxClaimCap = 1ULL << 29;      // 8 GiB of claim slots
+constexpr uint64_t kMinClaimCap = 1ULL << 16;
+
 // Bins of a storage whose batches of n_starts starts claim them directly (a
 // stamp word per bin), or 0: when that takes no more memory than the hashed
-// map's slots for the batch, or no more than 2^22 words (goetia's default
-// tables, 4 x 1e6 bins).
+// map's slots for the batch (two words each, never more than kMaxClaimCap), or
+// no more than 2^22 words (goetia's default tables, 4 x 1e6 bins).
 uint64_t direct_claim_bins(const gt_storage* st, const Scratch& sc, uint64_t n_starts) {
     if (sc.fixed || st->kind == kExact) return 0;
     uint64_t bins = 0;
     for (uint64_t p : st->sizes) bins += p;
-    return bins <= std::max<uint64_t>(1ULL << 22, 2 * (uint64_t)st->n_tables * n_starts) && bins < (1ULL << 32) ? bins
-                                                                                                              : 0;
+    const uint64_t most = std::min<uint64_t>(2 * (uint64_t)st->n_tables * n_starts, 2 * kMaxClaimCap);
+    return bins <= std::max<uint64_t>(1ULL << 22, most) ? bins : 0;
+}
+
+// Takes the direct map of `bins` stamps for a call, and the fresh bytes of sb
+// starts; false when they do not fit the device.
+bool take_direct_claims(Scratch& sc, uint64_t bins, uint64_t sb, hipStream_t s) {
+    if (sc.fresh.ensure(sb) != GT_OK) return false;
+    if (sc.claim_direct.bytes < bins * sizeof(uint64_t)) {
+        if (sc.claim_direct.ensure(bins * sizeof(uint64_t)) != GT_OK) return false;
+        launch_fill_u64(sc.claim_direct.as<uint64_t>(), sc.claim_direct.bytes / 8, 0, s);
+    }
+    return true;
 }
 
 // Largest sub-batch (in start positions, a multiple of kTileMax) whose claims fit
@@ -542,28 +556,31 @@ uint64_t direct_claim_bins(const gt_storage* st, const Scratch& sc, uint64_t n_s
 // map the call's claims go to; a direct map's older stamps, of this or other
 // storages' batches on the scratch, are earlier generations.
 int prepare_claims(gt_storage* st, Scratch& sc, uint64_t n_starts, uint64_t* sub, hipStream_t s) {
-    const uint64_t kMaxClaimCap = 1ULL << 29;      // 8 GiB of claim slots
-    const uint64_t kMinClaimCap = 1ULL << 16;
     const uint64_t per = std::max<uint32_t>(st->n_tables, 1);
     const uint64_t cap = sub_batch_cap();
     const uint64_t starts = (n_starts + kTileMax - 1) / kTileMax * kTileMax;
-    const uint64_t direct = direct_claim_bins(st, sc, n_starts);
-    sc.direct = direct != 0;
-    if (st->kind == kExact || direct) {
+    sc.direct = false;
+    if (st->kind == kExact) {
         uint64_t sb = std::min<uint64_t>(starts, 1ULL << 31);
         if (cap) sb = std::min(sb, cap);
         if (sb == 0) return fail(GT_ERR_INTERNAL, "scratch too small");
         if (!sc.claim_cap) GT_TRY(alloc_claims(sc, 2, s));   // the generation counter, and a valid view
-        if (direct) {
-            GT_TRY(sc.fresh.ensure(sb));
-            if (sc.claim_direct.bytes < direct * sizeof(uint64_t)) {
-                GT_TRY(sc.claim_direct.ensure(direct * sizeof(uint64_t)));
-                launch_fill_u64(sc.claim_direct.as<uint64_t>(), sc.claim_direct.bytes / 8, 0, s);
-                GT_HIP(hipGetLastError());
-            }
-        }
         *sub = sb;
         return GT_OK;
+    }
+    if (const uint64_t bins = direct_claim_bins(st, sc, n_starts)) {
+        // sub-batches as large as the hashed map's at its cap
+        uint64_t sb = std::min<uint64_t>(starts, kMaxClaimCap / (2 * per) / kTileMax * kTileMax);
+        if (cap) sb = std::min(sb, cap);
+        if (sb == 0) return fail(GT_ERR_INTERNAL, "scratch too small");
+        if (!sc.claim_cap) GT_TRY(alloc_claims(sc, 2, s));   // the generation counter
+        if (take_direct_claims(sc, bins, sb, s)) {
+            GT_HIP(hipGetLastError());
+            sc.direct = true;
+            *sub = sb;
+            return GT_OK;
+        }
+        sc.claim_direct.release();     // no room for it: the hashed map takes the batch
     }
     uint64_t want = std::min(kMaxClaimCap, std::max(kMinClaimCap, next_pow2(2 * per * (n_starts + kTileMax))));
     if (want > sc.claim_cap && !sc.fixed) GT_TRY(alloc_claims(sc, want, s));

@@ -305,3 +305,53 @@ def test_calls_without_room_for_their_events(oracle, monkeypatch, launches, kind
     for x, y in zip(g.get_raw(), o.tables()):
         np.testing.assert_array_equal(x, y)
     assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+
+
+@pytest.mark.parametrize('kind', [1, 2])
+def test_claims_without_room_for_a_stamp_per_bin(oracle, monkeypatch, kind):
+    """Small tables claim directly, a stamp per bin (8 MB here); without room
+    for that the hashed map (1 MB) takes the same batches."""
+    monkeypatch.setenv('GOETIA_AMD_BINNED', '0')
+    K, sizes = 31, [250_007, 250_013, 250_027, 250_031]
+    g, o = _pair(oracle, kind, sizes, K)
+    for step, limit in enumerate(('', str(4 << 20), str(4 << 20), '')):
+        monkeypatch.setenv('GOETIA_AMD_ALLOC_LIMIT', limit)
+        if step == 1:                                     # (a storage that took the direct map keeps it)
+            g, o = _pair(oracle, kind, sizes, K)
+        b = _reads(step, [150] * 120, genome=9000)
+        _, e_new, e_flags = o.insert_reads_flags(b.seq, b.offsets, K, True, N.MODE_RAW)
+        n_new, flags = g.insert_sequences(b, new_flags=True)
+        np.testing.assert_array_equal(n_new, e_new)
+        np.testing.assert_array_equal(flags, np.asarray(e_flags, bool))
+        assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+
+
+@pytest.mark.parametrize('n_tables,table,n_bases', [(4, (1 << 30) - 35, (1 << 29) + 12_345),
+                                                    (5, 1 << 28, (1 << 28) + 12_345)])
+def test_claims_of_a_large_batch_stay_within_the_hashed_maps_memory(n_tables, table, n_bases):
+    """Nearly 2^32 bins, and 1.3e9 in five tables, under a batch with more
+    starts than a claim map's cap has room for: sub-batches, and 8 GiB of
+    claims at most (a stamp for each of those bins is 10 to 32 GiB)."""
+    import torch
+    K, L = 31, 150
+    n = (n_bases + L - 1) // L
+    gen = torch.Generator(device='cuda')
+    gen.manual_seed(1)
+    seq = torch.tensor(list(b'ACGT'), dtype=torch.uint8, device='cuda')
+    seq = seq[torch.randint(0, 4, (n_bases,), generator=gen, device='cuda', dtype=torch.uint8).to(torch.int32)]
+    off = torch.clamp(torch.arange(n + 1, device='cuda', dtype=torch.int64) * L, max=n_bases)
+    from goetia_amd.reads import DeviceReads
+    d = DeviceReads(seq, off, n_bases)
+    n_new = torch.zeros(n, dtype=torch.int64, device='cuda')
+    g = lg.dBG[lg.BitStorage, lg.CanLemireShifter].build(lg.BitStorage([table - 2 * i for i in range(n_tables)]), K)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    g.insert_device(d, n_new=n_new)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= 9 << 30
+    first = int(n_new.sum())
+    windows = (n_bases // L) * (L - K + 1) + max(0, n_bases % L - K + 1)
+    assert 0.97 * windows < first <= windows and first == g.n_unique()
+    g.insert_device(d, n_new=n_new)
+    assert int(n_new.sum()) == 0 and g.n_unique() == first
