@@ -671,21 +671,40 @@ Launch make_launch(int kind, hipStream_t s) {
 Launch make_launch(hipStream_t s) { return make_launch(0, s); }
 Launch make_launch(const gt_storage* st, hipStream_t s) { return make_launch(st->kind, s); }
 
-// Launch of a walk over n_starts start positions.  Below kSmallStarts the
-// tuned tile shape leaves CUs without waves to hide a window's chain of table
-// accesses behind, so a thread takes four windows together instead (the
-// kernels' kPerSmall form): 500 reads into a 4 x 1e6 Bloom filter went from
-// 365 to 93 us (with direct claims), 4167 reads against 4 x 2^28 counts from
-// 86 to 58 us.
-constexpr uint64_t kSmallStarts = 1ULL << 22;
-Launch make_launch(const gt_storage* st, uint64_t n_starts, hipStream_t s) {
+// Launch of a walk over n_starts start positions, of which `few` are too few
+// for the tuned tile shape: it leaves CUs without waves to hide a window's
+// chain of table accesses behind, so a thread takes four windows together
+// instead (the kernels' kPerSmall form).
+Launch make_launch(const gt_storage* st, uint64_t n_starts, uint64_t few, hipStream_t s) {
     Launch L = make_launch(st->kind, s);
-    if (n_starts < kSmallStarts) {
+    if (n_starts < few) {
         L.per = 4;
         L.grid = std::max(1, g_dev.cus * 8);
     }
     return L;
 }
+
+// Queries, and all passes over an exact set: below 2^22 starts.  4167 reads of
+// 150 against 4 x 2^28 counts take 58 us together and 86 window by window,
+// 27000 take 270 and 285.
+constexpr uint64_t kFewStarts = 1ULL << 22;
+
+// Atomic inserts into Bloom / count-min tables: below 393,216 starts.  Their
+// claims and updates of four tables at a time take 248 registers, two
+// workgroups a CU, so 512 of 1024 starts are on the device at once and a batch
+// of more of them waits for its second round.  Inserts of 150-base reads into
+// an empty / a filled graph, us (together, window by window):
+//   4 x 2^30 bits       500 reads  186 /  59,  422 / 133
+//                      2500        330 / 117,  414 / 132
+//                      3500        496 / 178,  420 / 146
+//                     20000       2087 / 805, 1145 / 601
+//   6 x 2e7 counts     2500        483 / 241,  520 / 249
+//                      3500        811 / 351,  525 / 244
+//   5 x 1e6 counts     2500        416 / 233,  453 / 232   (claimed directly from 3400 on)
+//                      3500        488 / 347,  304 / 238
+//  16 x 2^28 counts    2500       1326 / 587, 1886 / 622
+//                      3500       2077 / 915, 1852 / 671
+constexpr uint64_t kFewInserts = 3ULL << 17;
 
 // Device work of one first-touch sub-batch [Rs.b0, Rs.b1) with the given
 // claim map and fresh buffer.  For the exact set, `growth` allows a
@@ -998,7 +1017,7 @@ int query_impl(gt_storage* st, Scratch& sc, const Reads& R, int16_t* counts, uin
         sc.release_events();            // no room for the lookups: read the tables window by window
     }
     ProfScope ps("query", s);
-    launch_query(make_launch(st, (uint64_t)R.n_bases, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
+    launch_query(make_launch(st, (uint64_t)R.n_bases, kFewStarts, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
     GT_HIP(hipGetLastError());
     return GT_OK;
 }
@@ -1149,7 +1168,8 @@ int dbg_insert_impl(gt_storage* st, Scratch& sc, Reads R, uint64_t* n_new, uint8
         sc.release_events();
         GT_TRY(prepare_claims(st, sc, (uint64_t)R.n_bases, &sub, s));
     }
-    const Launch L = make_launch(st, std::min<uint64_t>(sub, (uint64_t)R.n_bases), s);
+    const Launch L = make_launch(st, std::min<uint64_t>(sub, (uint64_t)R.n_bases),
+                                 st->kind == kExact ? kFewStarts : kFewInserts, s);
     for (int64_t b0 = 0; b0 < R.n_bases; b0 += (int64_t)sub) {
         Reads Rs = R;
         Rs.b0 = b0;

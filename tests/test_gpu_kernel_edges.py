@@ -355,3 +355,31 @@ def test_claims_of_a_large_batch_stay_within_the_hashed_maps_memory(n_tables, ta
     assert 0.97 * windows < first <= windows and first == g.n_unique()
     g.insert_device(d, n_new=n_new)
     assert int(n_new.sum()) == 0 and g.n_unique() == first
+
+
+@pytest.mark.parametrize('kind,n_tables,table', [(1, 4, 1_050_000), (2, 4, 1_050_000), (1, 9, 470_000),
+                                                 (2, 9, 470_000), (2, 5, 4_000_000), (1, 5, 3000)])
+@pytest.mark.parametrize('n_bases', [40_000, 131_071, 393_215, 393_216, 524_289, (1 << 22) - 1, 1 << 22])
+def test_atomic_inserts_at_every_shape_of_launch(oracle, monkeypatch, kind, n_tables, table, n_bases):
+    """Either side of the sizes where the atomic insert and the query change
+    their shape (one wave to a workgroup, four windows of a thread together,
+    window by window), over bins that are claimed by hash (more than 2^22, and
+    than the batch's own limit) and directly (3000 each, and past the limit);
+    more than four and more than eight tables.  Hot k-mers claim one bin from
+    many windows, and the second batch meets slots of the first one's keys."""
+    monkeypatch.setenv('GOETIA_AMD_BINNED', '0')
+    K, sizes = 31, oracle.primes_near_x(n_tables, table)
+    g, o = _pair(oracle, kind, sizes, K)
+    hot = np.frombuffer(b'A' * 100 + b'ACAC' * 50, np.uint8)
+    for seed in (1, 2):
+        n, tail = divmod(n_bases - len(hot), 150)
+        b = _reads(seed, [150] * n + [tail], genome=max(3000, n_bases // 12), sub=0.01)
+        b = ReadBatch(np.concatenate([b.seq, hot]), np.append(b.offsets, n_bases))
+        _, e_new, e_flags = o.insert_reads_flags(b.seq, b.offsets, K, True, N.MODE_RAW)
+        n_new, flags = g.insert_sequences(b, new_flags=True)
+        np.testing.assert_array_equal(n_new, e_new)
+        np.testing.assert_array_equal(flags, np.asarray(e_flags, bool))
+        np.testing.assert_array_equal(g.query_sequences(b), o.query_reads(b.seq, b.offsets, K))
+    assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+    for x, y in zip(g.get_raw(), o.tables()):
+        np.testing.assert_array_equal(x, y)
