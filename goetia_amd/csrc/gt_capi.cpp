@@ -772,22 +772,44 @@ uint32_t bin_buckets(const gt_storage* st) {
     return nb <= kMaxBuckets ? (uint32_t)nb : 0;
 }
 
+// Most buckets of n_tables tables whose small batches are inserted binned
+// (n_tables x at most 2^23 to 2^25 bins).
+uint32_t bin_small_buckets(uint32_t n_tables) {
+    constexpr uint32_t most[kBinMaxTables + 1] = {0, 1024, 2048, 6144, 16384};
+    return n_tables <= kBinMaxTables ? most[n_tables] : 0;
+}
+
 // Whether an insert goes through the binned path.  GOETIA_AMD_BINNED=0 / 1
-// forces it off / on (where the tables allow it); by default it is used from
-// 2^14 bases plus 5 per bucket on, about where the two paths cross: it passes
-// over every bucket that has an event (up to 6 ns each), and the atomic insert
-// takes 0.3 to 0.9 ns more per base.  Reset and insert of 150-base reads, us
-// (atomic / binned):
-//   4 x 1e6 bits       500 reads  101 /   75    2000 reads  170 /   95
-//   4 x 3e7 counts     500 reads  240 /  165    2000 reads  401 /  178
-//   4 x 2^28 bits     2000 reads  374 /  566    6000 reads  878 /  594
-//   4 x 2^28 counts   2000 reads  622 /  964    6000 reads 1178 / 1024
+// forces it off / on (where the tables allow it).  The binned insert passes
+// over every bucket that has an event, up to 6 ns each, whatever the bins
+// hold; the atomic one takes 0.3 to 0.9 ns more per base, and on a graph that
+// already holds most of a batch's k-mers, as it does for most of a sample,
+// about half of that.  So by default a batch of 2^20 bases and one per 256
+// bins is binned (4 x 2^28 counts: 28000 reads), where the two meet on a filled
+// graph, and on few buckets (bin_small_buckets) a batch from 2^14 bases plus 5
+// per bucket on: there the passes cost no more than the atomic insert's
+// shortest time.  Inserts of 150-base reads into an empty / a filled graph, us
+// (atomic, binned):
+//   4 x 1e6 bits       500 reads   365 / 123,    60 /   60
+//   4 x 2^25 bits     2000         336 / 131,   138 /  135
+//                     3500         316 / 145,   156 /  150
+//   4 x 2^26 bits     2000         332 / 131,   192 /  192   (and 300 / 109 by windows together)
+//   2 x 2^24 bits     3500         190 /  95,   111 /  106
+//   1 x 2^25 counts   4500         150 /  95,   118 /  114
+//   4 x 2^28 counts   6000         557 / 235,   815 /  796
+//                    20000        1286 / 654,   970 /  918
+//                    28000        1777 / 829,  1049 /  987
+//   4 x 2^28 bits     6000         375 / 204,   561 /  551
 bool use_binned(const gt_storage* st, const Scratch& sc, const Reads& R) {
     const uint32_t buckets = bin_buckets(st);
     if (R.dyn || sc.fixed || !buckets) return false;
     const char* v = std::getenv("GOETIA_AMD_BINNED");
     if (v && *v) return v[0] != '0';
-    return (uint64_t)R.n_bases >= (1ULL << 14) + 5 * (uint64_t)buckets;
+    const uint64_t n_bases = (uint64_t)R.n_bases;
+    if (buckets <= bin_small_buckets(st->n_tables) && n_bases >= (1ULL << 14) + 5 * (uint64_t)buckets) return true;
+    uint64_t bins = 0;
+    for (uint64_t p : st->sizes) bins += p;
+    return n_bases >= (1ULL << 20) && n_bases * 256 >= bins;
 }
 
 // First-pass tiles per second-pass work item: kBinGroup, or fewer when that

@@ -383,3 +383,17 @@ def test_atomic_inserts_at_every_shape_of_launch(oracle, monkeypatch, kind, n_ta
     assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
     for x, y in zip(g.get_raw(), o.tables()):
         np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize('kind,n_tables,table,n_reads,binned', [
+    (1, 4, 1_000_000, 100, False), (1, 4, 1_000_000, 300, True), (2, 4, 1 << 25, 1000, True),
+    (1, 4, 1 << 26, 6900, False), (1, 4, 1 << 26, 7000, True), (2, 2, 1 << 24, 3000, False),
+    (2, 1, 1 << 25, 3000, False), (2, 1, 1 << 25, 7000, True), (2, 4, 1 << 28, 6000, False),
+    (2, 4, 1 << 28, 27_900, False), (2, 4, 1 << 28, 28_000, True), (2, 1, 1 << 28, 3000, False)])
+def test_batches_are_binned_where_that_is_the_faster_insert(oracle, launches, kind, n_tables, table, n_reads, binned):
+    """Which insert a batch takes by itself, on both sides of its lines."""
+    sizes = [table - 2 * i for i in range(n_tables)]
+    g = _pair(oracle, kind, sizes, 31)[0]
+    b = _reads(1, [150] * n_reads, genome=20_000)
+    assert int(g.insert_sequences(b).sum()) == g.n_unique()
+    assert (launches('bin_hash') > 0) == binned and (launches('claim') > 0) != binned
