@@ -738,7 +738,7 @@ int enqueue_subbatch(gt_storage* st, Scratch& sc, const Launch& L, const Reads& 
         const ExactSet E = st->exact_view();
         {
             ProfScope ps("exact_insert", s);
-            launch_exact_add(L, Rs, E, n_new, ctr);
+            launch_exact_add(L, Rs, E, n_new, new_flags, ctr);
         }
         if (new_flags) {
             ProfScope ps("exact_resolve", s);

@@ -397,3 +397,27 @@ def test_batches_are_binned_where_that_is_the_faster_insert(oracle, launches, ki
     b = _reads(1, [150] * n_reads, genome=20_000)
     assert int(g.insert_sequences(b).sum()) == g.n_unique()
     assert (launches('bin_hash') > 0) == binned and (launches('claim') > 0) != binned
+
+
+@pytest.mark.parametrize('lengths', [[9000] * 12, [150] * 4000, [31] * 3000 + [4500] * 3, [40, 31, 2000, 33] * 200])
+@pytest.mark.parametrize('K,mode,sub', [(31, N.MODE_RAW, ''), (31, N.MODE_SKIP_N, '8192'), (4, N.MODE_SKIP_N, ''),
+                                        (255, N.MODE_RAW, '')])
+def test_exact_set_newness_among_overlapping_reads(oracle, monkeypatch, lengths, K, mode, sub):
+    """Reads that cover their genome many times, so that a window's newness
+    moves between reads, runs of windows to one read and to many: long reads,
+    reads of one window, several sub-batches; n_new alone and with flags, on an
+    empty set, a filled one and one that holds half of the keys."""
+    monkeypatch.setenv('GOETIA_AMD_SUB_BATCH', sub)
+    for seed in (1, 2):
+        g, o = _pair(oracle, 3, (), K, mode=mode)
+        for step in (1, 1, 2):
+            b = _reads(10 * seed + step, lengths, genome=12_000 if step == 1 else 20_000, sub=0.004, n_rate=0.001)
+            _, e_new, e_flags = o.insert_reads_flags(b.seq, b.offsets, K, True, mode)
+            if seed == 1:
+                n_new, flags = g.insert_sequences(b, new_flags=True)
+                np.testing.assert_array_equal(flags, np.asarray(e_flags, bool))
+            else:
+                n_new = g.insert_sequences(b)
+            np.testing.assert_array_equal(n_new, e_new)
+            assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+        np.testing.assert_array_equal(g.S.keys(), np.sort(o.exact_keys()))
