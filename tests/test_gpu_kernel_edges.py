@@ -421,3 +421,21 @@ def test_exact_set_newness_among_overlapping_reads(oracle, monkeypatch, lengths,
             np.testing.assert_array_equal(n_new, e_new)
             assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
         np.testing.assert_array_equal(g.S.keys(), np.sort(o.exact_keys()))
+
+
+def test_exact_set_looks_its_windows_up_only_before_it_may_grow(oracle, launches):
+    """Batches that fit the set whatever they hold are inserted in one pass,
+    however often they come; one that may not is looked up first."""
+    K = 31
+    store = lg.SparseppSetStorage.build(capacity_hint=60_000)       # 131072 slots
+    g, o = lg.dBG[lg.SparseppSetStorage, lg.CanLemireShifter].build(store, K), oracle.Storage(3, ())
+    b = _reads(1, [150] * 250, genome=15_000, sub=0.0)
+    for _ in range(6):
+        _, e_new = o.insert_reads(b.seq, b.offsets, K)
+        np.testing.assert_array_equal(g.insert_sequences(b), e_new)
+    assert launches('exact_insert') == 6 and launches('exact_lookup') == 0
+    b = _reads(2, [150] * 400, genome=15_000)
+    _, e_new = o.insert_reads(b.seq, b.offsets, K)
+    np.testing.assert_array_equal(g.insert_sequences(b), e_new)
+    assert launches('exact_lookup') == 1
+    assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
