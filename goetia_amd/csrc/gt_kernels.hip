@@ -55,9 +55,9 @@ __device__ __forceinline__ uint64_t wave_sum(uint64_t v) {
 // Adds a per-thread count to a device counter with one atomic per workgroup:
 // every thread of a workgroup of at most 512 threads calls it.  Atomics on one
 // address complete one after another, about 12 ns each: with one per wave the
-// 65536 waves of bin_iq_combine_kernel spent 803 us on 60M windows.
-__device__ __forceinline__ void add_counter(uint64_t* ctr, uint64_t v) {
-    __shared__ uint64_t part[8];
+// 65536 waves of bin_iq_combine_kernel spent 803 us on 60M windows.  part: 8
+// words of LDS that no thread uses from here on.
+__device__ __forceinline__ void add_counter(uint64_t* ctr, uint64_t v, uint64_t* part) {
     v = wave_sum(v);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -67,6 +67,11 @@ __device__ __forceinline__ void add_counter(uint64_t* ctr, uint64_t v) {
         if (sum) atomicAdd((unsigned long long*)ctr, (unsigned long long)sum);
     }
     __syncthreads();                                      // part may be used again
+}
+
+__device__ __forceinline__ void add_counter(uint64_t* ctr, uint64_t v) {
+    __shared__ uint64_t part[8];
+    add_counter(ctr, v, part);
 }
 
 __device__ __forceinline__ uint64_t wave_max(uint64_t v) {
@@ -2730,7 +2735,10 @@ __device__ __forceinline__ uint32_t* bin_stage_slice(const BinPlan& P, const Tab
 }
 
 // Replay: one wavefront per bucket (four per workgroup).  Masked: only the
-// events of kept reads before P.r_end take part (batched diginorm).
+// events of kept reads before P.r_end take part (batched diginorm).  The
+// slices and match slots are 40960 bytes of LDS, so that four workgroups fit a
+// CU; the counters are summed in the slots (8 words more, and three fit: 446 us
+// instead of 377 for 500 reads over 4 x 2^28 counts).
 //
 // insert_and_query's result bytes go to res1, where a first digit's events
 // are one dense range (2 MB per 2^27 starts), and the workgroups of one XCD
@@ -2850,7 +2858,8 @@ __device__ __forceinline__ void bin_apply_body(const BinPlan& P, const Tables& T
         for (uint32_t w = lane; w < nw; w += 64) __builtin_nontemporal_store(sw[w], src + w);
         __builtin_amdgcn_wave_barrier();
     }
-    add_counter(counters + kNOccupied, occ);
+    __syncthreads();                                      // the match slots are free
+    add_counter(counters + kNOccupied, occ, slots[0]);
 }
 
 __global__ __launch_bounds__(kBlock) void bin_apply_kernel(BinPlan P, Tables T, uint64_t* counters) {
