@@ -830,17 +830,23 @@ uint32_t bin_group(uint32_t n_d1, uint64_t tiles) {
 }
 
 // Binned sub-batch in start positions, a multiple of kTileMax: 2^27 for an
-// insert and 2^26 for insert_and_query (a first digit's result bytes are then
-// 1 MB, a quarter of an XCD's L2: 22.0 ms for the replays of 4M reads against
-// 24.1 at 2^27 and 27 at 2^25), or the whole batch when that is at most a
-// quarter over: every sub-batch passes over the tables, and the 16M starts
-// that 1M reads of 150 leave past 2^27 took as long to replay (2.1 ms) as the
-// rest.  (Even parts of a large batch cost its scatter 59.1 ms against 56.3
-// for 20M reads: 2^27 starts are a whole number of its rounds.)
+// insert or a query and 2^26 for insert_and_query (a first digit's result bytes
+// are then 1 MB, a quarter of an XCD's L2: 4M reads take 55.3 ms, 59.4 at 2^27
+// and 55.0 at 2^25), or the whole batch when that is at most a quarter over, or
+// a fifth for insert_and_query: every sub-batch passes over the tables, however
+// few events it has.  A batch of x times that many starts against 4 x 2^28
+// counts (whole, in two parts), ms:
+//   x                  1.1            1.2           1.25            1.3            1.5
+//   insert         7.99, 8.61    8.68, 9.18    8.83, 9.49     9.29, 9.87   10.68, 11.10
+//   query          6.86, 7.18    7.47, 7.85    7.77, 8.11     8.11, 8.43    9.43,  9.60
+//   ins. and query 7.35, 7.50    8.03, 8.04    8.32, 8.26     8.79, 8.57   10.24,  9.64
+// (An insert or a query could go to 1.5 at 11 GiB of events for 1.25.  Even
+// parts of a large batch cost its scatter 59.1 ms against 56.3 for 20M reads:
+// 2^27 starts are a whole number of its rounds.)
 // GOETIA_AMD_BIN_SUB sets the size (at most 2^29); GOETIA_AMD_SUB_BATCH caps it.
 uint64_t bin_sub_batch(uint64_t n_bases, bool iq) {
     const uint64_t most = iq ? 1ULL << 26 : 1ULL << 27;
-    uint64_t sb = n_bases <= most + most / 4 ? n_bases : most;
+    uint64_t sb = n_bases <= most + most / (iq ? 5 : 4) ? n_bases : most;
     if (const char* v = std::getenv("GOETIA_AMD_BIN_SUB")) {
         const unsigned long long x = std::strtoull(v, nullptr, 10);
         if (x) sb = std::min<uint64_t>(x, 1ULL << 29);

@@ -2748,7 +2748,7 @@ __device__ __forceinline__ uint32_t* bin_stage_slice(const BinPlan& P, const Tab
 // has no second use there (events, table slices) goes past it.  Writing each
 // byte to its window's place took 3.56 ms per 2^26 starts, of which 1.5 is the
 // replay without results; to its place in the tile's region (32 bytes per tile
-// and digit) 4.6, since the lines of a digit then span 8 MB; this takes 2.44.
+// and digit) 4.6, since the lines of a digit then span 8 MB; this takes 2.3.
 template <bool kMasked>
 __device__ __forceinline__ void bin_apply_body(const BinPlan& P, const Tables& T, uint64_t* counters,
                                                uint32_t (*slice)[kBucketBins / 4], uint64_t (*slots)[256]) {
