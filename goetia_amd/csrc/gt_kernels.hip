@@ -2682,7 +2682,8 @@ __device__ __forceinline__ uint64_t bin_match(uint64_t* slots, uint32_t key, boo
 // Whether two active lanes of the wavefront are on one bin of a slice of byte
 // counts; *pre gets each active lane's count.  Every active lane writes its
 // number over its count and reads it back, so the caller has to write each
-// active bin again.  64 random events of kBucketBins bins share none 78 times
+// active bin again.  (Another lane may have written the bin since: the lane's
+// own store must not stand in for the load, hence the atomic one.)  64 random events of kBucketBins bins share none 78 times
 // of 100, and then need no ranking: three LDS accesses in a row in place of
 // bin_match's three and its ballots.
 __device__ __forceinline__ bool bins_shared(uint8_t* sb, uint32_t key, bool active, uint32_t* pre) {
@@ -2692,7 +2693,7 @@ __device__ __forceinline__ bool bins_shared(uint8_t* sb, uint32_t key, bool acti
     __builtin_amdgcn_wave_barrier();
     if (active) sb[key] = (uint8_t)lane;
     __builtin_amdgcn_wave_barrier();
-    if (active) back = sb[key];
+    if (active) back = __hip_atomic_load(&sb[key], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
     __builtin_amdgcn_wave_barrier();
     *pre = p;
     return __ballot(back != lane) != 0;
