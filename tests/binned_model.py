@@ -4,11 +4,13 @@ Restates, step by step and with the kernels' own index arithmetic, what one
 binned call does: the plan (buckets of 8192 bins, first / second digits), the
 first pass (per 2048-start tile: events table-major, stable per-wave ranking
 by first digit, region writes and the 257-entry digit-offset row), the
-second-pass count and scan, the second-pass scatter (work items of 1024 tiles,
-chunks of 4096 events, per-digit runs written from the chunk's sorted order),
-the per-bucket replay with ranks inside 64-event chunks, and the per-read sum
-of new flags or the insert_and_query minimum.  Every buffer index is asserted
-against the buffer's size, so a plan or offset mistake fails here on the CPU.
+second-pass count and scan, the second-pass scatter (work items of 64 to 1024
+tiles, chunks of 4096 events, per-digit runs written from the chunk's sorted
+order), the per-bucket replay with ranks inside 64-event chunks, and the
+per-read sum of new flags, or insert_and_query's result byte per event and the
+minimum that its combine pass takes of a tile's runs of them.  Every buffer
+index is asserted against the buffer's size, so a plan or offset mistake fails
+here on the CPU.
 
 Test infrastructure: the hashes come from the oracle (oracle/pyoracle.py).
 """
@@ -21,6 +23,7 @@ DIGIT_BITS1, DIGITS1, DIGITS2 = 8, 256, 512
 BIN_TILE, BIN_GROUP, BIN_CHUNK, TILE_MAX = 2048, 1024, 4096, 8192
 MAX_TABLES, MAX_BUCKETS = 4, 1 << 17
 NO_BIN = 0xFFFFFFFF
+CUS = 256
 
 
 def _rank_chunk(keys):
@@ -61,6 +64,14 @@ def _windows(seq, off, K, mode):
     return wins, kmer_off, hv, valid
 
 
+def bin_group(n_d1, tiles):
+    """First-pass tiles per second-pass work item."""
+    g = BIN_GROUP
+    while g > 64 and n_d1 * ((tiles + g - 1) // g) < 4 * CUS:
+        g //= 2
+    return g
+
+
 def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
     """Tables (4-byte padded), per-read n_new, n_unique, n_occupied, and the
     insert_and_query counts when iq."""
@@ -86,7 +97,8 @@ def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
     sub = max((sub + TILE_MAX - 1) // TILE_MAX * TILE_MAX, TILE_MAX)
     sub = min(sub, (n_bases + TILE_MAX - 1) // TILE_MAX * TILE_MAX)
     tiles_max = sub // BIN_TILE
-    groups_max = (tiles_max + BIN_GROUP - 1) // BIN_GROUP
+    group = bin_group(n_d1, tiles_max)
+    groups_max = (tiles_max + group - 1) // group
     n_ent = tiles_max * nt * BIN_TILE
     cnt_max = (n_d1 << shift2) * groups_max
     if kind == po.BYTE:
@@ -94,20 +106,33 @@ def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
     else:
         tabs = [np.zeros((p // 8 + 1 + 3) // 4 * 4, np.uint8) for p in sizes]
     flags = np.zeros(n_bases, np.uint8)
-    vq = np.zeros((max(n_bases, 1), MAX_TABLES), np.uint8)
+    counts = np.full(nk, -2, np.int16)
     occ = 0
     for b0 in range(0, n_bases, sub):
         b1 = min(n_bases, b0 + sub)
         tile0 = b0 // BIN_TILE
         tiles1 = (b1 - b0 + BIN_TILE - 1) // BIN_TILE
-        n_groups = (tiles1 + BIN_GROUP - 1) // BIN_GROUP
-        r = int(np.searchsorted(off, b0, side='right') - 1)
-        kbase = int(kmer_off[r] + min(max(b0 - off[r], 0), wins[r]))
+        n_groups = (tiles1 + group - 1) // group
+
+        def first_window(x):
+            """Packed index of the first window starting at or after base x."""
+            r = min(int(np.searchsorted(off, x, side='right') - 1), n_reads - 1)
+            return int(kmer_off[r] + min(max(x - off[r], 0), wins[r]))
+
+        kbase = first_window(b0)
+        tile_k0 = np.full(tiles_max + 1, -1, np.int64)
+        tile_k0[tiles1] = first_window(b1)
+        win1 = np.full(n_ent, -1, np.int64)
+        off1t = np.full(tiles_max * DIGITS1, -1, np.int64)
+        run1 = np.full(tiles_max * DIGITS1, -1, np.int64)
+        item_n = np.full(DIGITS1 * groups_max, -1, np.int64)
+        res1 = np.full(n_ent, -1, np.int64)
         ent1 = np.full(n_ent, -1, np.int64)
         off1 = np.zeros((DIGITS1 + 1) * tiles_max, np.int64)
         # first pass
         for lt1 in range(tiles1):
             t0 = (tile0 + lt1) * BIN_TILE
+            tile_k0[lt1] = first_window(t0)
             g = np.full(MAX_TABLES * BIN_TILE, NO_BIN, np.int64)
             ordv = np.zeros(BIN_TILE, np.int64)
             for w in range(BIN_TILE):
@@ -137,6 +162,7 @@ def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
             for d in range(DIGITS1):
                 assert start[d] <= 0xFFFF
                 off1[d * tiles1 + lt1] = start[d]
+                off1t[lt1 * DIGITS1 + d] = start[d]
                 p = start[d]
                 for wave in range(4):
                     c = wpos[wave][d]
@@ -162,11 +188,14 @@ def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
                 e = int(perm[i])
                 assert base + i < n_ent
                 ent1[base + i] = (int(g[e]) << 32) | int(ordv[e & (BIN_TILE - 1)])
+                win = int(ordv[e & (BIN_TILE - 1)]) - (int(tile_k0[lt1]) - kbase)
+                assert 0 <= win < BIN_TILE
+                win1[base + i] = win
 
         def runs(d1, grp):
             rs = []
-            for j in range(BIN_GROUP):
-                lt = grp * BIN_GROUP + j
+            for j in range(group):
+                lt = grp * group + j
                 if lt < tiles1:
                     a, b = off1[d1 * tiles1 + lt], off1[(d1 + 1) * tiles1 + lt]
                     rs.append((lt * nt * BIN_TILE + a, b - a))
@@ -186,6 +215,7 @@ def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
         cnt2 = np.zeros(cnt_len + 1, np.int64)
         for d1 in range(n_d1):
             for grp in range(n_groups):
+                item_n[d1 * n_groups + grp] = len(item_events(d1, grp))
                 for e in item_events(d1, grp):
                     cnt2[(((d1 << shift2) | (((e >> 32) >> BIN_BITS) & mask2)) * n_groups) + grp] += 1
         cnt2 = np.concatenate([[0], np.cumsum(cnt2[:cnt_len])])
@@ -196,6 +226,11 @@ def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
                 cur = [int(cnt2[((d1 << shift2) | d2) * n_groups + grp]) if d2 <= mask2 else 0
                        for d2 in range(DIGITS2)]
                 ev_all = item_events(d1, grp)
+                item0 = int(cnt2[(d1 << shift2) * n_groups]) + int(item_n[d1 * n_groups:d1 * n_groups + grp].sum())
+                pre = 0
+                for j, (_, ln) in enumerate(runs(d1, grp)):
+                    run1[(grp * group + j) * DIGITS1 + d1] = item0 + pre
+                    pre += ln
                 for c0 in range(0, len(ev_all), BIN_CHUNK):
                     ev = ev_all[c0:c0 + BIN_CHUNK]
                     m = len(ev)
@@ -207,7 +242,7 @@ def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
                         d = d2s[j]
                         pos = cur[d] + (i - lstart[d])
                         assert cnt2[((d1 << shift2) | d) * n_groups + grp] <= pos < n_ent
-                        ent2[pos] = ev[j]
+                        ent2[pos] = (ev[j] >> 32 << 32) | (item0 + c0 + j) if iq else ev[j]
                     for d in range(DIGITS2):
                         cur[d] += int(lstart[d + 1] - lstart[d])
         # replay
@@ -233,11 +268,15 @@ def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
                 pre = [int(sl[k]) for k in keys]
                 for i, e in enumerate(ev):
                     assert 0 <= (e >> 32) - gbase[t] - bin0 < nbins
-                    o = kbase + (e & 0xFFFFFFFF)
-                    assert o < nk
+                    o = e & 0xFFFFFFFF
+                    if iq:
+                        assert o < n_ent and res1[o] == -1
+                    else:
+                        o += kbase
+                        assert o < nk
                     if kind == po.BYTE:
                         if iq:
-                            vq[o, t] = min(255, pre[i] + rank[i] + 1)
+                            res1[o] = min(255, pre[i] + rank[i] + 1)
                         elif pre[i] + rank[i] == 0:
                             flags[o] = 1
                         if rank[i] == 0:
@@ -251,10 +290,22 @@ def binned_insert(kind, sizes, seq, off, K, mode, sub, iq=False):
                 tabs[t][bin0:bin0 + 4 * nw] = sl.astype(np.uint8)
             else:
                 tabs[t][bin0 // 8:bin0 // 8 + 4 * nw] = np.packbits(sl.astype(np.uint8), bitorder='little')
+        # combine: a tile's windows from its runs of every first digit
+        for lt1 in range(tiles1 if iq else 0):
+            k0, n_win = int(tile_k0[lt1]), int(tile_k0[lt1 + 1] - tile_k0[lt1])
+            assert 0 <= n_win <= BIN_TILE
+            least = np.full(BIN_TILE, 256, np.int64)
+            ends = [int(off1t[lt1 * DIGITS1 + d]) for d in range(DIGITS1)] + [int(off1[DIGITS1 * tiles1 + lt1])]
+            for d in range(n_d1):
+                for i in range(ends[d + 1] - ends[d]):
+                    c = int(res1[run1[lt1 * DIGITS1 + d] + i])
+                    w = int(win1[lt1 * nt * BIN_TILE + ends[d] + i])
+                    assert c >= 1 and 0 <= w < n_win
+                    least[w] = min(least[w], c)
+            assert (counts[k0:k0 + n_win] == -2).all()
+            counts[k0:k0 + n_win] = np.where(least == 256, -1, least)[:n_win]
     if iq:
-        w = vq[:nk, :nt]
-        has = w.any(1)
-        counts = np.where(has, w.min(1).astype(np.int16), -1).astype(np.int16)
+        assert (counts != -2).all()
         return tabs, None, int((counts == 1).sum()), occ, counts
     n_new = np.array([int(flags[kmer_off[r]:kmer_off[r + 1]].sum()) for r in range(n_reads)], np.uint64)
     return tabs, n_new, int(n_new.sum()), occ, None

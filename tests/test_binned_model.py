@@ -6,6 +6,7 @@ import pytest
 
 from binned_model import binned_insert
 from goetia_amd import workload
+from goetia_amd.reads import ReadBatch
 from oracle import pyoracle as po
 
 
@@ -31,14 +32,26 @@ def test_binned_model_insert_vs_oracle(kind, sizes, n_reads, sub, mode):
     assert (nu, occ) == (o.n_unique, o.n_occupied)
 
 
-def test_binned_model_insert_and_query_vs_oracle():
-    batch = _batch(9, 60)
-    sizes = po.primes_near_x(3, 5000)
-    tabs, _, nu, occ, counts = binned_insert(po.BYTE, sizes, batch.seq, batch.offsets, 21, po.MODE_SKIP_N, 8192,
+def _uneven(seed, lengths):
+    """Reads below K, empty ones and long ones."""
+    rng = np.random.default_rng(seed)
+    seq = np.frombuffer(b'ACGT', np.uint8)[rng.integers(0, 4, sum(lengths))].copy()
+    seq[::97] = ord('N')
+    return ReadBatch(seq, np.concatenate([[0], np.cumsum(lengths)]))
+
+
+@pytest.mark.parametrize('batch,sizes,sub', [
+    (_batch(9, 60), po.primes_near_x(3, 5000), 8192),
+    (_batch(11, 60), po.primes_near_x(4, 2_200_000), 8192),                             # two-level routing
+    (_batch(13, 1100), [9001], 1 << 18),                                                 # two work items
+    (_uneven(15, [5, 9000, 12, 0, 0, 3000, 2048, 20, 2047, 21, 1]), [97, 20011], 8192),
+])
+def test_binned_model_insert_and_query_vs_oracle(batch, sizes, sub):
+    tabs, _, nu, occ, counts = binned_insert(po.BYTE, sizes, batch.seq, batch.offsets, 21, po.MODE_SKIP_N, sub,
                                              iq=True)
     o = po.Storage(po.BYTE, sizes)
     exp = np.concatenate([o.insert_and_query_sequence(batch.read(r), 21, True, po.MODE_SKIP_N)
-                          for r in range(batch.n_reads)])
+                          for r in range(batch.n_reads) if len(batch.read(r)) >= 21])
     np.testing.assert_array_equal(counts, exp)
     assert (nu, occ) == (o.n_unique, o.n_occupied)
     for a, b in zip(tabs, o.tables()):

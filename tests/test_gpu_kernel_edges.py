@@ -208,12 +208,13 @@ def test_diginorm_leaves_out_events_of_dropped_reads(oracle, monkeypatch, K, cut
         assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
 
 
-@pytest.mark.parametrize('kind,max_table', [(1, 40_009), (2, 2_000_003), (2, 60_000_011)])
-@pytest.mark.parametrize('n_reads', [130, 900, 9000])
+@pytest.mark.parametrize('kind,max_table,n_reads', [(k, m, n) for k, m in ((1, 40_009), (2, 2_000_003), (2, 60_000_011))
+                                                    for n in (130, 900, 9000)]
+                         + [(2, 2_000_003, 14_500), (1, 2_000_003, 28_500), (2, 60_000_011, 57_000)])
 def test_binned_insert_in_small_groups(oracle, monkeypatch, kind, max_table, n_reads):
-    """Batches whose second pass takes 64 to 1024 tiles per item and one or
-    more of them per counting workgroup, and whose counts are scanned by one
-    workgroup or several."""
+    """Batches whose second pass takes 64 tiles per item (up to 9000 reads on a
+    256-CU device), 256, 512 and 1024, one or more of the items per counting
+    workgroup, and whose counts are scanned by one workgroup or several."""
     monkeypatch.setenv('GOETIA_AMD_BINNED', '1')
     K, sizes = 31, oracle.primes_near_x(4, max_table)
     g, o = _pair(oracle, kind, sizes, K)
@@ -231,12 +232,15 @@ def test_binned_insert_in_small_groups(oracle, monkeypatch, kind, max_table, n_r
 
 @pytest.mark.parametrize('kind,sizes', [(1, [97]), (1, [1 << 21, (1 << 21) + 1]), (2, [8191, 8209, 8219, 8221]),
                                         (2, [(1 << 21) - 1, 1 << 21, (1 << 21) + 1, 5_000_011]),
-                                        (2, [1 << 28, 3, 70_000_001]), (1, [(1 << 30) - 35, 11])])
+                                        (2, [1 << 28, 3, 70_000_001]), (1, [(1 << 29) - 3, 1 << 21]),
+                                        (1, [(1 << 28) - 2 * i for i in range(4)]),
+                                        (2, [(1 << 28) - 2 * i for i in range(4)])])
 @pytest.mark.parametrize('K,mode', [(1, N.MODE_RAW), (31, N.MODE_SKIP_N), (64, N.MODE_RAW), (255, N.MODE_SKIP_N)])
-def test_routed_query_equals_the_direct_one(oracle, monkeypatch, kind, sizes, K, mode):
-    """Slices of one bin to 2^21, digits of 1 to several hundred per table (16,
-    32 and 64 lanes to a run), runs longer than two rounds of their lanes, N
-    bases, gaps, sub-batches, hashes; present and absent windows."""
+def test_routed_query_equals_the_direct_one(oracle, monkeypatch, launches, kind, sizes, K, mode):
+    """Slices of one bin to 2^21, 1 to 512 digits in all (64 lanes to a run to
+    128 digits, 32 to 256: 163 here, 16 past that: 257 and 512), runs longer
+    than two rounds of their lanes, N bases, gaps, sub-batches, hashes; present
+    and absent windows."""
     g, o = _pair(oracle, kind, [min(s, 5_000_011) for s in sizes], K, mode=mode)
     if max(sizes) > 5_000_011:                          # too large for the oracle here: the direct query is its stand-in
         g, o = _pair(oracle, kind, sizes, K, mode=mode)[0], None
@@ -251,9 +255,12 @@ def test_routed_query_equals_the_direct_one(oracle, monkeypatch, kind, sizes, K,
         for sub in ('', '8192'):
             monkeypatch.setenv('GOETIA_AMD_SUB_BATCH', sub)
             monkeypatch.setenv('GOETIA_AMD_ROUTED', '0')
+            N.call('gt_profile_reset')
             direct, dh = g.query_sequences(b, with_hashes=True)
+            assert launches('query_route') == 0
             monkeypatch.setenv('GOETIA_AMD_ROUTED', '1')
             routed, rh = g.query_sequences(b, with_hashes=True)
+            assert launches('query_route') > 0
             np.testing.assert_array_equal(routed, direct)
             np.testing.assert_array_equal(rh, dh)
             np.testing.assert_array_equal(g.query_sequences(b), direct)
@@ -439,3 +446,14 @@ def test_exact_set_looks_its_windows_up_only_before_it_may_grow(oracle, launches
     np.testing.assert_array_equal(g.insert_sequences(b), e_new)
     assert launches('exact_lookup') == 1
     assert g.n_unique() == o.n_unique and g.n_occupied() == o.n_occupied
+
+
+@pytest.mark.parametrize('kind,sizes', [(1, [(1 << 30) - 35, 11]), (2, [1 << 30])])
+def test_tables_past_the_routed_query_are_read_directly(monkeypatch, launches, kind, sizes):
+    """More than 512 slices, and 2^30 bins: not routed even where asked for."""
+    monkeypatch.setenv('GOETIA_AMD_ROUTED', '1')
+    g = lg.dBG[STORES[kind], lg.CanLemireShifter].build(STORES[kind](sizes), 31)
+    b = _reads(1, [300] * 60, genome=6000)
+    g.insert_sequences(b)
+    assert (g.query_sequences(b) >= 1).all()
+    assert launches('query_route') == 0
