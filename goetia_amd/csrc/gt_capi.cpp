@@ -737,7 +737,7 @@ int enqueue_subbatch(gt_storage* st, Scratch& sc, const Launch& L, const Reads& 
                 ProfScope ps("exact_lookup", s);
                 Launch LL = L;
                 if (LL.per < kPerMin) LL.per = kPerMin;
-                launch_exact_lookup(LL, Rs, st->exact_view(), nullptr, ctr);
+                launch_exact_lookup(LL, Rs, st->exact_view(), ctr);
             }
             GT_HIP(hipGetLastError());
             GT_TRY(read_counters(st, c, s));
@@ -2509,7 +2509,7 @@ int gt_autotune(gt_storage* st, uint16_t K, int canonical, int mode, const uint8
                 // read-only passes: the claim (or lookup) pass writes only
                 // scratch; a later insert starts a new generation first.
                 if (st->kind == kExact) {
-                    launch_exact_lookup(L, R, st->exact_view(), nullptr, ctr);
+                    launch_exact_lookup(L, R, st->exact_view(), ctr);
                 } else {
                     launch_claim(L, R, st->tables_view(), claim_view(st, st->own), st->own.fresh.as<uint8_t>(), ctr);
                 }
@@ -2660,7 +2660,8 @@ int gt_pipeline_new(gt_storage* st, uint16_t K, int canonical, int mode, uint64_
         if (rc == GT_OK) rc = sl.d_nnew.ensure(max_reads * sizeof(uint64_t));
     }
     if (rc == GT_OK) rc = p->sc.tile_read.ensure(((max_bases + kTileGrain - 1) / kTileGrain + 1) * sizeof(uint32_t));
-    if (rc == GT_OK) rc = p->sc.fresh.ensure((max_bases + kTileMax - 1) / kTileMax * kTileMax);
+    if (rc == GT_OK && st->kind != kExact)
+        rc = p->sc.fresh.ensure((max_bases + kTileMax - 1) / kTileMax * kTileMax);
     if (rc == GT_OK) rc = alloc_claims(p->sc, st->kind != kExact ? cap : 2, p->compute);
     p->sc.fixed = true;
     if (rc == GT_OK) hip_ok(hipStreamSynchronize(p->compute), "hipStreamSynchronize");

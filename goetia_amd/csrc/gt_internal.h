@@ -171,7 +171,7 @@ struct RoutePlan {
     uint8_t* res;                         // the table's answer to each lookup: by digit, then by tile
     uint32_t* blk;                        // n_digits x blocks of 64 tiles (+1): lookups, then first index in res
     uint32_t* run;                        // n_digits x tiles: index in res of a digit's lookups of a tile
-    uint16_t* off;                        // (kRouteDigits + 1) x tiles, digit-major: start of a digit in its tile
+    uint16_t* off;                        // (n_digits + 1) x tiles, digit-major: start of a digit in its tile
     uint64_t* tile_k0;                    // per tile and one past: packed index of its first window
     uint32_t* next;                       // per XCD, kRouteNextStep words apart: blocks handed out by the gather
 };

@@ -1037,18 +1037,14 @@ struct ApplyTogetherOp : ApplyOp {
 // ------------------------------------------------------------ exact-set ops
 
 // Counts the windows whose value is absent (an upper bound of the keys that a
-// batch adds; fresh, when given, gets a byte per start).
+// batch adds).
 struct ExactLookupOp {
     ExactSet E;
-    uint8_t* fresh;
-    int64_t b0;
     int canonical;
     uint64_t n_fresh = 0;
     __device__ void operator()(int64_t s, uint32_t, int64_t, uint64_t fw, uint64_t rc, bool valid) {
         if (!valid) return;
-        const uint8_t f = exact_find(E, kmer_value(fw, rc, canonical)) == kEmpty;
-        if (fresh) fresh[s - b0] = f;
-        n_fresh += f;
+        n_fresh += exact_find(E, kmer_value(fw, rc, canonical)) == kEmpty;
     }
     __device__ void begin_tile(int64_t) {}
     __device__ void flush() {}
@@ -1494,10 +1490,9 @@ __global__ __launch_bounds__(BLK) void apply_together_kernel(Reads R, Tables T, 
 }
 
 template <int PER>
-__global__ __launch_bounds__(kBlock) void exact_lookup_kernel(Reads R, ExactSet E, uint8_t* fresh,
-                                                            uint64_t* counters) {
+__global__ __launch_bounds__(kBlock) void exact_lookup_kernel(Reads R, ExactSet E, uint64_t* counters) {
     __shared__ TileSharedT<kBlock * PER> sh;
-    ExactLookupOp op{E, fresh, R.b0, R.canonical};
+    ExactLookupOp op{E, R.canonical};
     walk_tiles<PER>(R, sh, op);
     add_counter(counters + kFresh, op.n_fresh);
 }
@@ -3168,7 +3163,8 @@ __global__ __launch_bounds__(kBlock) void solid_reads_kernel(const int64_t* off,
 // large tables therefore go through three passes:
 //
 //   route    hash a tile's windows, sort its (window, table) lookups by slice
-//            of 2 MB (a digit) in LDS and write them to the tile's region;
+//            of 2^21 bins (a digit: 2 MB of counts, 256 KB of bits) in LDS and
+//            write them to the tile's region;
 //   gather   the workgroups of one XCD take the lookups of one digit at a time,
 //            read its slice through their L2 and write a byte per lookup;
 //   combine  per tile, the minimum over the tables in LDS, written as counts.
@@ -3888,8 +3884,8 @@ void launch_apply(const Launch& L, const Reads& R, const Tables& T, const ClaimM
         GT_TILE_LAUNCH(L, apply_kernel, R, T, cm, fresh, n_new, new_flags, counters);
 }
 
-void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* fresh, uint64_t* counters) {
-    GT_TILE_LAUNCH(L, exact_lookup_kernel, R, E, fresh, counters);
+void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uint64_t* counters) {
+    GT_TILE_LAUNCH(L, exact_lookup_kernel, R, E, counters);
 }
 
 void launch_exact_add(const Launch& L, const Reads& R, const ExactSet& E, uint64_t* n_new, uint8_t* new_flags,
