@@ -46,7 +46,8 @@ BYTES_PER_KMER = {'claim': 4 * 64, 'apply': 4 * 2 * 64, 'query': 4 * (3 * 4 + 2)
 # HBM bytes per k-mer (read + write) measured with rocprofv3 FETCH_SIZE /
 # WRITE_SIZE on this workload and scaled by a 1 GiB copy (the table and the
 # commands are in profiles/cms_20m_hbm_traffic.md).
-MEASURED_BYTES_PER_KMER = {'bin_hash': 36.3, 'bin_count': 37.1, 'bin_route': 93.6, 'bin_apply': 64.0, 'bin_new': 1.2}
+MEASURED_BYTES_PER_KMER = {'bin_hash': 44.2, 'bin_count': 9.0, 'bin_route': 86.7, 'bin_apply': 64.1, 'bin_new': 1.3,
+                           'query': 153.4}
 
 
 def log(*a):
@@ -250,7 +251,8 @@ def main():
                 'unit': 'GB/s', 'frac': round(achieved / HBM_PEAK_GBPS, 4),
                 'traffic': round(traffic * n_kmers / launches) if traffic else None,
                 'traffic_source': 'profile: rocprofv3 FETCH_SIZE + WRITE_SIZE bytes per k-mer of this kernel on '
-                                  'this workload (profiles/cms_20m_hbm_traffic.md) x k-mers per launch',
+                                  'this workload (profiles/cms_20m_hbm_traffic.md) x k-mers per launch'
+                                  if traffic else None,
                 'algorithmic_bytes_per_launch': round(BYTES_PER_KMER[dom] * n_kmers / launches),
                 'launches_per_step': launches,
                 'bytes_per_kmer': BYTES_PER_KMER[dom],
