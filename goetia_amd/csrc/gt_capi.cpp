@@ -255,6 +255,7 @@ struct gt_storage {
     std::vector<uint64_t> nbytes;      // reference layout bytes per table
     std::vector<uint64_t> table_off;   // offsets in d_tables (256-aligned)
     DevBuf tables;
+    bool empty = false;                // nothing has been put into the tables since they were cleared (use_binned)
     DevBuf counters;                   // kNCounters u64
     // exact set
     DevBuf ekv, eones;                     // exact set: key / stamp word pairs, all-ones flag
@@ -379,6 +380,7 @@ int zero_tables(gt_storage* st, hipStream_t s) {
         launch_exact_clear(st->exact_view(), st->counters.as<uint64_t>(), s);
     } else {
         launch_fill_u64(st->tables.as<uint64_t>(), st->tables.bytes / 8, 0, s);
+        st->empty = true;
     }
     GT_HIP(hipGetLastError());
     return GT_OK;
@@ -782,9 +784,9 @@ uint32_t bin_buckets(const gt_storage* st) {
 }
 
 // Most buckets of n_tables tables whose small batches are inserted binned
-// (n_tables x at most 2^23 to 2^25 bins).
+// whatever the tables hold (n_tables x at most 2^22 to 2^25 bins).
 uint32_t bin_small_buckets(uint32_t n_tables) {
-    constexpr uint32_t most[kBinMaxTables + 1] = {0, 1024, 2048, 6144, 16384};
+    constexpr uint32_t most[kBinMaxTables + 1] = {0, 512, 2048, 6144, 16384};
     return n_tables <= kBinMaxTables ? most[n_tables] : 0;
 }
 
@@ -793,32 +795,40 @@ uint32_t bin_small_buckets(uint32_t n_tables) {
 // over every bucket that has an event, up to 6 ns each, whatever the bins
 // hold; the atomic one takes 0.3 to 0.9 ns more per base, and on a graph that
 // already holds most of a batch's k-mers, as it does for most of a sample,
-// about half of that.  So by default a batch of 2^20 bases and one per 256
-// bins is binned (4 x 2^28 counts: 28000 reads), where the two meet on a filled
-// graph, and on few buckets (bin_small_buckets) a batch from 2^14 bases plus 5
-// per bucket on: there the passes cost no more than the atomic insert's
-// shortest time.  Inserts of 150-base reads into an empty / a filled graph, us
-// (atomic, binned):
-//   4 x 1e6 bits       500 reads   365 / 123,    60 /   60
-//   4 x 2^25 bits     2000         336 / 131,   138 /  135
+// about half of that.  So there are two lines.  By default a batch is binned
+// from 2^20 bases and one per 256 bins on (4 x 2^28 counts: 28000 reads of
+// 150), where the two meet on a filled graph, and on few buckets
+// (bin_small_buckets) from 2^14 bases plus 5 per bucket on: there the passes
+// cost no more than the atomic insert's shortest time.  The first batch since
+// the tables were cleared is binned from 2^14 bases plus 5 per bucket, or the
+// square of a table's buckets over 192 times the tables, on.  Inserts of
+// 150-base reads into an empty / a filled graph, us (atomic in the form that
+// such a batch takes, binned):
+//   4 x 1e6 bits       500 reads   105 /  59,    60 /   60
+//   4 x 2^25 bits     2000         250 / 108,   138 /  135
 //                     3500         316 / 145,   156 /  150
-//   4 x 2^26 bits     2000         332 / 131,   192 /  192   (and 300 / 109 by windows together)
+//   4 x 2^26 bits     1000         190 /  73,   179 /  177
+//                     6000         363 / 204,   218 /  214
+//   4 x 2^27 counts   3000         440 / 205,   447 /  424
+//                     4500         497 / 185,   470 /  447
 //   2 x 2^24 bits     3500         190 /  95,   111 /  106
 //   1 x 2^25 counts   4500         150 /  95,   118 /  114
 //   4 x 2^28 counts   6000         557 / 235,   815 /  796
-//                    20000        1286 / 654,   970 /  918
+//                    14000        1015 / 480,   925 /  882
 //                    28000        1777 / 829,  1049 /  987
 //   4 x 2^28 bits     6000         375 / 204,   561 /  551
 bool use_binned(const gt_storage* st, const Scratch& sc, const Reads& R) {
-    const uint32_t buckets = bin_buckets(st);
+    const uint64_t buckets = bin_buckets(st);
     if (R.dyn || sc.fixed || !buckets) return false;
     const char* v = std::getenv("GOETIA_AMD_BINNED");
     if (v && *v) return v[0] != '0';
-    const uint64_t n_bases = (uint64_t)R.n_bases;
-    if (buckets <= bin_small_buckets(st->n_tables) && n_bases >= (1ULL << 14) + 5 * (uint64_t)buckets) return true;
+    const uint64_t n_bases = (uint64_t)R.n_bases, nt = st->n_tables;
     uint64_t bins = 0;
     for (uint64_t p : st->sizes) bins += p;
-    return n_bases >= (1ULL << 20) && n_bases * 256 >= bins;
+    if (n_bases >= (1ULL << 20) && n_bases * 256 >= bins) return true;
+    if (n_bases < (1ULL << 14) + 5 * buckets) return false;
+    if (buckets <= bin_small_buckets(st->n_tables)) return true;
+    return st->empty && n_bases >= buckets * buckets / (192 * nt * nt * nt);
 }
 
 // First-pass tiles per second-pass work item: kBinGroup, or fewer when that
@@ -1065,6 +1075,7 @@ int query_impl(gt_storage* st, Scratch& sc, const Reads& R, int16_t* counts, uin
 // (count-min only), the insert_and_query count of every window.
 int binned_insert_impl(gt_storage* st, Scratch& sc, const Reads& R, uint64_t* n_new, uint8_t* new_flags,
                        int16_t* iq_counts, hipStream_t s) {
+    st->empty = false;
     const bool iq = iq_counts != nullptr;
     const uint64_t sub = bin_sub_batch((uint64_t)R.n_bases, iq);
     BinPlan P;
@@ -1134,6 +1145,7 @@ int bigcount_iq_chunks(gt_storage* st, const uint64_t* fw, const uint64_t* rc, c
 
 int bigcount_insert_impl(gt_storage* st, Reads R, uint64_t* n_new, uint8_t* new_flags, int16_t* iq_counts,
                          hipStream_t s) {
+    st->empty = false;
     if (n_new && R.n_reads) launch_fill_u64(n_new, R.n_reads, 0, s);
     if (R.n_reads == 0 || R.n_bases == 0) return GT_OK;
     GT_TRY(prepare_reads(st, R, true, s));
@@ -1189,6 +1201,7 @@ int dbg_insert_impl(gt_storage* st, Scratch& sc, Reads R, uint64_t* n_new, uint8
         return GT_OK;
     }
     const bool binned = use_binned(st, sc, R);
+    st->empty = false;
     uint64_t sub = 0;
     GenBump bump;
     if (!binned) {
@@ -1222,6 +1235,7 @@ int dbg_insert_impl(gt_storage* st, Reads R, uint64_t* n_new, uint8_t* new_flags
 
 int hashes_insert_impl(gt_storage* st, const uint64_t* h, uint64_t n, uint8_t* is_new, hipStream_t s) {
     if (n == 0) return GT_OK;
+    st->empty = false;
     if (st->use_bigcount) {
         DevBuf full;
         GT_TRY(full.ensure(n));
@@ -1629,6 +1643,7 @@ int gt_storage_write_table(gt_storage* st, uint32_t i, const uint8_t* host_src) 
     StorageLock lk(st);
     GT_TRY(lk.rc);
     GT_HIP(hipDeviceSynchronize());
+    st->empty = false;
     GT_HIP(hipMemcpy(st->tables.as<uint8_t>() + st->table_off[i], host_src, st->nbytes[i], hipMemcpyHostToDevice));
     return GT_OK;
 }
@@ -1642,6 +1657,7 @@ int gt_storage_update_from(gt_storage* st, const gt_storage* other) {
     GT_TRY(lk.rc);
     GT_TRY(refuse_bigcount(st, "update_from"));
     GT_TRY(refuse_bigcount(other, "update_from"));
+    st->empty = false;
     GT_HIP(hipDeviceSynchronize());
     for (uint32_t i = 0; i < st->n_tables; ++i) {
         const uint64_t words = (st->nbytes[i] + 3) / 4;
@@ -1705,6 +1721,7 @@ int gt_storage_load_async(gt_storage* st, const uint8_t* const* host_tables, con
     GT_TRY(lk.rc);
     GT_TRY(order_after_fence(st, (hipStream_t)stream));
     hipStream_t s = (hipStream_t)stream;
+    st->empty = !host_tables;
     if (!host_tables) {
         launch_fill_u64(st->tables.as<uint64_t>(), st->tables.bytes / 8, 0, s);
         launch_fill_u64(st->counters.as<uint64_t>(), 2, 0, s);
@@ -1947,6 +1964,7 @@ int gt_dbg_insert_and_query_dev(gt_storage* st, uint16_t K, int canonical, int m
         st->own.release_events();       // no room for the event buffers: strict order below
     }
     if (st->kind == kByte) {
+        st->empty = false;
         // More than four tables or 2^30 bins: hash the batch, then apply it
         // with the sort-based exact insert_and_query.
         GT_TRY(prepare_reads(st, R, true, s));
@@ -2073,6 +2091,7 @@ int gt_diginorm_dev(gt_storage* st, uint16_t K, int canonical, int mode, const u
     StorageLock lk(st);
     GT_TRY(lk.rc);
     GT_TRY(refuse_bigcount(st, "the batched diginorm filter"));
+    st->empty = false;
     GT_TRY(order_after_fence(st, (hipStream_t)stream));
     hipStream_t s = (hipStream_t)stream;
     // chunks end at read boundaries: the offsets come to the host once
@@ -2431,6 +2450,7 @@ int gt_insert_and_query_hashes(gt_storage* st, const uint64_t* hashes, uint64_t 
             GT_TRY(full.ensure(n));
             fl = full.as<uint8_t>();
         }
+        st->empty = false;
         GT_TRY(sorted_insert_query(st->tables_view(), st->h_out3.as<uint64_t>(), nullptr, nullptr, n, 0,
                                    st->h_out1.as<int16_t>(), nullptr, st->counters.as<uint64_t>(), g_dev.cus, s, fl));
         if (fl)
@@ -2686,6 +2706,7 @@ int gt_pipeline_submit(gt_pipeline* p, const uint8_t* seq, const int64_t* offset
     StorageLock lk(st);
     GT_TRY(lk.rc);
     GT_TRY(refuse_bigcount(st, "the captured pipeline"));
+    st->empty = false;
     GT_TRY(order_after_fence(st, p->compute));
     gt_pipeline::Slot& sl = p->slot[p->next];
     p->next ^= 1;

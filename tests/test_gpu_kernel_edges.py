@@ -392,18 +392,49 @@ def test_atomic_inserts_at_every_shape_of_launch(oracle, monkeypatch, kind, n_ta
         np.testing.assert_array_equal(x, y)
 
 
-@pytest.mark.parametrize('kind,n_tables,table,n_reads,binned', [
-    (1, 4, 1_000_000, 100, False), (1, 4, 1_000_000, 300, True), (2, 4, 1 << 25, 1000, True),
-    (1, 4, 1 << 26, 6900, False), (1, 4, 1 << 26, 7000, True), (2, 2, 1 << 24, 3000, False),
-    (2, 1, 1 << 25, 3000, False), (2, 1, 1 << 25, 7000, True), (2, 4, 1 << 28, 6000, False),
-    (2, 4, 1 << 28, 27_900, False), (2, 4, 1 << 28, 28_000, True), (2, 1, 1 << 28, 3000, False)])
-def test_batches_are_binned_where_that_is_the_faster_insert(oracle, launches, kind, n_tables, table, n_reads, binned):
-    """Which insert a batch takes by itself, on both sides of its lines."""
+@pytest.mark.parametrize('kind,n_tables,table,n_reads,empty,filled', [
+    (1, 4, 1_000_000, 100, False, False), (1, 4, 1_000_000, 300, True, True), (2, 4, 1 << 25, 1000, True, True),
+    (1, 4, 1 << 26, 1100, False, False), (1, 4, 1 << 26, 1300, True, False), (1, 4, 1 << 26, 7000, True, True),
+    (2, 2, 1 << 24, 3000, True, False), (2, 1, 1 << 25, 700, True, False), (2, 1, 1 << 25, 7000, True, True),
+    (2, 4, 1 << 28, 6000, False, False), (2, 4, 1 << 28, 9400, True, False), (2, 4, 1 << 28, 27_900, True, False),
+    (2, 4, 1 << 28, 28_000, True, True), (2, 1, 1 << 28, 3000, False, False)])
+def test_batches_are_binned_where_that_is_the_faster_insert(oracle, launches, kind, n_tables, table, n_reads, empty,
+                                                            filled):
+    """Which insert a batch takes by itself, on both sides of the lines for an
+    empty graph and for one that holds k-mers; a reset or new tables make it
+    empty, every other call that writes to it does not."""
     sizes = [table - 2 * i for i in range(n_tables)]
     g = _pair(oracle, kind, sizes, 31)[0]
     b = _reads(1, [150] * n_reads, genome=20_000)
-    assert int(g.insert_sequences(b).sum()) == g.n_unique()
-    assert (launches('bin_hash') > 0) == binned and (launches('claim') > 0) != binned
+
+    def binned(batch):
+        N.call('gt_profile_reset')
+        g.insert_sequences(batch)
+        assert launches('bin_hash') + launches('claim') == 1
+        return launches('bin_hash') > 0
+    assert binned(b) == empty
+    assert binned(b) == filled
+    g.reset()
+    g.S.insert_hashes(np.arange(3, dtype=np.uint64))
+    assert binned(b) == filled
+    g.reset()
+    assert binned(b) == empty
+    if kind == 2:
+        g.reset()
+        g.insert_and_query_sequences(_reads(2, [40], genome=100))
+        assert binned(b) == filled
+        g.reset()
+        lg.DiginormFilter.build(g, 5).filter_sequences(_reads(2, [40], genome=100))
+        assert binned(b) == filled
+    else:
+        h = _pair(oracle, kind, sizes, 31)[0]
+        g.reset()
+        g.S.update_from(h.S)
+        assert binned(b) == filled
+    if table <= 1_000_000:
+        g.reset()
+        g.S.set_raw_table(0, g.S.get_raw_tables()[0])
+        assert binned(b) == filled
 
 
 @pytest.mark.parametrize('lengths', [[9000] * 12, [150] * 4000, [31] * 3000 + [4500] * 3, [40, 31, 2000, 33] * 200])
