@@ -286,13 +286,13 @@ __device__ int16_t storage_query(const Tables& T, const ExactSet& E, uint64_t h)
 // nearly all of those.  The reads of one table are issued together.  Bound by
 // random table lines: for the 32M new k-mers of 1M reads (4 x 2^28 bins, count
 // >= 2) reading all 32 bins of every window took 21.5 ms, this takes 7 ms.
-// One storage kind per kernel: the three together need a quarter more registers
-// than the widest, and one wave less to a SIMD.
-template <int KIND>
+// An exact set has a kernel of its own (kSet): next to the tables' code its
+// probes take 15 registers more, and one wave less to a SIMD.
+template <bool kSet>
 __device__ __forceinline__ uint32_t neighbors_present(const Tables& T, const ExactSet& E, const uint64_t (&v)[8],
                                                       int min_count) {
     uint32_t alive = 0xFFu;
-    if constexpr (KIND == kByte) {
+    if (!kSet && T.kind == kByte) {
         GT_FOR_TABLES(i, T) {
             uint32_t c[8];
 #pragma unroll
@@ -307,7 +307,7 @@ __device__ __forceinline__ uint32_t neighbors_present(const Tables& T, const Exa
         return alive;
     }
     if (min_count > 1) return 0;                         // presence storages answer 0 or 1
-    if constexpr (KIND == kBit) {
+    if constexpr (!kSet) {
         GT_FOR_TABLES(i, T) {
             uint32_t w[8];
 #pragma unroll
@@ -1345,7 +1345,7 @@ struct DegreeStage {
     int64_t k0, k1;
 };
 
-template <int TILE, int KIND>
+template <int TILE, bool kSet>
 struct DegreeOp {
     Tables T;
     ExactSet E;
@@ -1393,7 +1393,7 @@ struct DegreeOp {
             const uint64_t R2 = lr ^ tr[x];
             v[c] = kmer_value(F2, R2, R.canonical);
         }
-        const uint32_t mask = neighbors_present<KIND>(T, E, v, min_count);
+        const uint32_t mask = neighbors_present<kSet>(T, E, v, min_count);
         if (nb_val) {
 #pragma unroll
             for (int c = 0; c < 8; ++c) nb_val[(k0 + i) * 8 + c] = v[c];
@@ -1550,13 +1550,13 @@ __global__ __launch_bounds__(kBlock) void hash_kernel(Reads R, uint64_t* fw, uin
     walk_tiles<PER>(R, sh, op);
 }
 
-template <int PER, int KIND>
-__global__ __launch_bounds__(kBlock, PER == 32 ? 3 : 4) void degree_kernel(Reads R, Tables T, ExactSet E, int min_count,
+template <int PER, bool kSet>
+__global__ __launch_bounds__(kBlock) void degree_kernel(Reads R, Tables T, ExactSet E, int min_count,
                                                       const uint8_t* only, uint8_t* in_deg, uint8_t* out_deg,
                                                       uint64_t* nb_val, uint8_t* nb_mask) {
     __shared__ TileSharedT<kBlock * PER> sh;
     __shared__ DegreeStage<kBlock * PER> st;
-    DegreeOp<kBlock * PER, KIND> op{T,       E,       R,        kBlock * PER, min_count, only, in_deg,
+    DegreeOp<kBlock * PER, kSet> op{T,       E,       R,        kBlock * PER, min_count, only, in_deg,
                                     out_deg, nb_val,  nb_mask,  sh.bytes,     sh.tf,     sh.tr, &st};
     walk_tiles<PER>(R, sh, op);
 }
@@ -3925,20 +3925,16 @@ void launch_hash(const Launch& L, const Reads& R, uint64_t* fw, uint64_t* rc, ui
 }
 
 template <int PER>
-constexpr auto byte_degree_kernel = degree_kernel<PER, kByte>;
+constexpr auto table_degree_kernel = degree_kernel<PER, false>;
 template <int PER>
-constexpr auto bit_degree_kernel = degree_kernel<PER, kBit>;
-template <int PER>
-constexpr auto exact_degree_kernel = degree_kernel<PER, kExact>;
+constexpr auto set_degree_kernel = degree_kernel<PER, true>;
 
 void launch_degrees(const Launch& L, const Reads& R, const Tables& T, const ExactSet& E, int min_count,
                     const uint8_t* only, uint8_t* in_deg, uint8_t* out_deg, uint64_t* nb_val, uint8_t* nb_mask) {
-    if (T.kind == kByte)
-        GT_TILE_LAUNCH(L, byte_degree_kernel, R, T, E, min_count, only, in_deg, out_deg, nb_val, nb_mask);
-    else if (T.kind == kBit)
-        GT_TILE_LAUNCH(L, bit_degree_kernel, R, T, E, min_count, only, in_deg, out_deg, nb_val, nb_mask);
+    if (T.kind == kExact)
+        GT_TILE_LAUNCH(L, set_degree_kernel, R, T, E, min_count, only, in_deg, out_deg, nb_val, nb_mask);
     else
-        GT_TILE_LAUNCH(L, exact_degree_kernel, R, T, E, min_count, only, in_deg, out_deg, nb_val, nb_mask);
+        GT_TILE_LAUNCH(L, table_degree_kernel, R, T, E, min_count, only, in_deg, out_deg, nb_val, nb_mask);
 }
 
 void launch_hash_claim(const Launch& L, const uint64_t* h, uint64_t n, const Tables& T, const ClaimMap& cm,
