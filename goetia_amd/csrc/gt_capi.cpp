@@ -686,10 +686,26 @@ Launch make_launch(const gt_storage* st, uint64_t n_starts, uint64_t few, hipStr
     return L;
 }
 
-// Queries, and all passes over an exact set: below 2^22 starts.  4167 reads of
-// 150 against 4 x 2^28 counts take 58 us together and 86 window by window,
-// 27000 take 270 and 285.
+// Queries, and inserts into an exact set: below 2^22 starts.  4167 reads of 150
+// against 4 x 2^28 counts take 58 us together and 86 window by window, 27900
+// take 274 and 292; with hashes the together form is the faster one past that.
 constexpr uint64_t kFewStarts = 1ULL << 22;
+
+// Counts alone from an exact set, or from at most two tables past the L2s:
+// below 1,572,864 starts, since a window has few accesses to take together.
+// Reads of 150 whose k-mers are there / are not, us (together, window by window):
+//   exact set       9000   55 / 62,   59 /  62      20000   88 /  97,   79 /  83
+//   1 x 2^28 counts 9000   53 / 56,   55 /  55      20000   82 /  85,   80 /  83
+//   2 x 2^28 bits   9000   66 / 70,   78 /  72      20000  114 / 117,  119 /  93
+// (4 x 1e6 bits, 125 KB each: 52 / 53, 78 / 75 and 80 / 81, 94 / 91.)
+constexpr uint64_t kFewLoneStarts = 3ULL << 19;
+constexpr uint64_t kPastL2 = 30ULL << 20;          // bytes: smaller tables are read mostly out of the L2s
+uint64_t few_query_starts(const gt_storage* st, const uint64_t* hashes) {
+    uint64_t bytes = 0;
+    for (uint64_t nb : st->nbytes) bytes += nb;
+    const bool lone = st->kind == kExact || (st->n_tables <= 2 && bytes >= kPastL2);
+    return lone && !hashes ? kFewLoneStarts : kFewStarts;
+}
 
 // Atomic inserts into Bloom / count-min tables: below 393,216 starts.  Their
 // claims and updates of four tables at a time take 248 registers, two
@@ -775,6 +791,16 @@ int enqueue_subbatch(gt_storage* st, Scratch& sc, const Launch& L, const Reads& 
 
 // ------------------------------------------------------------ binned insert
 
+// The bases of a batch as the lines below count them, those of 150-base reads at
+// K = 31, where four of five start a window: fewer where reads are not much
+// longer than K.  (Reads below K make it fewer still; their number is only
+// known on the device.)
+uint64_t busy_bases(const Reads& R) {
+    const uint64_t n = (uint64_t)R.n_bases, ends = R.n_reads * (uint64_t)(R.K - 1);
+    const uint64_t windows = n > ends ? n - ends : 0;
+    return std::min(n, windows + windows / 4);
+}
+
 // Buckets of the binned insert over a storage's tables (0: not eligible).
 uint32_t bin_buckets(const gt_storage* st) {
     if ((st->kind != kByte && st->kind != kBit) || st->n_tables == 0 || st->n_tables > kBinMaxTables) return 0;
@@ -795,7 +821,9 @@ uint32_t bin_small_buckets(uint32_t n_tables) {
 // over every bucket that has an event, up to 6 ns each, whatever the bins
 // hold; the atomic one takes 0.3 to 0.9 ns more per base, and on a graph that
 // already holds most of a batch's k-mers, as it does for most of a sample,
-// about half of that.  So there are two lines.  By default a batch is binned
+// about half of that.  So there are two lines, both in busy bases (75-base reads
+// at K = 63 into a filled 4 x 2^28 counts: 0.95 and 1.16 ms for 3.2M of them in
+// 15M bases, 4.30 and 2.70 ms for 16M).  By default a batch is binned
 // from 2^20 bases and one per 256 bins on (4 x 2^28 counts: 28000 reads of
 // 150), where the two meet on a filled graph, and on few buckets
 // (bin_small_buckets) from 2^14 bases plus 5 per bucket on: there the passes
@@ -822,7 +850,7 @@ bool use_binned(const gt_storage* st, const Scratch& sc, const Reads& R) {
     if (R.dyn || sc.fixed || !buckets) return false;
     const char* v = std::getenv("GOETIA_AMD_BINNED");
     if (v && *v) return v[0] != '0';
-    const uint64_t n_bases = (uint64_t)R.n_bases, nt = st->n_tables;
+    const uint64_t n_bases = busy_bases(R), nt = st->n_tables;
     uint64_t bins = 0;
     for (uint64_t p : st->sizes) bins += p;
     if (n_bases >= (1ULL << 20) && n_bases * 256 >= bins) return true;
@@ -979,9 +1007,10 @@ uint32_t route_digits(const gt_storage* st) {
 // Whether a query goes through the routed passes (GOETIA_AMD_ROUTED=0 / 1
 // forces it off / on where the tables allow it): by default on two tables or
 // more of 30 MiB together (smaller ones are read mostly out of the L2s as they
-// are; one table's reads cost less than their routing), from 2^23 bases plus
-// one per 64 table bytes on (every slice is read into an L2 once per
-// sub-batch).  150-base reads, us (direct / routed):
+// are; one table's reads cost less than their routing), from 2^23 busy bases
+// plus one per 64 table bytes on (every slice is read into an L2 once per
+// sub-batch), on reads most of whose bases start a window: a base is hashed and
+// sorted whether it does or not.  150-base reads, us (direct / routed):
 //   4 x 2^21 counts   300k reads 1332 / 3278
 //   4 x 2^23 counts   30k reads  247 /  382    100k  792 /  729     1M 7431 / 6016
 //   4 x 2^25 counts   30k reads  293 /  333    100k  937 /  848     1M 8852 / 5473
@@ -989,13 +1018,19 @@ uint32_t route_digits(const gt_storage* st) {
 //   4 x 2^28 bits     30k reads  270 /  267    100k  859 /  670     1M 8076 / 5984
 //   2 x 2^28 bits     30k reads  152 /  188    100k  458 /  414     1M 4183 / 3707
 //   1 x 2^28 counts   1M reads  2468 / 3255
+// and 1M reads by the share of bases that start a window:
+//   4 x 2^28 counts   0.28 1820 / 2848   0.39 3219 / 4158   0.60 4765 / 4470
+//   4 x 2^28 bits     0.28 1781 / 2509   0.39 3170 / 3460   0.60 4803 / 3671
+//   2 x 2^28 counts   0.39 1759 / 2670   0.60 2516 / 2763
 bool use_routed(const gt_storage* st, const Scratch& sc, const Reads& R) {
     if (R.dyn || sc.fixed || !route_digits(st)) return false;
     const char* v = std::getenv("GOETIA_AMD_ROUTED");
     if (v && *v) return v[0] != '0';
     uint64_t bytes = 0;
     for (uint64_t nb : st->nbytes) bytes += nb;
-    return st->n_tables >= 2 && bytes >= (30ULL << 20) && (uint64_t)R.n_bases >= (1ULL << 23) + bytes / 64;
+    const uint64_t busy = busy_bases(R), n = (uint64_t)R.n_bases;      // (busy is at most 5/4 of the windows)
+    if (st->n_tables < 2 || 80 * busy < (st->n_tables == 2 ? 70ULL : 45ULL) * n) return false;
+    return bytes >= kPastL2 && busy >= (1ULL << 23) + bytes / 64;
 }
 
 // Query of prepared reads through the routed passes, in sub-batches of 2^27
@@ -1064,7 +1099,8 @@ int query_impl(gt_storage* st, Scratch& sc, const Reads& R, int16_t* counts, uin
         sc.release_events();            // no room for the lookups: read the tables window by window
     }
     ProfScope ps("query", s);
-    launch_query(make_launch(st, (uint64_t)R.n_bases, kFewStarts, s), R, st->tables_view(), st->exact_or_empty(), counts, hashes);
+    launch_query(make_launch(st, (uint64_t)R.n_bases, few_query_starts(st, hashes), s), R, st->tables_view(),
+                 st->exact_or_empty(), counts, hashes);
     GT_HIP(hipGetLastError());
     return GT_OK;
 }

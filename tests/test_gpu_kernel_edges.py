@@ -488,3 +488,51 @@ def test_tables_past_the_routed_query_are_read_directly(monkeypatch, launches, k
     g.insert_sequences(b)
     assert (g.query_sequences(b) >= 1).all()
     assert launches('query_route') == 0
+
+
+@pytest.mark.parametrize('kind,sizes', [(1, [60_013]), (2, [60_013]), (2, [60_013, 60_017]), (3, ())])
+@pytest.mark.parametrize('n_bases', [(3 << 19) - 1, 3 << 19, 1 << 22])
+@pytest.mark.parametrize('with_hashes', [False, True])
+def test_queries_of_few_tables_at_every_shape_of_launch(oracle, kind, sizes, n_bases, with_hashes):
+    """Either side of the sizes where a query of an exact set or of one or two
+    tables changes its shape, alone and with hashes (whose line is another)."""
+    K = 31
+    g, o = _pair(oracle, kind, sizes, K, mode=N.MODE_SKIP_N)
+    fill = _reads(1, [150] * 300, genome=60_000)
+    o.insert_reads(fill.seq, fill.offsets, K, True, N.MODE_SKIP_N)
+    g.insert_sequences(fill)
+    n, tail = divmod(n_bases, 150)
+    b = _reads(1, [150] * n + [tail], genome=60_000, sub=0.004, n_rate=0.001)
+    exp = o.query_reads(b.seq, b.offsets, K, True, N.MODE_SKIP_N)
+    if with_hashes:
+        counts, hashes = g.query_sequences(b, with_hashes=True)
+        for r in (0, n // 2, n):
+            if len(b.read(r)) >= K:
+                k0 = int(b.kmer_offsets(K)[r])
+                fw, rc = oracle.hash_read(bytes(b.read(r)), K)
+                live = exp[k0:k0 + len(fw)] >= 0
+                np.testing.assert_array_equal(hashes[k0:k0 + len(fw)][live], np.minimum(fw, rc)[live])
+    else:
+        counts = g.query_sequences(b)
+    np.testing.assert_array_equal(counts, exp)
+
+
+@pytest.mark.parametrize('n_tables,L,K,n_reads,routed', [
+    (4, 150, 31, 70_000, True), (4, 150, 31, 58_000, False), (4, 75, 63, 200_000, False), (4, 75, 55, 700_000, False),
+    (4, 101, 41, 160_000, True), (2, 150, 31, 70_000, True), (2, 75, 31, 400_000, False), (1, 150, 31, 200_000, False)])
+def test_queries_are_routed_where_windows_are_many(oracle, launches, n_tables, L, K, n_reads, routed):
+    """Which way a query goes by itself: by its bases, less those that start no
+    window, and by their share."""
+    import torch
+    from goetia_amd.reads import DeviceReads
+    sizes = [(1 << 25) // n_tables - 2 * i for i in range(n_tables)]
+    g = _pair(oracle, 2, sizes, K)[0]
+    fill = _reads(1, [L] * 2000, genome=40_000, sub=0.0)
+    g.insert_sequences(fill)
+    d = DeviceReads(torch.from_numpy(np.tile(fill.seq, n_reads // 2000)).cuda(),
+                    torch.arange(n_reads + 1, dtype=torch.int64, device='cuda') * L, n_reads * L)
+    counts = torch.empty(n_reads * (L - K + 1), dtype=torch.int16, device='cuda')
+    g.query_device(d, counts)
+    exp = torch.from_numpy(g.query_sequences(fill)).cuda()
+    assert bool((counts.view(n_reads // 2000, -1) == exp).all())
+    assert (launches('query_route') > 0) == routed
