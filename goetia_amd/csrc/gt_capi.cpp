@@ -735,6 +735,7 @@ int enqueue_subbatch(gt_storage* st, Scratch& sc, const Launch& L, const Reads& 
     const ClaimMap cm = claim_view(st, sc);
     if (st->kind == kExact) {
         const uint64_t nstarts = (uint64_t)(Rs.b1 - Rs.b0);
+        uint8_t* absent = nullptr;
         // ecount_ub counts every window since the last look at the set's real
         // size; that look is enough unless the set may have to grow, and only
         // then is the growth bounded by this sub-batch's absent windows.  (With
@@ -750,12 +751,14 @@ int enqueue_subbatch(gt_storage* st, Scratch& sc, const Launch& L, const Reads& 
         if (fits) {
             st->ecount_ub += nstarts;
         } else {
+            // the windows found are left out of the insert (where their bytes fit)
+            if (sc.fresh.ensure((nstarts + 3) / 4 * 4) == GT_OK) absent = sc.fresh.as<uint8_t>();
             launch_fill_u64(ctr + kFresh, 1, 0, s);
             {
                 ProfScope ps("exact_lookup", s);
                 Launch LL = L;
                 if (LL.per < kPerMin) LL.per = kPerMin;
-                launch_exact_lookup(LL, Rs, st->exact_view(), ctr);
+                launch_exact_lookup(LL, Rs, st->exact_view(), absent, ctr);
             }
             GT_HIP(hipGetLastError());
             GT_TRY(read_counters(st, c, s));
@@ -765,7 +768,7 @@ int enqueue_subbatch(gt_storage* st, Scratch& sc, const Launch& L, const Reads& 
         const ExactSet E = st->exact_view();
         {
             ProfScope ps("exact_insert", s);
-            launch_exact_add(L, Rs, E, n_new, new_flags, ctr);
+            launch_exact_add(L, Rs, E, n_new, new_flags, absent, ctr);
         }
         if (new_flags) {
             ProfScope ps("exact_resolve", s);
@@ -2565,7 +2568,7 @@ int gt_autotune(gt_storage* st, uint16_t K, int canonical, int mode, const uint8
                 // read-only passes: the claim (or lookup) pass writes only
                 // scratch; a later insert starts a new generation first.
                 if (st->kind == kExact) {
-                    launch_exact_lookup(L, R, st->exact_view(), ctr);
+                    launch_exact_lookup(L, R, st->exact_view(), nullptr, ctr);
                 } else {
                     launch_claim(L, R, st->tables_view(), claim_view(st, st->own), st->own.fresh.as<uint8_t>(), ctr);
                 }

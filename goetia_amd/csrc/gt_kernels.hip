@@ -1037,14 +1037,18 @@ struct ApplyTogetherOp : ApplyOp {
 // ------------------------------------------------------------ exact-set ops
 
 // Counts the windows whose value is absent (an upper bound of the keys that a
-// batch adds).
+// batch adds); absent, when given, gets a byte per start of a window.
 struct ExactLookupOp {
     ExactSet E;
+    uint8_t* absent;
+    int64_t b0;
     int canonical;
     uint64_t n_fresh = 0;
     __device__ void operator()(int64_t s, uint32_t, int64_t, uint64_t fw, uint64_t rc, bool valid) {
         if (!valid) return;
-        n_fresh += exact_find(E, kmer_value(fw, rc, canonical)) == kEmpty;
+        const uint8_t f = exact_find(E, kmer_value(fw, rc, canonical)) == kEmpty;
+        if (absent) absent[s - b0] = f;
+        n_fresh += f;
     }
     __device__ void begin_tile(int64_t) {}
     __device__ void flush() {}
@@ -1070,6 +1074,7 @@ struct ExactAddOp {
     uint64_t* per_read;                    // new k-mers per read, or null
     const int64_t* kmer_off;
     uint8_t* new_flags;                    // or null: 1 for windows that were their key's first for a while
+    const uint8_t* absent;                 // or null: a byte per start, 0 for windows of keys of earlier batches
     uint64_t n_new = 0;
     uint64_t last_ins = 0;                 // position + 1 of the last inserted window
 
@@ -1129,18 +1134,27 @@ struct ExactAddOp {
     __device__ void together(const Windows<PER>& w) {
         uint64_t slot[PER];
         ulonglong2 kv[PER];
+        // a batch that was looked up first has nothing to do for the keys it found
+        uint32_t live = w.valid;
+        if (absent) {
+            static_assert(PER == 4, "a word of absent bytes");
+            const uint32_t a = *reinterpret_cast<const uint32_t*>(absent + (w.s0 - b0));
+#pragma unroll
+            for (int j = 0; j < PER; ++j)
+                if (!(a >> (8 * j) & 1u)) live &= ~(1u << j);
+        }
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             slot[j] = w.h[j] == kEmpty ? 0 : exact_home(E, w.h[j]);
-            if (w.valid >> j & 1u) kv[j] = exact_pair(E, slot[j]);
+            if (live >> j & 1u) kv[j] = exact_pair(E, slot[j]);
         }
         uint64_t got[PER];
         uint32_t todo = 0, fresh = 0;      // windows to probe on, windows of new keys
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             got[j] = kEmpty;
-            if (!(w.valid >> j & 1u)) continue;
-            last_ins = (uint64_t)(w.s0 + j - b0) + 1;
+            if (w.valid >> j & 1u) last_ins = (uint64_t)(w.s0 + j - b0) + 1;
+            if (!(live >> j & 1u)) continue;
             if (w.h[j] != kEmpty && kv[j].x == w.h[j])
                 fresh |= (stamp_is_fresh(kv[j].y, gen) ? 1u : 0u) << j;
             else if (w.h[j] != kEmpty && kv[j].x == kEmpty)
@@ -1151,7 +1165,7 @@ struct ExactAddOp {
         }
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
-            if (!(w.valid >> j & 1u)) continue;
+            if (!(live >> j & 1u)) continue;
             if (!(todo >> j & 1u) && kv[j].x == kEmpty) {
                 if (got[j] == kEmpty || got[j] == w.h[j]) fresh |= 1u << j; else todo |= 1u << j;
             }
@@ -1490,9 +1504,10 @@ __global__ __launch_bounds__(BLK) void apply_together_kernel(Reads R, Tables T, 
 }
 
 template <int PER>
-__global__ __launch_bounds__(kBlock) void exact_lookup_kernel(Reads R, ExactSet E, uint64_t* counters) {
+__global__ __launch_bounds__(kBlock) void exact_lookup_kernel(Reads R, ExactSet E, uint8_t* absent,
+                                                            uint64_t* counters) {
     __shared__ TileSharedT<kBlock * PER> sh;
-    ExactLookupOp op{E, R.canonical};
+    ExactLookupOp op{E, absent, R.b0, R.canonical};
     walk_tiles<PER>(R, sh, op);
     add_counter(counters + kFresh, op.n_fresh);
 }
@@ -1504,14 +1519,14 @@ __global__ __launch_bounds__(kBlock) void exact_lookup_kernel(Reads R, ExactSet 
 // 220k uneven reads at 5% substitutions; this takes 20 ms.
 template <int BLK>
 __global__ __launch_bounds__(BLK) void exact_add_kernel(Reads R, ExactSet E, uint64_t* n_new, uint8_t* new_flags,
-                                                      uint64_t* counters) {
+                                                      const uint8_t* absent, uint64_t* counters) {
     __shared__ TileSharedT<BLK * kPerSmall> sh;
     __shared__ SegScratchT<BLK + kSegExtra> seg;
     uint64_t n_reads;
     int64_t n_bases;
     batch_sizes(R, n_reads, n_bases);      // the reads that are there, not a captured batch's bound
     Stitched<ExactAddOp, BLK> op{{E, R.b0, current_gen(counters), R.off, n_reads, counters + kErrors, n_new,
-                                  R.kmer_off, new_flags}, &seg};
+                                  R.kmer_off, new_flags, absent}, &seg};
     walk_tiles<kPerSmall, BLK>(R, sh, op);
     add_counter(counters + kNUnique, op.n_new);
     max_counter(counters + kLastIns, op.last_ins);
@@ -3884,15 +3899,15 @@ void launch_apply(const Launch& L, const Reads& R, const Tables& T, const ClaimM
         GT_TILE_LAUNCH(L, apply_kernel, R, T, cm, fresh, n_new, new_flags, counters);
 }
 
-void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uint64_t* counters) {
-    GT_TILE_LAUNCH(L, exact_lookup_kernel, R, E, counters);
+void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* absent, uint64_t* counters) {
+    GT_TILE_LAUNCH(L, exact_lookup_kernel, R, E, absent, counters);
 }
 
 void launch_exact_add(const Launch& L, const Reads& R, const ExactSet& E, uint64_t* n_new, uint8_t* new_flags,
-                      uint64_t* counters) {
+                      const uint8_t* absent, uint64_t* counters) {
     Launch small = L;
     small.per = kPerSmall;
-    GT_TOGETHER_LAUNCH(small, exact_add_kernel, R, E, n_new, new_flags, counters);
+    GT_TOGETHER_LAUNCH(small, exact_add_kernel, R, E, n_new, new_flags, absent, counters);
 }
 
 void launch_exact_flags(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* new_flags,

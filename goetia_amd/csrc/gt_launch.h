@@ -31,10 +31,11 @@ void launch_claim(const Launch& L, const Reads& R, const Tables& T, const ClaimM
                   uint64_t* counters);
 void launch_apply(const Launch& L, const Reads& R, const Tables& T, const ClaimMap& cm, const uint8_t* fresh,
                   uint64_t* n_new, uint8_t* new_flags, uint64_t* counters);
-void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uint64_t* counters);
-// new_flags (with R.kmer_off), where given: launch_exact_flags then settles them.
+void launch_exact_lookup(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* absent, uint64_t* counters);
+// new_flags (with R.kmer_off), where given: launch_exact_flags then settles them.  absent, where given: the same
+// sub-batch's lookup (the set may have been rehashed since).
 void launch_exact_add(const Launch& L, const Reads& R, const ExactSet& E, uint64_t* n_new, uint8_t* new_flags,
-                      uint64_t* counters);
+                      const uint8_t* absent, uint64_t* counters);
 void launch_exact_flags(const Launch& L, const Reads& R, const ExactSet& E, uint8_t* new_flags,
                         const uint64_t* counters);
 void launch_exact_tail(uint64_t* counters, hipStream_t s);
