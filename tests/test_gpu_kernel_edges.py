@@ -124,7 +124,7 @@ def test_small_batches_take_windows_together(oracle, monkeypatch, kind, n_tables
                 np.testing.assert_array_equal(x, y)
 
 
-@pytest.mark.parametrize('n_reads', [1, 1023, 1025, 16384, 16385])
+@pytest.mark.parametrize('n_reads', [1, 1023, 1025, 12288, 12289, 16384, 16385])
 @pytest.mark.parametrize('binned', ['0', '1'])
 def test_layout_of_small_batches(oracle, monkeypatch, n_reads, binned):
     """Either side of the one-launch layout's limit: packed results of reads of
