@@ -830,24 +830,25 @@ uint32_t bin_small_buckets(uint32_t n_tables) {
 // from 2^20 bases and one per 256 bins on (4 x 2^28 counts: 28000 reads of
 // 150), where the two meet on a filled graph, and on few buckets
 // (bin_small_buckets) from 2^14 bases plus 5 per bucket on: there the passes
-// cost no more than the atomic insert's shortest time.  The first batch since
+// cost half of the atomic insert's time on an empty graph and 0.9 to 1.2 of it
+// on a filled one.  The first batch since
 // the tables were cleared is binned from 2^14 bases plus 5 per bucket, or the
 // square of a table's buckets over 192 times the tables, on.  Inserts of
 // 150-base reads into an empty / a filled graph, us (atomic in the form that
 // such a batch takes, binned):
-//   4 x 1e6 bits       500 reads   105 /  59,    60 /   60
-//   4 x 2^25 bits     2000         250 / 108,   138 /  135
-//                     3500         316 / 145,   156 /  150
-//   4 x 2^26 bits     1000         190 /  73,   179 /  177
-//                     6000         363 / 204,   218 /  214
-//   4 x 2^27 counts   3000         440 / 205,   447 /  424
-//                     4500         497 / 185,   470 /  447
-//   2 x 2^24 bits     3500         190 /  95,   111 /  106
-//   1 x 2^25 counts   4500         150 /  95,   118 /  114
-//   4 x 2^28 counts   6000         557 / 235,   815 /  796
-//                    14000        1015 / 480,   925 /  882
-//                    28000        1777 / 829,  1049 /  987
-//   4 x 2^28 bits     6000         375 / 204,   561 /  551
+//   4 x 2^22 bits      500 reads   155 /  56,    66 /  62
+//   4 x 2^25 bits     2000         263 / 111,   138 / 135
+//                     3500         316 / 145,   156 / 150
+//   4 x 2^26 bits     1000         188 /  73,   179 / 177
+//                     6000         363 / 194,   218 / 214
+//   4 x 2^27 counts   3000         454 / 183,   447 / 424
+//                     4500         497 / 185,   470 / 447
+//   2 x 2^24 bits     3500         190 /  95,   111 / 106
+//   1 x 2^25 counts   4500         150 /  95,   118 / 114
+//   4 x 2^28 counts   6000         562 / 224,   816 / 795
+//                    14000        1021 / 477,   924 / 887
+//                    28000        2023 / 943,  1049 / 987
+//   4 x 2^28 bits     6000         367 / 199,   560 / 548
 bool use_binned(const gt_storage* st, const Scratch& sc, const Reads& R) {
     const uint64_t buckets = bin_buckets(st);
     if (R.dyn || sc.fixed || !buckets) return false;
