@@ -1013,8 +1013,8 @@ uint32_t route_digits(const gt_storage* st) {
 // more of 30 MiB together (smaller ones are read mostly out of the L2s as they
 // are; one table's reads cost less than their routing), from 2^23 busy bases
 // plus one per 64 table bytes on (every slice is read into an L2 once per
-// sub-batch), on reads most of whose bases start a window: a base is hashed and
-// sorted whether it does or not.  150-base reads, us (direct / routed):
+// sub-batch), on reads of whose bases enough start a window: a base is hashed
+// and its tile sorted whether it does or not.  150-base reads, us (direct / routed):
 //   4 x 2^21 counts   300k reads 1332 / 3278
 //   4 x 2^23 counts   30k reads  247 /  382    100k  792 /  729     1M 7431 / 6016
 //   4 x 2^25 counts   30k reads  293 /  333    100k  937 /  848     1M 8852 / 5473
@@ -1022,18 +1022,28 @@ uint32_t route_digits(const gt_storage* st) {
 //   4 x 2^28 bits     30k reads  270 /  267    100k  859 /  670     1M 8076 / 5984
 //   2 x 2^28 bits     30k reads  152 /  188    100k  458 /  414     1M 4183 / 3707
 //   1 x 2^28 counts   1M reads  2468 / 3255
-// and 1M reads by the share of bases that start a window:
-//   4 x 2^28 counts   0.28 1820 / 2848   0.39 3219 / 4158   0.60 4765 / 4470
-//   4 x 2^28 bits     0.28 1781 / 2509   0.39 3170 / 3460   0.60 4803 / 3671
-//   2 x 2^28 counts   0.39 1759 / 2670   0.60 2516 / 2763
+// The share of bases that has to start a window grows with the slices, since a
+// tile's run of one gets shorter.  100M bases, ms, by that share (direct / routed):
+//                        0.28          0.39          0.47          0.60          0.80
+//   4 x 2^28 counts   2.41 / 3.90   3.19 / 4.24   3.83 / 4.34   4.70 / 4.49   6.06 / 4.80
+//   4 x 2^26 counts   2.35 / 2.77   3.11 / 3.06   3.77 / 3.26   4.64 / 3.60   6.11 / 3.93
+//   4 x 2^28 bits     2.38 / 3.36   3.07 / 3.43   3.66 / 3.47   4.64 / 3.63   5.94 / 4.07
+//   3 x 2^28 counts   1.89 / 2.84   2.50 / 3.09   2.96 / 3.23   3.56 / 3.33   4.73 / 3.69
+//   2 x 2^28 counts   1.31 / 2.58   1.70 / 2.62   2.04 / 2.64   2.48 / 2.70   3.20 / 2.93
+//   2 x 2^28 bits     1.44 / 2.34   1.64 / 2.39   1.89 / 2.38   2.37 / 2.45   3.03 / 2.57
+//   2 x 2^25 counts   1.20 / 1.71   1.53 / 1.79   1.83 / 1.89   2.26 / 2.08   2.93 / 2.32
 bool use_routed(const gt_storage* st, const Scratch& sc, const Reads& R) {
     if (R.dyn || sc.fixed || !route_digits(st)) return false;
     const char* v = std::getenv("GOETIA_AMD_ROUTED");
     if (v && *v) return v[0] != '0';
     uint64_t bytes = 0;
     for (uint64_t nb : st->nbytes) bytes += nb;
-    const uint64_t busy = busy_bases(R), n = (uint64_t)R.n_bases;      // (busy is at most 5/4 of the windows)
-    if (st->n_tables < 2 || 80 * busy < (st->n_tables == 2 ? 70ULL : 45ULL) * n) return false;
+    if (st->n_tables < 2) return false;
+    const uint64_t digits = route_digits(st), busy = busy_bases(R);
+    uint64_t percent = st->n_tables == 2 ? 50 + (digits > 64 ? 10 : 0) + (digits > 128 ? 10 : 0)
+                                         : 38 + (digits > 128 ? 7 : 0) + (digits > 256 ? 7 : 0);
+    if (st->kind == kBit) percent -= 6;
+    if (80 * busy < percent * (uint64_t)R.n_bases) return false;       // (busy is 5/4 of the windows, or all bases)
     return bytes >= kPastL2 && busy >= (1ULL << 23) + bytes / 64;
 }
 

@@ -519,7 +519,8 @@ def test_queries_of_few_tables_at_every_shape_of_launch(oracle, kind, sizes, n_b
 
 @pytest.mark.parametrize('n_tables,L,K,n_reads,routed', [
     (4, 150, 31, 70_000, True), (4, 150, 31, 58_000, False), (4, 75, 63, 200_000, False), (4, 75, 55, 700_000, False),
-    (4, 101, 41, 160_000, True), (2, 150, 31, 70_000, True), (2, 75, 31, 400_000, False), (1, 150, 31, 200_000, False)])
+    (4, 101, 41, 160_000, True), (2, 150, 31, 70_000, True), (2, 75, 31, 400_000, True), (2, 101, 63, 400_000, False),
+    (1, 150, 31, 200_000, False)])
 def test_queries_are_routed_where_windows_are_many(oracle, launches, n_tables, L, K, n_reads, routed):
     """Which way a query goes by itself: by its bases, less those that start no
     window, and by their share."""
